@@ -295,6 +295,21 @@ int paged_attention_prefill(const gdn_tensor* q, const gdn_tensor* k_cache, cons
                             void* stream);
 
 /*
+ * paged_attention_prefill with a workspace, in which rows (32 queries of up
+ * to four heads) over long contexts are cut into pieces of keys that run as
+ * workgroups of their own and are merged by a second launch.  Whether and how
+ * far follows from the sizes alone; paged_attention_prefill_workspace_size is
+ * the fp32 elements that the choice needs, 0 when nothing is split (max_keys =
+ * max_blocks * page).  workspace: 1-D fp32, 16-byte aligned, overwritten.
+ */
+int64_t paged_attention_prefill_workspace_size(int64_t num_tokens, int64_t num_seqs, int64_t num_q_heads,
+                                               int64_t num_kv_heads, int64_t head_dim, int64_t max_keys);
+int paged_attention_prefill_split(const gdn_tensor* q, const gdn_tensor* k_cache, const gdn_tensor* v_cache,
+                                  const gdn_tensor* block_tables, const gdn_tensor* context_lens,
+                                  const gdn_tensor* cu_seqlens, gdn_tensor* out, gdn_tensor* workspace,
+                                  int64_t max_seqlen, float scale, void* stream);
+
+/*
  * paged_attention_decode <- paged_flash_attention_decode, ops/full_attention.py:282-335
  *   q, out (B, Hq, D): one query per sequence, at position context_lens[b] - 1;
  *   caches and block_tables (B, max_blocks) as above.  num_splits 1..256.

@@ -44,6 +44,8 @@ EXPORTED_SYMBOLS = (
     "gdn_gating",
     "flash_attention_varlen",
     "paged_attention_prefill",
+    "paged_attention_prefill_workspace_size",
+    "paged_attention_prefill_split",
     "paged_attention_decode_workspace_size",
     "paged_attention_decode",
     "paged_attention_decode_noalloc",
@@ -119,6 +121,10 @@ def load() -> ctypes.CDLL:
                                                            ctypes.c_void_p]
         lib.paged_attention_prefill.restype = ctypes.c_int
         lib.paged_attention_prefill.argtypes = [_PT] * 7 + [ctypes.c_int64, ctypes.c_float, ctypes.c_void_p]
+        lib.paged_attention_prefill_workspace_size.restype = ctypes.c_int64
+        lib.paged_attention_prefill_workspace_size.argtypes = [ctypes.c_int64] * 6
+        lib.paged_attention_prefill_split.restype = ctypes.c_int
+        lib.paged_attention_prefill_split.argtypes = [_PT] * 8 + [ctypes.c_int64, ctypes.c_float, ctypes.c_void_p]
         lib.paged_attention_decode_workspace_size.restype = ctypes.c_int64
         lib.paged_attention_decode_workspace_size.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int64,
                                                               ctypes.c_int32]

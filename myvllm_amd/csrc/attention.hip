@@ -115,7 +115,17 @@ struct AttnArgs {
   int32_t Hq, Hkv, gh;  // gh: query heads per workgroup (1, 2 or 4)
   float c;              // softmax scale * log2(e)
   bool cu64, ctx64, causal;
+  // split prefill: key tiles of a piece (even), (tile, head group) rows of the
+  // grid, and the pieces' partials (slot row * splits + piece)
+  int32_t piece_tiles, splits;
+  int64_t rows;
+  float* part;
 };
+
+// Floats of one piece's partial: per wave, the accumulators of its 32 queries
+// in register order (lane-contiguous 16-byte pieces), then m and l per lane.
+template <int D> constexpr int64_t prefill_part_wave() { return 32 * D + 128; }
+template <int D> constexpr int64_t prefill_part_floats() { return 4 * prefill_part_wave<D>(); }
 
 template <bool PAGED>
 GDN_DEVICE const char* kv_row(const KvSource& s, const PagedTable& tb, int64_t n, int64_t s0, int64_t j, int kvh) {
@@ -152,9 +162,22 @@ __device__ __attribute__((always_inline)) SeqTile attn_tile_lookup(const void* c
   return r;
 }
 
-template <typename T, int D, int BN, int PG>
+// SPLIT: the key range of every (query tile, head group) row is cut into
+// pieces of a.piece_tiles key tiles, one workgroup each (piece index
+// outermost in the grid, so that the pieces that run together read the same
+// stretch of their sequence's K/V rows).  A row of one piece writes its output
+// rows; otherwise every piece writes m, l and the unnormalised O to the
+// workspace and attn_prefill_combine_kernel merges them.  It serves batches
+// whose rows are few or uneven for 256 CUs (one workgroup per CU at D = 256):
+// a workgroup runs 1.2 us per key tile, so 1,000 new tokens over a 15,000-key
+// prefix are 128 rows of 550 us each.  Measured (16 / 2 heads, D = 256, one
+// piece -> split): four prompts of 800 to 1,500 tokens over prefixes of 500 to
+// 15,800 keys 1,192 -> 951 us (574 -> 720 TFLOP/s), one of 512 over 8,000 98 ->
+// 47 us, five of 18 over 11,700 301 -> 64 us.
+template <typename T, int D, int BN, int PG, bool SPLIT>
 __global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnArgs a) {
   constexpr bool PAGED = PG != 0;
+  static_assert(!SPLIT || PG >= 2, "split rows are paged rows of whole 16-row groups");
   typedef Mma<T> M;
   typedef typename M::v8 v8;
   typedef typename M::v4 v4;
@@ -191,10 +214,12 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnArgs a) {
   // sequence's workgroups run together and share its K/V rows in L2.
   __shared__ int32_t lookup[8];
   const int hg = a.Hq / gh;  // head groups
-  const SeqTile st = attn_tile_lookup(a.cu, a.cu64, a.nseq, a.T, 32 * qsubs, blockIdx.x / hg, lookup);
+  const uint32_t piece = SPLIT ? blockIdx.x / (uint32_t)a.rows : 0u;
+  const uint32_t row_id = SPLIT ? blockIdx.x - piece * (uint32_t)a.rows : blockIdx.x;
+  const SeqTile st = attn_tile_lookup(a.cu, a.cu64, a.nseq, a.T, 32 * qsubs, row_id / hg, lookup);
   if (st.seq < 0) return;
   const int64_t n = st.seq;
-  const int y = (int)(blockIdx.x % hg);
+  const int y = (int)(row_id % hg);
   const int kvh = y / groups;
   const int head = kvh * R + (y % groups) * gh + (w % gh);
 
@@ -216,8 +241,15 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnArgs a) {
   const int64_t q0 = qb + (w / gh) * 32;
   const int64_t wg_qend = qb + 32 * qsubs < len ? qb + 32 * qsubs : len;
   const int64_t w_qend = q0 + 32 < len ? q0 + 32 : len;
-  const int64_t kend = a.causal ? clamp64(off + wg_qend, 0, Lk) : Lk;
-  const int64_t kend_w = q0 >= len ? 0 : (a.causal ? clamp64(off + w_qend, 0, Lk) : Lk);
+  const int64_t kend_row = a.causal ? clamp64(off + wg_qend, 0, Lk) : Lk;
+  const int64_t kend_roww = q0 >= len ? 0 : (a.causal ? clamp64(off + w_qend, 0, Lk) : Lk);
+  // this piece's key tiles [tile0, ntiles); keys past its end are not loaded
+  const int tile0 = SPLIT ? (int)piece * a.piece_tiles : 0;
+  const bool whole = !SPLIT || kend_row <= (int64_t)a.piece_tiles * BN;  // the row is one piece
+  if (SPLIT && piece > 0 && (int64_t)tile0 * BN >= kend_row) return;
+  const int64_t piece_end = SPLIT ? (int64_t)(tile0 + a.piece_tiles) * BN : 0;
+  const int64_t kend = SPLIT && kend_row > piece_end ? piece_end : kend_row;
+  const int64_t kend_w = SPLIT && kend_roww > piece_end ? piece_end : kend_roww;
   const int ntiles = (int)((kend + BN - 1) / BN);
 
   // query fragments (B operand of S^T = K Q^T): lane holds query q0 + lane % 32,
@@ -309,7 +341,11 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnArgs a) {
       }
     }
   };
-  if (G16) load_ids(0, idlo, idhi, idin, slots);
+  if (SPLIT) {
+    gcol = (uint32_t)tile0 * NG / gpp;
+    grem = (uint32_t)tile0 * NG - gcol * gpp;
+  }
+  if (G16) load_ids(tile0, idlo, idhi, idin, slots);
   const uint32_t kst = (uint32_t)a.k.st, vst = (uint32_t)a.v.st;  // row strides in bytes (below 2^31)
   const char* kbase = a.k.base + kvh * a.k.sh;
   const char* vbase = a.v.base + kvh * a.v.sh;
@@ -521,16 +557,16 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnArgs a) {
   // tile t computes from LDS buffer t % 2 while tile t + 1 waits in registers
   // and tile t + 2 is in flight: two register sets (A: even tiles, B: odd)
   uint4 kA[NLD], vA[NLD], kB[NLD], vB[NLD];
-  load_tile(0, kA, vA);
+  load_tile(tile0, kA, vA);
   stage_q();  // (waits for the query loads with tile 0's loads in flight)
   store_tile(0, kA, vA);
-  load_tile(1, kB, vB);
-  load_tile(2, kA, vA);
+  load_tile(tile0 + 1, kB, vB);
+  load_tile(tile0 + 2, kA, vA);
   __syncthreads();
   // (packed rows: the next tiles' stores and loads go out between the score
   // MFMAs and the softmax; paged rows: after the tile, since their loads
   // first wait for the block ids, and the longer live ranges cost registers)
-  for (int t = 0; t < ntiles; t += 2) {
+  for (int t = tile0; t < ntiles; t += 2) {
     if constexpr (PG == 0) {
       compute(t, 0, [&]() __attribute__((always_inline)) {
         store_tile(1, kB, vB);
@@ -556,6 +592,20 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnArgs a) {
   }
 
   const float lt = lsum + __shfl_xor(lsum, 32);
+  if constexpr (SPLIT) {
+    if (!whole) {
+      float* pw = a.part + ((int64_t)row_id * a.splits + piece) * prefill_part_floats<D>() + w * prefill_part_wave<D>();
+#pragma unroll
+      for (int d = 0; d < NDT; ++d)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *reinterpret_cast<f32x4*>(pw + ((4 * d + g) * 64 + lane) * 4) =
+              f32x4{oacc[d][4 * g], oacc[d][4 * g + 1], oacc[d][4 * g + 2], oacc[d][4 * g + 3]};
+      pw[32 * D + lane] = m_used;
+      pw[32 * D + 64 + lane] = lt;
+      return;
+    }
+  }
   const float inv = lt > 0.f ? 1.f / lt : 0.f;
   if constexpr (QL) {
     // O goes out through the wave's own query rows in LDS (no longer read):
@@ -595,6 +645,63 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnArgs a) {
         for (int e = 0; e < 4; ++e) ov[e] = (T)(oacc[d][4 * g + e] * inv);
         *reinterpret_cast<v4*>(op + 32 * d + 8 * g) = ov;
       }
+  }
+}
+
+// Merge of a split prefill's pieces: workgroup (row, dim group) of the same
+// 4 waves x 32 queries as the prefill kernel, each lane reading back its own
+// accumulator pieces of DG 32-dim blocks.  Rows of one piece were written by
+// the prefill itself.
+template <typename T, int D, int BN, int DG>
+__global__ __launch_bounds__(256) void attn_prefill_combine_kernel(const AttnArgs a) {
+  typedef typename Mma<T>::v4 v4;
+  __shared__ int32_t lookup[8];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int R = a.Hq / a.Hkv, gh = a.gh, qsubs = 4 / gh, groups = R / gh, hg = a.Hq / gh;
+  const SeqTile st = attn_tile_lookup(a.cu, a.cu64, a.nseq, a.T, 32 * qsubs, blockIdx.x / hg, lookup);
+  if (st.seq < 0) return;
+  const int y = (int)(blockIdx.x % hg);
+  const int head = (y / groups) * R + (y % groups) * gh + (w % gh);
+  int64_t s0, s1;
+  seq_range(a.cu, a.cu64, st.seq, a.T, s0, s1);
+  const int64_t len = s1 - s0;
+  const int64_t ntile = (len + 32 * qsubs - 1) / (32 * qsubs);
+  const int64_t qb = (ntile - 1 - st.tile) * 32 * qsubs;
+  const int64_t ctx = load_index(a.ctx, st.seq, a.ctx64);
+  const int64_t Lk = clamp64(ctx, 0, a.tab.cols * a.tab.page);
+  const int64_t wg_qend = qb + 32 * qsubs < len ? qb + 32 * qsubs : len;
+  const int64_t kend = clamp64(ctx - len + wg_qend, 0, Lk);
+  const int64_t pk = (int64_t)a.piece_tiles * BN;
+  const int np = (int)((kend + pk - 1) / pk);  // at most a.splits: kend <= columns x page
+  const int64_t qi = qb + (w / gh) * 32 + (lane & 31);
+  if (np <= 1 || qi >= len) return;
+  const float* base = a.part + (int64_t)blockIdx.x * a.splits * prefill_part_floats<D>() + w * prefill_part_wave<D>();
+  float mx = -INFINITY;
+  for (int p = 0; p < np; ++p) mx = fmaxf(mx, base[p * prefill_part_floats<D>() + 32 * D + lane]);
+  f32x4 acc[4 * DG];
+#pragma unroll
+  for (int i = 0; i < 4 * DG; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float l = 0.f;
+  for (int p = 0; p < np; ++p) {
+    const float* pp = base + p * prefill_part_floats<D>();
+    const float m = pp[32 * D + lane];
+    const float wt = m == -INFINITY ? 0.f : exp2_fast(m - mx);
+    l += wt * pp[32 * D + 64 + lane];
+#pragma unroll
+    for (int i = 0; i < 4 * DG; ++i) {
+      const f32x4 o = *reinterpret_cast<const f32x4*>(pp + ((4 * DG * blockIdx.y + i) * 64 + lane) * 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[i][e] += wt * o[e];
+    }
+  }
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  T* op = reinterpret_cast<T*>(a.o) + (s0 + qi) * a.o_st + (int64_t)head * a.o_sh + 4 * (lane >> 5) + 32 * DG * blockIdx.y;
+#pragma unroll
+  for (int i = 0; i < 4 * DG; ++i) {
+    v4 ov;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) ov[e] = (T)(acc[i][e] * inv);
+    *reinterpret_cast<v4*>(op + 8 * i) = ov;
   }
 }
 
@@ -1118,17 +1225,28 @@ hipError_t launch_prefill_t(const AttnArgs& a, int64_t nseq, int64_t max_len, hi
   // query tiles: at most T / tile_len + one partial tile per sequence
   const int64_t tiles = a.T / (32 * qsubs) + nseq;
   const dim3 grid((unsigned)(tiles * (a.Hq / a.gh)));
-  if (!PAGED)
-    hipLaunchKernelGGL((attn_prefill_kernel<T, D, BN, 0>), grid, dim3(256), 0, st, a);
-  else if (a.tab.page % 16 == 0 && a.k.sb < (int64_t(1) << 32) && a.v.sb < (int64_t(1) << 32) && a.tab.cols > 0 &&
-           a.tab.cols * a.tab.page < (int64_t(1) << 31) && a.tab.num_blocks < (int64_t(1) << 31)) {
+  if constexpr (!PAGED) {
+    hipLaunchKernelGGL((attn_prefill_kernel<T, D, BN, 0, false>), grid, dim3(256), 0, st, a);
+  } else if (a.tab.page % 16 == 0 && a.k.sb < (int64_t(1) << 32) && a.v.sb < (int64_t(1) << 32) && a.tab.cols > 0 &&
+             a.tab.cols * a.tab.page < (int64_t(1) << 31) && a.tab.num_blocks < (int64_t(1) << 31)) {
     // whole 16-row groups per page, 32-bit table arithmetic
-    if (a.tab.is64)
-      hipLaunchKernelGGL((attn_prefill_kernel<T, D, BN, 3>), grid, dim3(256), 0, st, a);
+    if (a.splits > 1) {
+      const dim3 sgrid((unsigned)(a.rows * a.splits));
+      constexpr int DG = D == 256 ? 2 : 1;  // 32-dim blocks per combine workgroup
+      if (a.tab.is64)
+        hipLaunchKernelGGL((attn_prefill_kernel<T, D, BN, 3, true>), sgrid, dim3(256), 0, st, a);
+      else
+        hipLaunchKernelGGL((attn_prefill_kernel<T, D, BN, 2, true>), sgrid, dim3(256), 0, st, a);
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return e;
+      hipLaunchKernelGGL((attn_prefill_combine_kernel<T, D, BN, DG>), dim3((unsigned)a.rows, D / (32 * DG)), dim3(256),
+                         0, st, a);
+    } else if (a.tab.is64)
+      hipLaunchKernelGGL((attn_prefill_kernel<T, D, BN, 3, false>), grid, dim3(256), 0, st, a);
     else
-      hipLaunchKernelGGL((attn_prefill_kernel<T, D, BN, 2>), grid, dim3(256), 0, st, a);
+      hipLaunchKernelGGL((attn_prefill_kernel<T, D, BN, 2, false>), grid, dim3(256), 0, st, a);
   } else
-    hipLaunchKernelGGL((attn_prefill_kernel<T, D, BN, 1>), grid, dim3(256), 0, st, a);
+    hipLaunchKernelGGL((attn_prefill_kernel<T, D, BN, 1, false>), grid, dim3(256), 0, st, a);
   return hipGetLastError();
 }
 
@@ -1145,6 +1263,53 @@ hipError_t launch_prefill(const AttnArgs& a, int dtype, int D, int64_t nseq, int
 }
 
 int heads_per_group(int R) { return R % 4 == 0 ? 4 : (R % 2 == 0 ? 2 : 1); }
+
+// Pieces per row of a split paged prefill over at most `cap` keys (1: not
+// split) and the key tiles of a piece.  The host does not see the context
+// lengths, so the choice prices the batch in key-tile steps of one workgroup
+// (1.18 us at D = 256) as if its rows held half the table's capacity on
+// average and the last row to start all of it: per workgroup slot
+// rows n / slots pieces of kFixed + nt / 2n steps, the last piece's nt / n,
+// and for n > 1 the combine (its launch, and the partials' traffic).  The
+// fixed part of a workgroup (tile lookup, query staging, pipeline fill,
+// output) was measured at about 10 steps.  One split from about 2,000 rows on
+// (16 prompts of 1,200 tokens over 16 heads): there the rows themselves fill
+// the chip evenly.
+struct PrefillSplit {
+  int32_t splits, piece_tiles;
+  int64_t rows;
+};
+PrefillSplit prefill_split(int64_t T, int64_t nseq, int64_t Hq, int64_t Hkv, int64_t D, int64_t cap) {
+  constexpr double kSlots = 256, kFixed = 10, kCombine = 6, kPiece = 0.03;
+  constexpr int64_t kMaxSplits = 64, kMaxFloats = int64_t(1) << 27;  // partials of at most 512 MiB
+  PrefillSplit r{1, 0, 0};
+  if (T <= 0 || nseq <= 0 || Hkv <= 0 || cap <= 0) return r;
+  const int gh = heads_per_group((int)(Hq / Hkv));
+  const int BN = D == 256 ? 32 : 64;
+  r.rows = (T / (32 * (4 / gh)) + nseq) * (Hq / gh);
+  const int64_t nt = (cap + BN - 1) / BN;
+  const double slots = D == 256 ? kSlots : 2 * kSlots;  // D <= 128: two workgroups fit a CU
+  const int64_t per_piece = 4 * (32 * D + 128);
+  double best = 0;
+  for (int64_t n = 1; n <= kMaxSplits; ++n) {
+    if (n > 1 && (nt / n < 8 || r.rows * n * per_piece > kMaxFloats)) break;
+    const double step = (double)nt / n;
+    const double t = r.rows * n / slots * (kFixed + 0.5 * step) + step +
+                     (n > 1 ? kCombine + kPiece * r.rows * n * D / 256 : 0);
+    if (n == 1) {
+      best = 0.9 * t;  // (a split has to win clearly)
+    } else if (t < best) {
+      best = t;
+      r.splits = (int32_t)n;
+    }
+  }
+  if (r.splits > 1) {
+    r.piece_tiles = (int32_t)((nt + r.splits - 1) / r.splits);
+    r.piece_tiles += r.piece_tiles & 1;
+    r.splits = (int32_t)((nt + r.piece_tiles - 1) / r.piece_tiles);
+  }
+  return r;
+}
 
 template <typename T, int D>
 hipError_t launch_decode_t(const DecodeArgs& a, hipStream_t st) {
@@ -1197,10 +1362,20 @@ hipError_t attn_varlen_prefill_launch(const gdn_tensor* q, const gdn_tensor* k, 
 
 hipError_t attn_paged_prefill_launch(const gdn_tensor* q, const gdn_tensor* kc, const gdn_tensor* vc,
                                      const gdn_tensor* tab, const gdn_tensor* ctx, const gdn_tensor* cu,
-                                     gdn_tensor* out, int64_t max_seqlen, float scale, hipStream_t st) {
+                                     gdn_tensor* out, float* workspace, int64_t max_seqlen, float scale,
+                                     hipStream_t st) {
   const int64_t nseq = cu->shape[0] - 1;
   if (q->shape[0] == 0) return hipSuccess;
   AttnArgs a{};
+  a.splits = 1;
+  if (workspace) {
+    const PrefillSplit sp = prefill_split(q->shape[0], nseq, q->shape[1], kc->shape[2], q->shape[2],
+                                          tab->shape[1] * kc->shape[1]);
+    a.splits = sp.splits;
+    a.piece_tiles = sp.piece_tiles;
+    a.rows = sp.rows;
+    a.part = workspace;
+  }
   a.q = q->data;
   a.q_st = q->stride[0];
   a.q_sh = q->stride[1];
@@ -1222,6 +1397,11 @@ hipError_t attn_paged_prefill_launch(const gdn_tensor* q, const gdn_tensor* kc, 
   a.c = scale * kLog2e;
   a.causal = true;
   return launch_prefill<true>(a, q->dtype, (int)q->shape[2], nseq, max_seqlen, st);
+}
+
+int64_t attn_paged_prefill_workspace(int64_t T, int64_t nseq, int64_t Hq, int64_t Hkv, int64_t D, int64_t cap) {
+  const PrefillSplit sp = prefill_split(T, nseq, Hq, Hkv, D, cap);
+  return sp.splits > 1 ? sp.rows * sp.splits * 4 * (32 * D + 128) : 0;
 }
 
 namespace {

@@ -37,7 +37,9 @@ hipError_t attn_varlen_prefill_launch(const gdn_tensor* q, const gdn_tensor* k, 
                                       int causal, hipStream_t st);
 hipError_t attn_paged_prefill_launch(const gdn_tensor* q, const gdn_tensor* kc, const gdn_tensor* vc,
                                      const gdn_tensor* tab, const gdn_tensor* ctx, const gdn_tensor* cu,
-                                     gdn_tensor* out, int64_t max_seqlen, float scale, hipStream_t st);
+                                     gdn_tensor* out, float* workspace, int64_t max_seqlen, float scale,
+                                     hipStream_t st);
+int64_t attn_paged_prefill_workspace(int64_t T, int64_t nseq, int64_t Hq, int64_t Hkv, int64_t D, int64_t cap);
 hipError_t attn_paged_decode_launch(const gdn_tensor* q, const gdn_tensor* kc, const gdn_tensor* vc,
                                     const gdn_tensor* tab, const gdn_tensor* ctx, gdn_tensor* out, float* workspace,
                                     int32_t splits, float scale, hipStream_t st);
@@ -471,10 +473,11 @@ GDN_EXPORT int flash_attention_varlen(const gdn_tensor* q, const gdn_tensor* k, 
                                               reinterpret_cast<hipStream_t>(stream)));
 }
 
-GDN_EXPORT int paged_attention_prefill(const gdn_tensor* q, const gdn_tensor* k_cache, const gdn_tensor* v_cache,
-                                       const gdn_tensor* block_tables, const gdn_tensor* context_lens,
-                                       const gdn_tensor* cu_seqlens, gdn_tensor* out, int64_t max_seqlen,
-                                       float scale, void* stream) {
+namespace {
+// Checks and launch of the paged prefill; without a workspace its rows are not split.
+int paged_prefill(const gdn_tensor* q, const gdn_tensor* k_cache, const gdn_tensor* v_cache,
+                  const gdn_tensor* block_tables, const gdn_tensor* context_lens, const gdn_tensor* cu_seqlens,
+                  gdn_tensor* out, const gdn_tensor* workspace, int64_t max_seqlen, float scale, void* stream) {
   GDN_TRY(check_desc(q, 3));
   GDN_TRY(check_desc(out, 3));
   GDN_TRY(check_desc(cu_seqlens, 1));
@@ -493,8 +496,48 @@ GDN_EXPORT int paged_attention_prefill(const gdn_tensor* q, const gdn_tensor* k_
   if (k_cache->shape[1] * std::max(k_cache->stride[1], v_cache->stride[1]) * es >= (int64_t(1) << 31) ||
       block_tables->shape[1] * k_cache->shape[1] >= (int64_t(1) << 31))
     return GDN_ERR_RANGE;
-  return launch_rc(attn_paged_prefill_launch(q, k_cache, v_cache, block_tables, context_lens, cu_seqlens, out,
+  float* ws = nullptr;
+  if (workspace) {
+    GDN_TRY(check_desc(workspace, 1));
+    if (workspace->dtype != GDN_DTYPE_F32) return GDN_ERR_DTYPE;
+    if (workspace->stride[0] != 1) return GDN_ERR_STRIDE;
+    const int64_t need = paged_attention_prefill_workspace_size(q->shape[0], N, q->shape[1], k_cache->shape[2],
+                                                                q->shape[2], block_tables->shape[1] * k_cache->shape[1]);
+    if (workspace->shape[0] < need) return GDN_ERR_SHAPE;
+    if (need > 0) {
+      if (!aligned(workspace, 16)) return GDN_ERR_ALIGN;
+      ws = reinterpret_cast<float*>(workspace->data);
+    }
+  }
+  return launch_rc(attn_paged_prefill_launch(q, k_cache, v_cache, block_tables, context_lens, cu_seqlens, out, ws,
                                              max_seqlen, scale, reinterpret_cast<hipStream_t>(stream)));
+}
+}  // namespace
+
+GDN_EXPORT int paged_attention_prefill(const gdn_tensor* q, const gdn_tensor* k_cache, const gdn_tensor* v_cache,
+                                       const gdn_tensor* block_tables, const gdn_tensor* context_lens,
+                                       const gdn_tensor* cu_seqlens, gdn_tensor* out, int64_t max_seqlen,
+                                       float scale, void* stream) {
+  return paged_prefill(q, k_cache, v_cache, block_tables, context_lens, cu_seqlens, out, nullptr, max_seqlen, scale,
+                       stream);
+}
+
+GDN_EXPORT int64_t paged_attention_prefill_workspace_size(int64_t num_tokens, int64_t num_seqs, int64_t num_q_heads,
+                                                          int64_t num_kv_heads, int64_t head_dim, int64_t max_keys) {
+  if (num_q_heads < 1 || num_kv_heads < 1 || num_q_heads % num_kv_heads != 0 ||
+      (head_dim != 64 && head_dim != 128 && head_dim != 256))
+    return 0;
+  return attn_paged_prefill_workspace(num_tokens, num_seqs, num_q_heads, num_kv_heads, head_dim, max_keys);
+}
+
+GDN_EXPORT int paged_attention_prefill_split(const gdn_tensor* q, const gdn_tensor* k_cache,
+                                             const gdn_tensor* v_cache, const gdn_tensor* block_tables,
+                                             const gdn_tensor* context_lens, const gdn_tensor* cu_seqlens,
+                                             gdn_tensor* out, gdn_tensor* workspace, int64_t max_seqlen, float scale,
+                                             void* stream) {
+  if (!workspace) return GDN_ERR_NULL;
+  return paged_prefill(q, k_cache, v_cache, block_tables, context_lens, cu_seqlens, out, workspace, max_seqlen, scale,
+                       stream);
 }
 
 GDN_EXPORT int64_t paged_attention_decode_workspace_size(int64_t num_seqs, int64_t num_q_heads, int64_t head_dim,

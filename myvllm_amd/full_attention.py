@@ -205,7 +205,9 @@ def paged_flash_attention_prefill(
     sequence n sits at position ``context_lens[n] - len_n + i`` and attends
     causally to the cached keys.  ``block_m_indices`` (the reference's
     per-16-row work list) is accepted for interface parity and not needed:
-    the kernel tiles the queries itself from ``cu_seqlens``."""
+    the kernel tiles the queries itself from ``cu_seqlens``.  Few new tokens
+    over a long cache are split over the keys as well; the partials then take a
+    temporary workspace of up to 512 MiB."""
     if k_cache.shape[1] != page_block_size:
         raise ValueError(f"page_block_size {page_block_size} != k_cache.shape[1] {k_cache.shape[1]}")
     dev = _lib.require_device(q, k_cache, v_cache, page_block_tables, context_lens, cu_seqlens)
@@ -214,9 +216,20 @@ def paged_flash_attention_prefill(
     q, k_cache, v_cache = _lib.vec16(q), _lib.vec16(k_cache), _lib.vec16(v_cache)
     o = _out_for(out, (q.shape[0], q.shape[1], v_cache.shape[-1]), q.dtype, dev)
     D = _lib.describe
-    rc = _lib.load().paged_attention_prefill(
-        D(q), D(k_cache), D(v_cache), D(page_block_tables), D(context_lens), D(cu_seqlens), D(o),
-        int(max_seqlen), float(scale), _lib.stream_handle(dev),
-    )
+    lib = _lib.load()
+    n_ws = lib.paged_attention_prefill_workspace_size(q.shape[0], cu_seqlens.numel() - 1, q.shape[1],
+                                                      k_cache.shape[2], q.shape[2],
+                                                      page_block_tables.shape[1] * page_block_size)
+    if n_ws > 0:
+        ws = torch.empty(n_ws, dtype=torch.float32, device=dev)
+        rc = lib.paged_attention_prefill_split(
+            D(q), D(k_cache), D(v_cache), D(page_block_tables), D(context_lens), D(cu_seqlens), D(o), D(ws),
+            int(max_seqlen), float(scale), _lib.stream_handle(dev),
+        )
+    else:
+        rc = lib.paged_attention_prefill(
+            D(q), D(k_cache), D(v_cache), D(page_block_tables), D(context_lens), D(cu_seqlens), D(o),
+            int(max_seqlen), float(scale), _lib.stream_handle(dev),
+        )
     _lib.check("paged_attention_prefill", rc)
     return _finish(out, o)

@@ -1,0 +1,69 @@
+"""GPU: the split paged prefill (few new tokens over a long context: the key
+range of a row runs as several workgroups) vs the fp64 oracle and vs the
+unsplit entry.  Same bars as the attention tests; between the two entries the
+outputs differ by the order of fp32 sums and by P rounded against another
+base, so they also share the 5e-3 relative norm."""
+import pytest
+import torch
+
+from conftest import assert_out_close
+from myvllm_amd import _lib, paged_flash_attention_prefill
+from myvllm_amd.workloads import paged_case
+from oracle.attention import paged_attention_ref
+
+
+def _splits(T, N, Hq, Hkv, D, cap):
+    f = _lib.load().paged_attention_prefill_workspace_size(T, N, Hq, Hkv, D, cap)
+    R = Hq // Hkv
+    gh = 4 if R % 4 == 0 else (2 if R % 2 == 0 else 1)
+    rows = (T // (32 * (4 // gh)) + N) * (Hq // gh)
+    per = rows * 4 * (32 * D + 128)
+    assert f % per == 0
+    return max(1, f // per)
+
+
+def test_split_rule():
+    """Few rows over long tables are split; full batches, short tables and empty calls are not,
+    and the partials stay within 512 MiB."""
+    assert _splits(16, 1, 16, 2, 256, 8192) > 8
+    assert 1 < _splits(4538, 4, 16, 2, 256, 16832) <= 8
+    assert _splits(19041, 16, 16, 2, 256, 6144) == 1
+    assert _splits(64, 2, 16, 2, 256, 256) == 1
+    for T, N, Hq, Hkv, D, cap in ((0, 1, 16, 2, 256, 8192), (16, 0, 16, 2, 256, 8192), (16, -1, 16, 2, 256, 8192),
+                                  (16, 1, 16, 2, 96, 8192), (16, 1, 16, 3, 256, 8192), (16, 1, 16, 2, 256, 0)):
+        assert _lib.load().paged_attention_prefill_workspace_size(T, N, Hq, Hkv, D, cap) == 0
+    for T in (1, 100, 2000, 30000):
+        for cap in (1 << 12, 1 << 20, 1 << 30):
+            assert _lib.load().paged_attention_prefill_workspace_size(T, 3, 16, 2, 256, cap) * 4 <= 1 << 29
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize(
+    "ctx, new, page, Hq, Hkv, Dh, dtype, tab64",
+    [
+        ([4096, 37, 1500], [3, 37, 40], 16, 16, 2, 256, torch.bfloat16, False),  # one row of many pieces, rows of one
+        ([2048, 2049, 511], [1, 33, 1], 16, 8, 1, 256, torch.float16, True),  # ends on and past a piece's end
+        ([3000, 0, 20], [70, 0, 50], 16, 16, 4, 128, torch.bfloat16, False),  # an empty sequence; queries without keys
+        ([5000, 1], [129, 1], 48, 4, 4, 128, torch.bfloat16, True),  # one head per kv head: four query blocks
+        ([2500, 700], [31, 90], 32, 8, 4, 64, torch.float16, False),  # two heads per kv head
+    ],
+)
+def test_split_paged_prefill(dev, ctx, new, page, Hq, Hkv, Dh, dtype, tab64):
+    case = paged_case(ctx, new, page=page, seed=len(ctx) + page, Hq=Hq, Hkv=Hkv, D=Dh, dtype=dtype)
+    assert _splits(sum(new), len(new), Hq, Hkv, Dh, case.block_tables.shape[1] * page) > 1
+    tab = case.block_tables.to(torch.int64) if tab64 else case.block_tables
+    d = [t.to(dev) for t in (case.q, case.k_cache, case.v_cache, tab, case.context_lens, case.cu)]
+    print(f"split paged prefill ctx={ctx} new={new} page={page} Hq={Hq} Hkv={Hkv} D={Dh}", flush=True)
+    out = paged_flash_attention_prefill(*d, None, case.scale, page)
+    ref = paged_attention_ref(case.q, case.k_cache, case.v_cache, case.block_tables, case.context_lens, case.cu,
+                              case.scale).nan_to_num(0.0)  # (a query without keys: 0/0 there, a zero row here)
+    assert torch.isfinite(out).all()
+    plain = torch.empty_like(out)
+    D = _lib.describe
+    rc = _lib.load().paged_attention_prefill(*(D(t) for t in d), D(plain), max(new), float(case.scale),
+                                             _lib.stream_handle(plain.device))
+    _lib.check("paged_attention_prefill", rc)
+    for got, want in ((out.cpu(), ref), (out.cpu(), plain.cpu())):
+        assert_out_close(got, want)
+        err = (got.double() - want.double()).norm() / want.double().norm().clamp_min(1e-12)
+        assert err < 5e-3, f"relative error norm {err:.3e}"
