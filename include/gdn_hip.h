@@ -276,6 +276,14 @@ int gdn_gating(const gdn_tensor* a, const gdn_tensor* b, const gdn_tensor* A_log
 int flash_attention_varlen(const gdn_tensor* q, const gdn_tensor* k, const gdn_tensor* v,
                            const gdn_tensor* cu_seqlens, gdn_tensor* out, int64_t max_seqlen, float scale,
                            int32_t causal, void* stream);
+/*
+ * The same for any head dim D that is a multiple of 8 up to 256 (the vision
+ * tower's 72), read as it lies; the token strides of k and v must be at least
+ * D (GDN_ERR_STRIDE).
+ */
+int flash_attention_varlen_any_dim(const gdn_tensor* q, const gdn_tensor* k, const gdn_tensor* v,
+                                   const gdn_tensor* cu_seqlens, gdn_tensor* out, int64_t max_seqlen, float scale,
+                                   int32_t causal, void* stream);
 
 /*
  * paged_attention_prefill <- paged_flash_attention_prefill, ops/full_attention.py:454-512

@@ -43,6 +43,7 @@ EXPORTED_SYMBOLS = (
     "gdn_rms_norm_gated",
     "gdn_gating",
     "flash_attention_varlen",
+    "flash_attention_varlen_any_dim",
     "paged_attention_prefill",
     "paged_attention_prefill_workspace_size",
     "paged_attention_prefill_split",
@@ -119,6 +120,8 @@ def load() -> ctypes.CDLL:
         lib.flash_attention_varlen.restype = ctypes.c_int
         lib.flash_attention_varlen.argtypes = [_PT] * 5 + [ctypes.c_int64, ctypes.c_float, ctypes.c_int32,
                                                            ctypes.c_void_p]
+        lib.flash_attention_varlen_any_dim.restype = ctypes.c_int
+        lib.flash_attention_varlen_any_dim.argtypes = lib.flash_attention_varlen.argtypes
         lib.paged_attention_prefill.restype = ctypes.c_int
         lib.paged_attention_prefill.argtypes = [_PT] * 7 + [ctypes.c_int64, ctypes.c_float, ctypes.c_void_p]
         lib.paged_attention_prefill_workspace_size.restype = ctypes.c_int64

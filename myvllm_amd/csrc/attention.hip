@@ -113,6 +113,7 @@ struct AttnArgs {
   PagedTable tab;
   int64_t T, nseq;
   int32_t Hq, Hkv, gh;  // gh: query heads per workgroup (1, 2 or 4)
+  int32_t dim;          // head dim (a multiple of 8, at most the kernel's D)
   float c;              // softmax scale * log2(e)
   bool cu64, ctx64, causal;
   // split prefill: key tiles of a piece (even), (tile, head group) rows of the
@@ -174,16 +175,25 @@ __device__ __attribute__((always_inline)) SeqTile attn_tile_lookup(const void* c
 // piece -> split): four prompts of 800 to 1,500 tokens over prefixes of 500 to
 // 15,800 keys 1,192 -> 951 us (574 -> 720 TFLOP/s), one of 512 over 8,000 98 ->
 // 47 us, five of 18 over 11,700 301 -> 64 us.
-template <typename T, int D, int BN, int PG, bool SPLIT>
+template <typename T, int D, int BN, int PG, bool SPLIT, int DQ = 0>
 __global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnArgs a) {
   constexpr bool PAGED = PG != 0;
+  // DQ > 0: head dims of a.dim <= DQ <= D elements (packed rows only), a
+  // multiple of 8.  The rows are read as they lie and the 16-byte pieces past
+  // a.dim become zeros on the way (query pieces by a select, key and value
+  // pieces by an offset past the buffer's range), so nothing is padded in
+  // memory; the score product runs over DQ dims, P V over D.  Six images of
+  // 450 to 2,900 patches, 16 heads of 72: 306 -> 122 us against padded copies
+  // at D = 128 (40 us of copies, and the MFMAs and fragment reads of 56 dims).
+  constexpr bool RAG = DQ > 0;
+  static_assert(!RAG || (PG == 0 && DQ <= D && DQ % 16 == 0), "ragged head dims are packed rows");
   static_assert(!SPLIT || PG >= 2, "split rows are paged rows of whole 16-row groups");
   typedef Mma<T> M;
   typedef typename M::v8 v8;
   typedef typename M::v4 v4;
   constexpr int LDK = D + 8;   // row stride (elements): 16-byte row skew for the b128 reads
-  constexpr int LDV = D + 32;  // 64-byte row skew for the transposed reads
-  constexpr int NKS = D / 16;
+  constexpr int LDV = D == 96 ? D : D + 32;  // 64 bytes of row skew modulo the banks for the transposed reads
+  constexpr int NKS = (RAG ? DQ : D) / 16;
   constexpr int NA = BN / 32;
   constexpr int NDT = D / 32;
   constexpr int CH = D / 8;  // 16-byte chunks per row
@@ -264,7 +274,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnArgs a) {
   {
     const T* qp = reinterpret_cast<const T*>(a.q) + (s0 + (qvalid ? qi : 0)) * a.q_st + (int64_t)head * a.q_sh + 8 * hh;
 #pragma unroll
-    for (int s = 0; s < NKS; ++s) qf[s] = *reinterpret_cast<const v8*>(qp + 16 * s);
+    for (int s = 0; s < NKS; ++s) qf[s] = *reinterpret_cast<const v8*>(qp + (!RAG || 16 * s + 8 * hh < a.dim ? 16 * s : 0));
   }
   // the softmax below assumes c > 0: a negative scale is folded into q (an
   // exact sign flip), a zero scale is q = 0 with c = 1 (equal weights)
@@ -272,7 +282,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnArgs a) {
   T* const qw = qs + (QL ? w * 32 * LDK : 0);  // this wave's query rows (only the wave reads them)
   auto stage_q = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int s = 0; s < NKS; ++s) qf[s] = qvalid ? qf[s] : v8{};
+    for (int s = 0; s < NKS; ++s) qf[s] = qvalid && (!RAG || 16 * s + 8 * hh < a.dim) ? qf[s] : v8{};
     if (c <= 0.f) {
 #pragma unroll
       for (int s = 0; s < NKS; ++s) qf[s] = c < 0.f ? -qf[s] : v8{};
@@ -293,7 +303,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnArgs a) {
   const char* const kseq = a.k.base + s0 * a.k.st + kvh * a.k.sh;
   const char* const vseq = a.v.base + s0 * a.v.st + kvh * a.v.sh;
   constexpr int NG = BN / 16;  // 16-row groups of a tile
-  static_assert(CH >= 8 && 64 % CH == 0, "a wave's rows of a tile lie in one 16-row group");
+  static_assert(PG == 0 || (CH >= 8 && 64 % CH == 0), "a wave's rows of a tile lie in one 16-row group");
   // PG 2, 3: each 16-row group of a tile lies in one page.  Its block id is a
   // vector load issued one tile ahead, before the previous tile's data loads,
   // so waiting for it leaves those data loads in flight (a scalar load would
@@ -418,8 +428,10 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnArgs a) {
       if (!PAGED) {
         // (the row offset times the stride fits 32 bits: the launcher checks
         // max(max_seqlen, 64) rows of either stride against 2^31)
-        kd[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rkt, (uint32_t)row * kst + 16u * ch, 0, 0));
-        vd[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rvt, (uint32_t)row * vst + 16u * ch, 0, 0));
+        // (ranges are below 2^31 bytes, so 2^31 more is past them whatever the row)
+        const uint32_t co = !RAG || 8 * ch < a.dim ? 16u * ch : 0x80000000u;
+        kd[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rkt, (uint32_t)row * kst + co, 0, 0));
+        vd[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rvt, (uint32_t)row * vst + co, 0, 0));
         continue;
       }
       const char* pk = j < kend ? kv_row<PAGED>(a.k, a.tab, n, s0, j, kvh) : nullptr;
@@ -632,7 +644,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnArgs a) {
     for (int r0 = 0; r0 < 32; r0 += RPP) {
       const int r = r0 + rsub;
       const v8 ov = *reinterpret_cast<const v8*>(qw + r * LDK + 8 * cpos);
-      if (r < qrem) *reinterpret_cast<v8*>(orow + (int64_t)r * a.o_st) = ov;
+      if (r < qrem && (!RAG || 8 * cpos < a.dim)) *reinterpret_cast<v8*>(orow + (int64_t)r * a.o_st) = ov;
     }
   } else if (qvalid) {
     T* op = reinterpret_cast<T*>(a.o) + (s0 + qi) * a.o_st + (int64_t)head * a.o_sh + 4 * hh;
@@ -640,6 +652,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnArgs a) {
     for (int d = 0; d < NDT; ++d)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
+        if (RAG && 32 * d + 8 * g >= a.dim) break;
         v4 ov;
 #pragma unroll
         for (int e = 0; e < 4; ++e) ov[e] = (T)(oacc[d][4 * g + e] * inv);
@@ -1212,21 +1225,21 @@ PagedTable paged_table(const gdn_tensor* tab, const gdn_tensor* kc) {
   return p;
 }
 
-template <typename T, int D, int BN, bool PAGED>
+template <typename T, int D, int BN, bool PAGED, int DQ = 0>
 hipError_t launch_prefill_t(const AttnArgs& a, int64_t nseq, int64_t max_len, hipStream_t st) {
   const int qsubs = 4 / a.gh;
   // output rows no sequence covers are zero, as the reference allocates o
   // zero-filled (ops/full_attention.py:467); a kernel of its own, launched
   // first (a call inside the attention kernel changed its register allocation
   // and cost it about a fifth of its speed)
-  zero_uncovered_rows_kernel<(int)sizeof(T)><<<dim3(64), dim3(256), 0, st>>>(a.o, a.o_st, a.o_sh, a.Hq, D, a.cu,
+  zero_uncovered_rows_kernel<(int)sizeof(T)><<<dim3(64), dim3(256), 0, st>>>(a.o, a.o_st, a.o_sh, a.Hq, a.dim, a.cu,
                                                                              a.cu64, a.nseq, a.T);
   if (nseq <= 0 || max_len <= 0) return hipGetLastError();
   // query tiles: at most T / tile_len + one partial tile per sequence
   const int64_t tiles = a.T / (32 * qsubs) + nseq;
   const dim3 grid((unsigned)(tiles * (a.Hq / a.gh)));
   if constexpr (!PAGED) {
-    hipLaunchKernelGGL((attn_prefill_kernel<T, D, BN, 0, false>), grid, dim3(256), 0, st, a);
+    hipLaunchKernelGGL((attn_prefill_kernel<T, D, BN, 0, false, DQ>), grid, dim3(256), 0, st, a);
   } else if (a.tab.page % 16 == 0 && a.k.sb < (int64_t(1) << 32) && a.v.sb < (int64_t(1) << 32) && a.tab.cols > 0 &&
              a.tab.cols * a.tab.page < (int64_t(1) << 31) && a.tab.num_blocks < (int64_t(1) << 31)) {
     // whole 16-row groups per page, 32-bit table arithmetic
@@ -1250,8 +1263,24 @@ hipError_t launch_prefill_t(const AttnArgs& a, int64_t nseq, int64_t max_len, hi
   return hipGetLastError();
 }
 
+// Packed rows of any head dim that is a multiple of 8 up to 256: the next
+// larger tile (the score product in steps of 16 dims, P V in steps of 32).
+template <typename T>
+hipError_t launch_prefill_ragged(const AttnArgs& a, int64_t nseq, int64_t max_len, hipStream_t st) {
+  if (a.dim <= 64) return launch_prefill_t<T, 64, 64, false, 64>(a, nseq, max_len, st);
+  if (a.dim <= 80) return launch_prefill_t<T, 96, 64, false, 80>(a, nseq, max_len, st);
+  if (a.dim <= 96) return launch_prefill_t<T, 96, 64, false, 96>(a, nseq, max_len, st);
+  if (a.dim <= 128) return launch_prefill_t<T, 128, 64, false, 128>(a, nseq, max_len, st);
+  return launch_prefill_t<T, 256, 32, false, 256>(a, nseq, max_len, st);
+}
+
 template <bool PAGED>
 hipError_t launch_prefill(const AttnArgs& a, int dtype, int D, int64_t nseq, int64_t max_len, hipStream_t st) {
+  if constexpr (!PAGED) {
+    if (D != 64 && D != 128 && D != 256)
+      return dtype == GDN_DTYPE_BF16 ? launch_prefill_ragged<bf16_t>(a, nseq, max_len, st)
+                                     : launch_prefill_ragged<f16_t>(a, nseq, max_len, st);
+  }
   if (dtype == GDN_DTYPE_BF16) {
     if (D == 64) return launch_prefill_t<bf16_t, 64, 64, PAGED>(a, nseq, max_len, st);
     if (D == 128) return launch_prefill_t<bf16_t, 128, 64, PAGED>(a, nseq, max_len, st);
@@ -1353,6 +1382,7 @@ hipError_t attn_varlen_prefill_launch(const gdn_tensor* q, const gdn_tensor* k, 
   a.T = q->shape[0];
   a.nseq = nseq;
   a.Hq = (int32_t)q->shape[1];
+  a.dim = (int32_t)q->shape[2];
   a.Hkv = (int32_t)k->shape[1];
   a.gh = heads_per_group(a.Hq / a.Hkv);
   a.c = scale * kLog2e;
@@ -1392,6 +1422,7 @@ hipError_t attn_paged_prefill_launch(const gdn_tensor* q, const gdn_tensor* kc, 
   a.T = q->shape[0];
   a.nseq = nseq;
   a.Hq = (int32_t)q->shape[1];
+  a.dim = (int32_t)q->shape[2];
   a.Hkv = (int32_t)kc->shape[2];
   a.gh = heads_per_group(a.Hq / a.Hkv);
   a.c = scale * kLog2e;

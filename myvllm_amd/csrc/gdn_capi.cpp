@@ -270,7 +270,7 @@ constexpr int32_t kMaxDecodeSplits = 256;
 // q / out (rows, Hq, D) with the kv tensors' head count and head dim: bf16 or
 // fp16 throughout, D = 64, 128 or 256, unit inner strides, 16-byte rows.
 int check_attn_qo(const gdn_tensor* q, const gdn_tensor* out, const gdn_tensor* kv0, const gdn_tensor* kv1,
-                  int64_t Hkv) {
+                  int64_t Hkv, bool any_dim = false) {
   const int64_t rows = q->shape[0], Hq = q->shape[1], D = q->shape[2];
   if (out->shape[0] != rows || out->shape[1] != Hq || out->shape[2] != D) return GDN_ERR_SHAPE;
   const int kd = kv0->ndim - 1;
@@ -278,7 +278,7 @@ int check_attn_qo(const gdn_tensor* q, const gdn_tensor* out, const gdn_tensor* 
   if (Hkv <= 0 || Hq <= 0 || Hq % Hkv != 0) return GDN_ERR_HEADS;
   if (q->dtype != GDN_DTYPE_BF16 && q->dtype != GDN_DTYPE_F16) return GDN_ERR_DTYPE;
   if (kv0->dtype != q->dtype || kv1->dtype != q->dtype || out->dtype != q->dtype) return GDN_ERR_DTYPE;
-  if (D != 64 && D != 128 && D != 256) return GDN_ERR_HEAD_DIM;
+  if (any_dim ? (D <= 0 || D > 256 || D % 8 != 0) : (D != 64 && D != 128 && D != 256)) return GDN_ERR_HEAD_DIM;
   if (q->stride[2] != 1 || out->stride[2] != 1 || kv0->stride[kd] != 1 || kv1->stride[kd] != 1)
     return GDN_ERR_STRIDE;
   if (numel(q) > 0 && (!vec_ok(q, 16) || !vec_ok(out, 16))) return GDN_ERR_ALIGN;
@@ -447,9 +447,9 @@ GDN_EXPORT int gdn_gating(const gdn_tensor* a, const gdn_tensor* b, const gdn_te
   return launch_rc(gdn_gating_launch(a, b, A_log, dt_bias, g, beta, reinterpret_cast<hipStream_t>(stream)));
 }
 
-GDN_EXPORT int flash_attention_varlen(const gdn_tensor* q, const gdn_tensor* k, const gdn_tensor* v,
-                                      const gdn_tensor* cu_seqlens, gdn_tensor* out, int64_t max_seqlen, float scale,
-                                      int32_t causal, void* stream) {
+namespace {
+int varlen_prefill(const gdn_tensor* q, const gdn_tensor* k, const gdn_tensor* v, const gdn_tensor* cu_seqlens,
+                   gdn_tensor* out, int64_t max_seqlen, float scale, int32_t causal, void* stream, bool any_dim) {
   GDN_TRY(check_desc(q, 3));
   GDN_TRY(check_desc(k, 3));
   GDN_TRY(check_desc(v, 3));
@@ -457,9 +457,11 @@ GDN_EXPORT int flash_attention_varlen(const gdn_tensor* q, const gdn_tensor* k, 
   GDN_TRY(check_desc(cu_seqlens, 1));
   if (k->shape[0] != q->shape[0] || v->shape[0] != q->shape[0] || v->shape[1] != k->shape[1]) return GDN_ERR_SHAPE;
   if (cu_seqlens->shape[0] < 1 || max_seqlen < 0) return GDN_ERR_SHAPE;
-  GDN_TRY(check_attn_qo(q, out, k, v, k->shape[1]));
+  GDN_TRY(check_attn_qo(q, out, k, v, k->shape[1], any_dim));
   if (!is_index(cu_seqlens->dtype)) return GDN_ERR_DTYPE;
   if (cu_seqlens->stride[0] != 1) return GDN_ERR_STRIDE;
+  // (a key tile's range is its rows times their stride: a row has to lie inside its stride)
+  if (any_dim && (k->stride[0] < q->shape[2] || v->stride[0] < q->shape[2])) return GDN_ERR_STRIDE;
   const int64_t R = q->shape[1] / k->shape[1];
   const int64_t gh = R % 4 == 0 ? 4 : (R % 2 == 0 ? 2 : 1);
   if (cu_seqlens->shape[0] - 1 > kMaxGridYZ || q->shape[1] / gh > kMaxGridYZ || max_seqlen / 32 > kMaxGrid)
@@ -471,6 +473,19 @@ GDN_EXPORT int flash_attention_varlen(const gdn_tensor* q, const gdn_tensor* k, 
     return GDN_ERR_RANGE;
   return launch_rc(attn_varlen_prefill_launch(q, k, v, cu_seqlens, out, max_seqlen, scale, causal,
                                               reinterpret_cast<hipStream_t>(stream)));
+}
+}  // namespace
+
+GDN_EXPORT int flash_attention_varlen(const gdn_tensor* q, const gdn_tensor* k, const gdn_tensor* v,
+                                      const gdn_tensor* cu_seqlens, gdn_tensor* out, int64_t max_seqlen, float scale,
+                                      int32_t causal, void* stream) {
+  return varlen_prefill(q, k, v, cu_seqlens, out, max_seqlen, scale, causal, stream, false);
+}
+
+GDN_EXPORT int flash_attention_varlen_any_dim(const gdn_tensor* q, const gdn_tensor* k, const gdn_tensor* v,
+                                              const gdn_tensor* cu_seqlens, gdn_tensor* out, int64_t max_seqlen,
+                                              float scale, int32_t causal, void* stream) {
+  return varlen_prefill(q, k, v, cu_seqlens, out, max_seqlen, scale, causal, stream, true);
 }
 
 namespace {

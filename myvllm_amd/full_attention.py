@@ -71,28 +71,43 @@ def flash_attention_prefill(
     dev = _lib.require_device(q, k, v, cu_seqlens)
     if max_seqlen is None:
         max_seqlen = _max_seqlen(cu_seqlens)
-    if head_dim not in _KERNEL_HEAD_DIMS or head_v_dim != head_dim:
+    own = head_dim in _KERNEL_HEAD_DIMS and head_v_dim == head_dim
+    if not own and not _direct_head_dim(q, k, v, head_dim, head_v_dim, max_seqlen):
         return _padded_prefill(q, k, v, cu_seqlens, scale, head_dim, head_v_dim, is_causal, max_seqlen, out)
     q, k, v = _lib.vec16(q), _lib.vec16(k), _lib.vec16(v)
     o = _out_for(out, (q.shape[0], q.shape[1], head_v_dim), q.dtype, dev)
     D = _lib.describe
-    rc = _lib.load().flash_attention_varlen(
+    name = "flash_attention_varlen" if own else "flash_attention_varlen_any_dim"
+    rc = getattr(_lib.load(), name)(
         D(q), D(k), D(v), D(cu_seqlens), D(o), int(max_seqlen), float(scale), int(bool(is_causal)),
         _lib.stream_handle(dev),
     )
-    _lib.check("flash_attention_varlen", rc)
+    _lib.check(name, rc)
     return _finish(out, o)
 
 
 _KERNEL_HEAD_DIMS = (64, 128, 256)
 
 
+def _direct_head_dim(q, k, v, head_dim, head_v_dim, max_seqlen) -> bool:
+    """Whether the kernels of any head dim read q, k and v as they lie: 16-bit
+    rows of a multiple of 8 elements (the vision tower's 1152 / 16 = 72,
+    ``models/qwen/vision.py:18``, ``configs/qwen3_5.py:11``, ``:16``), each
+    inside its token stride, within the kernels' 32-bit offsets.  The rest is
+    padded: other dims, v narrower or wider than k, overlapping rows."""
+    if head_dim != head_v_dim or head_dim % 8 or not 0 < head_dim <= _KERNEL_HEAD_DIMS[-1]:
+        return False
+    if q.dim() != 3 or k.dim() != 3 or v.dim() != 3 or k.shape[0] != q.shape[0] or v.shape != k.shape:
+        return False
+    st = max(k.stride(0), v.stride(0), k.shape[1] * head_dim)
+    return min(k.stride(0), v.stride(0)) >= head_dim and max(max_seqlen, 64) * st * q.element_size() < 2**31
+
+
 def _padded_prefill(q, k, v, cu_seqlens, scale, head_dim, head_v_dim, is_causal, max_seqlen, out):
-    """Head dims the kernel has no instantiation for (the vision tower's
-    1152 / 16 = 72, ``models/qwen/vision.py:18``, ``configs/qwen3_5.py:11``,
-    ``:16``) run zero-padded to the next of 64, 128 and 256: zero dims add
-    nothing to q.k and give zero output columns, which are dropped.  The
-    padded copies cost one pass over q, k and v."""
+    """Head dims no kernel reads as they lie (:func:`_direct_head_dim`) run
+    zero-padded to the next of 64, 128 and 256: zero dims add nothing to q.k
+    and give zero output columns, which are dropped.  The padded copies cost
+    one pass over q, k and v."""
     Dp = next((d for d in _KERNEL_HEAD_DIMS if d >= max(head_dim, head_v_dim)), None)
     if Dp is None:
         raise ValueError(f"head dims {head_dim}/{head_v_dim} above {_KERNEL_HEAD_DIMS[-1]} are not supported")

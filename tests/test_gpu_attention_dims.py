@@ -1,0 +1,63 @@
+"""GPU: packed attention at head dims the kernels read as they lie (any
+multiple of 8, no padded copies) vs the fp64 oracle, with the attention
+tests' bars.  k and v are views of one interleaved buffer whose gaps hold NaN
+and infinities, so that a piece read past a row's end would show."""
+import pytest
+import torch
+
+from conftest import assert_out_close
+from myvllm_amd import _lib, flash_attention_prefill
+from myvllm_amd.full_attention import _direct_head_dim
+from myvllm_amd.workloads import attn_varlen_case
+from oracle.attention import flash_attention_prefill_ref
+
+
+def test_direct_head_dim_rule():
+    """Rows of a multiple of 8 elements inside their stride go as they lie, the rest is padded."""
+    def rule(D, Dv=None, stride=None, T=10, max_seqlen=10):
+        t = torch.empty(T, 2, D, dtype=torch.bfloat16)
+        kv = t if stride is None else torch.empty(T * max(stride, 1) + 4 * D,
+                                                  dtype=torch.bfloat16).as_strided((T, 2, D), (stride, D, 1))
+        return _direct_head_dim(t, kv, kv, D, D if Dv is None else Dv, max_seqlen)
+
+    assert rule(72) and rule(8) and rule(248) and rule(72, stride=72)
+    assert not rule(72, Dv=64) and not rule(12) and not rule(264) and not rule(0)
+    assert not rule(72, stride=64) and not rule(72, stride=0)  # overlapping rows
+    assert not rule(72, max_seqlen=2**24)  # past 32-bit offsets
+
+
+@pytest.mark.parametrize("stride", [64, 0])
+def test_any_dim_refuses_overlapping_rows(stride):
+    D = _lib.describe
+    q = torch.zeros(8, 2, 72, dtype=torch.bfloat16)
+    k = D(q)
+    k.stride[0] = stride
+    cu = torch.tensor([0, 8], dtype=torch.int32)
+    rc = _lib.load().flash_attention_varlen_any_dim(D(q), k, D(q), D(cu), D(q), 8, 1.0, 1, None)
+    assert rc == _lib.load().flash_attention_varlen_any_dim(D(q), D(q), k, D(cu), D(q), 8, 1.0, 1, None)
+    assert "stride" in _lib.strerror(rc).lower()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Dh", [8, 40, 64 + 8, 80, 88, 96, 104, 120, 136, 200, 248])
+@pytest.mark.parametrize("Hq, Hkv, causal, dtype", [(4, 4, False, torch.bfloat16), (8, 2, True, torch.float16)])
+def test_any_head_dim(dev, Dh, Hq, Hkv, causal, dtype):
+    lengths = [1, 64, 31, 200, 65]
+    case = attn_varlen_case(lengths, seed=Dh + Hq, Hq=Hq, Hkv=Hkv, D=Dh, dtype=dtype)
+    T = sum(lengths)
+    print(f"any head dim {Dh} Hq={Hq} Hkv={Hkv} causal={causal} {dtype}", flush=True)
+    ref = flash_attention_prefill_ref(case.q, case.k, case.v, case.cu, case.scale, is_causal=causal)
+    # rows of k and v heads apart by gaps of NaN and +-inf, more past the end
+    gap = torch.tensor([float("nan"), float("inf"), -float("inf"), 65504.0], dtype=dtype).repeat(4)
+    buf = gap.repeat((T + 4) * 2 * Hkv, 1 + Dh // 16 + 1)[:, : Dh + 16].reshape(T + 4, 2 * Hkv, Dh + 16).contiguous()
+    buf[:T, :Hkv, :Dh] = case.k
+    buf[:T, Hkv:, :Dh] = case.v
+    buf = buf.to(dev)
+    k, v = buf[:T, :Hkv, :Dh], buf[:T, Hkv:, :Dh]
+    out = torch.full((T, Hq, Dh + 8), 7.0, dtype=dtype, device=dev)
+    got = flash_attention_prefill(case.q.to(dev), k, v, case.cu.to(dev), case.scale, Hq, Hkv, Dh, Dh, causal,
+                                  out=out[..., :Dh])
+    assert got.data_ptr() == out.data_ptr() and (out[..., Dh:] == 7.0).all()
+    assert_out_close(got, ref)
+    err = (got.double().cpu() - ref.double()).norm() / ref.double().norm()
+    assert err < 5e-3, f"relative error norm {err:.3e}"
