@@ -175,8 +175,16 @@ __device__ __attribute__((always_inline)) SeqTile attn_tile_lookup(const void* c
 // piece -> split): four prompts of 800 to 1,500 tokens over prefixes of 500 to
 // 15,800 keys 1,192 -> 951 us (574 -> 720 TFLOP/s), one of 512 over 8,000 98 ->
 // 47 us, five of 18 over 11,700 301 -> 64 us.
+//
+// Key tiles: 32 keys, which at D = 64 and 128 leave room for two waves per
+// SIMD (at least) whose softmax and MFMAs overlap; D = 96 fits two with 64.
+// At D = 128 tiles of 64 keys took 259 to 280 registers, one wave per SIMD:
+// eight prompts of 512 to 4,096 tokens (16 / 4 heads) 363 -> 254 us, with 64
+// keys held to 256 registers 259; eight chunks over up to 4,096 cached keys
+// 563 -> 329 us (345).  D = 64: 180 -> 165 us.  D = 96 (vision): 64 keys 142,
+// 32 keys 157, three waves per SIMD 158 (32 keys) and 197 (64, spills).
 template <typename T, int D, int BN, int PG, bool SPLIT, int DQ = 0>
-__global__ __launch_bounds__(256) void attn_prefill_kernel(const AttnArgs a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 1 : 2))) void attn_prefill_kernel(const AttnArgs a) {
   constexpr bool PAGED = PG != 0;
   // DQ > 0: head dims of a.dim <= DQ <= D elements (packed rows only), a
   // multiple of 8.  The rows are read as they lie and the 16-byte pieces past
@@ -1267,10 +1275,10 @@ hipError_t launch_prefill_t(const AttnArgs& a, int64_t nseq, int64_t max_len, hi
 // larger tile (the score product in steps of 16 dims, P V in steps of 32).
 template <typename T>
 hipError_t launch_prefill_ragged(const AttnArgs& a, int64_t nseq, int64_t max_len, hipStream_t st) {
-  if (a.dim <= 64) return launch_prefill_t<T, 64, 64, false, 64>(a, nseq, max_len, st);
+  if (a.dim <= 64) return launch_prefill_t<T, 64, 32, false, 64>(a, nseq, max_len, st);
   if (a.dim <= 80) return launch_prefill_t<T, 96, 64, false, 80>(a, nseq, max_len, st);
   if (a.dim <= 96) return launch_prefill_t<T, 96, 64, false, 96>(a, nseq, max_len, st);
-  if (a.dim <= 128) return launch_prefill_t<T, 128, 64, false, 128>(a, nseq, max_len, st);
+  if (a.dim <= 128) return launch_prefill_t<T, 128, 32, false, 128>(a, nseq, max_len, st);
   return launch_prefill_t<T, 256, 32, false, 256>(a, nseq, max_len, st);
 }
 
@@ -1282,12 +1290,12 @@ hipError_t launch_prefill(const AttnArgs& a, int dtype, int D, int64_t nseq, int
                                      : launch_prefill_ragged<f16_t>(a, nseq, max_len, st);
   }
   if (dtype == GDN_DTYPE_BF16) {
-    if (D == 64) return launch_prefill_t<bf16_t, 64, 64, PAGED>(a, nseq, max_len, st);
-    if (D == 128) return launch_prefill_t<bf16_t, 128, 64, PAGED>(a, nseq, max_len, st);
+    if (D == 64) return launch_prefill_t<bf16_t, 64, 32, PAGED>(a, nseq, max_len, st);
+    if (D == 128) return launch_prefill_t<bf16_t, 128, 32, PAGED>(a, nseq, max_len, st);
     return launch_prefill_t<bf16_t, 256, 32, PAGED>(a, nseq, max_len, st);
   }
-  if (D == 64) return launch_prefill_t<f16_t, 64, 64, PAGED>(a, nseq, max_len, st);
-  if (D == 128) return launch_prefill_t<f16_t, 128, 64, PAGED>(a, nseq, max_len, st);
+  if (D == 64) return launch_prefill_t<f16_t, 64, 32, PAGED>(a, nseq, max_len, st);
+  if (D == 128) return launch_prefill_t<f16_t, 128, 32, PAGED>(a, nseq, max_len, st);
   return launch_prefill_t<f16_t, 256, 32, PAGED>(a, nseq, max_len, st);
 }
 
@@ -1314,7 +1322,7 @@ PrefillSplit prefill_split(int64_t T, int64_t nseq, int64_t Hq, int64_t Hkv, int
   PrefillSplit r{1, 0, 0};
   if (T <= 0 || nseq <= 0 || Hkv <= 0 || cap <= 0) return r;
   const int gh = heads_per_group((int)(Hq / Hkv));
-  const int BN = D == 256 ? 32 : 64;
+  constexpr int BN = 32;
   r.rows = (T / (32 * (4 / gh)) + nseq) * (Hq / gh);
   const int64_t nt = (cap + BN - 1) / BN;
   const double slots = D == 256 ? kSlots : 2 * kSlots;  // D <= 128: two workgroups fit a CU
