@@ -149,17 +149,43 @@ GDN_DEVICE const char* kv_row(const KvSource& s, const PagedTable& tb, int64_t n
 // PG: 0 packed rows, 1 paged (any page size: a table lookup per row),
 // 2 / 3 paged with a page size that is a multiple of 16 and an int32 / int64
 // block table (one lookup per 16 rows, a tile ahead, 32-bit arithmetic)
-// Workgroup id -> (sequence, query tile): tiles of tile_len queries, laid out
-// sequence after sequence over the tiles that exist (no workgroup of a
-// padded grid exits idle).  Out of line, so that the lookup's registers and
-// barriers leave the kernel's own allocation alone.
+// Workgroup id -> (sequence, query tile): tiles of tile_len queries (a power
+// of two), laid out sequence after sequence over the tiles that exist (no
+// workgroup of a padded grid exits idle).  Below D = 256 batches of up to 64
+// sequences go longest first (by keys, ties by index), so that what runs last
+// is short: every lane ranks one sequence against the others and sums the
+// tiles before it, with no barrier.  Six images of 450 to 2,900 patches 143 ->
+// 137 us, eight causal prompts of 512 to 4,096 tokens 171 -> 159 (D = 64) and
+// 259 -> 247 (128), eight chunks over up to 4,096 cached keys 340 -> 331 (128).
+// Larger batches, and D = 256 (sixteen prompts: 974 in index order, 985
+// ranked), are taken in index order by a scan over the workgroup.
 struct SeqTile {
   int64_t seq, tile;
 };
-__device__ __attribute__((always_inline)) SeqTile attn_tile_lookup(const void* cu, bool cu64, int64_t nseq, int64_t T,
-                                                              int tile_len, int64_t target, int32_t* lds) {
+template <int D, bool PAGED>
+GDN_DEVICE SeqTile attn_tile_lookup(const AttnArgs& a, int tile_len, int64_t target, int32_t* lds) {
   SeqTile r;
-  find_seq_tile<256>(cu, cu64, nseq, T, tile_len, target, r.seq, r.tile, lds);
+  if (D < 256 && a.nseq <= 64) {
+    const int lane = threadIdx.x & 63, sh = __builtin_ctz(tile_len);
+    int nt = 0, key = 0;
+    if (lane < a.nseq) {
+      int64_t s, e;
+      seq_range(a.cu, a.cu64, lane, a.T, s, e);
+      nt = (int)((e - s + tile_len - 1) >> sh);
+      key = PAGED ? (int)clamp64(load_index(a.ctx, lane, a.ctx64), 0, 0x7fffffff) : (int)(e - s);
+    }
+    int base = 0;
+    for (int j = 0; j < (int)a.nseq; ++j) {
+      const int kj = __builtin_amdgcn_readlane(key, j), tj = __builtin_amdgcn_readlane(nt, j);
+      base += kj > key || (kj == key && j < lane) ? tj : 0;
+    }
+    const int t = (int)target - base;
+    const uint64_t own = __builtin_amdgcn_ballot_w64(t >= 0 && t < nt);
+    r.seq = own ? __builtin_ctzll(own) : -1;
+    r.tile = own ? __builtin_amdgcn_readlane(t, (int)r.seq) : 0;
+    return r;
+  }
+  find_seq_tile<256>(a.cu, a.cu64, a.nseq, a.T, tile_len, target, r.seq, r.tile, lds);
   return r;
 }
 
@@ -234,7 +260,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   const int hg = a.Hq / gh;  // head groups
   const uint32_t piece = SPLIT ? blockIdx.x / (uint32_t)a.rows : 0u;
   const uint32_t row_id = SPLIT ? blockIdx.x - piece * (uint32_t)a.rows : blockIdx.x;
-  const SeqTile st = attn_tile_lookup(a.cu, a.cu64, a.nseq, a.T, 32 * qsubs, row_id / hg, lookup);
+  const SeqTile st = attn_tile_lookup<D, PAGED>(a, 32 * qsubs, row_id / hg, lookup);
   if (st.seq < 0) return;
   const int64_t n = st.seq;
   const int y = (int)(row_id % hg);
@@ -679,7 +705,7 @@ __global__ __launch_bounds__(256) void attn_prefill_combine_kernel(const AttnArg
   __shared__ int32_t lookup[8];
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int R = a.Hq / a.Hkv, gh = a.gh, qsubs = 4 / gh, groups = R / gh, hg = a.Hq / gh;
-  const SeqTile st = attn_tile_lookup(a.cu, a.cu64, a.nseq, a.T, 32 * qsubs, blockIdx.x / hg, lookup);
+  const SeqTile st = attn_tile_lookup<D, true>(a, 32 * qsubs, blockIdx.x / hg, lookup);
   if (st.seq < 0) return;
   const int y = (int)(blockIdx.x % hg);
   const int head = (y / groups) * R + (y % groups) * gh + (w % gh);

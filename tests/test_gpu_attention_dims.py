@@ -61,3 +61,17 @@ def test_any_head_dim(dev, Dh, Hq, Hkv, causal, dtype):
     assert_out_close(got, ref)
     err = (got.double().cpu() - ref.double()).norm() / ref.double().norm()
     assert err < 5e-3, f"relative error norm {err:.3e}"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N", [1, 63, 64, 65])  # ranked by length up to 64 sequences, in index order past that
+@pytest.mark.parametrize("Dh", [64, 72, 128])
+def test_sequence_order(dev, N, Dh):
+    """Ragged batches with empty and equal sequences on both sides of the ranking's limit."""
+    lengths = [(37 * n * n + 11) % 150 if n % 7 else 0 for n in range(N)] if N > 1 else [129]
+    lengths[N // 2] = lengths[-1] = 33
+    case = attn_varlen_case(lengths, seed=N + Dh, Hq=4, Hkv=1, D=Dh)
+    print(f"sequence order N={N} D={Dh}", flush=True)
+    got = flash_attention_prefill(case.q.to(dev), case.k.to(dev), case.v.to(dev), case.cu.to(dev), case.scale, 4, 1, Dh,
+                                  Dh, True)
+    assert_out_close(got, flash_attention_prefill_ref(case.q, case.k, case.v, case.cu, case.scale))
