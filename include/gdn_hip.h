@@ -140,6 +140,26 @@ int gdn_chunk_prefill(const gdn_tensor* q, const gdn_tensor* k, const gdn_tensor
                       gdn_tensor* out, float scale, int32_t chunk_size, void* stream);
 
 /*
+ * gdn_chunk_prefill in two launches over a workspace, for batches of few
+ * sequences (no counterpart in the reference): what does not depend on the
+ * state is computed for all chunks at once, then each sequence and head is
+ * walked by eight workgroups.  The result is gdn_chunk_prefill's to the
+ * rounding of its operands' splits.
+ *   gdn_chunk_prefill_workspace_size: floats of workspace with which a batch
+ *     of T tokens in num_seqs sequences runs so; 0 where gdn_chunk_prefill is
+ *     the faster one (no workspace is read then, and the call is the same).
+ *   workspace: (>= that many,) fp32, 16-byte aligned, not kept after the call's
+ *     work; its contents need not be set.
+ */
+int64_t gdn_chunk_prefill_workspace_size(int64_t T, int64_t num_seqs, int64_t num_k_heads, int64_t num_v_heads,
+                                         int64_t k_head_dim, int64_t v_head_dim);
+int gdn_chunk_prefill_split(const gdn_tensor* q, const gdn_tensor* k, const gdn_tensor* v,
+                            const gdn_tensor* g, const gdn_tensor* beta, gdn_tensor* state,
+                            const gdn_tensor* state_indices, const gdn_tensor* cu_seqlens,
+                            gdn_tensor* out, const gdn_tensor* workspace, float scale, int32_t chunk_size,
+                            void* stream);
+
+/*
  * gdn_chunk_prefill with options (no counterpart in the reference).  With
  * flags = 0, items_per_wg = -1 and spin_limit = -1 it is gdn_chunk_prefill.
  *   flags: GDN_PREFILL_ZERO_INIT    every sequence starts from a zero state

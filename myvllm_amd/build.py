@@ -23,6 +23,7 @@ SOURCES = [
     "gdn_decode.hip",
     "gdn_decode_fused.hip",
     "gdn_prefill.hip",
+    "gdn_prefill_split.hip",
     "causal_conv1d.hip",
     "gdn_norm.hip",
     "attention.hip",

@@ -56,15 +56,38 @@ def chunk_gated_delta_rule(
     o = torch.empty(v.shape, dtype=v.dtype, device=dev) if out is None or not _lib.vec16_ok(out) else out
     lib = _lib.load()
     D = _lib.describe
-    rc = lib.gdn_chunk_prefill(
-        D(q), D(k), D(v), D(g), D(beta), D(recurrent_state), D(recurrent_state_indices), D(cu_seqlens), D(o),
-        float(scale), CHUNK_SIZE, _lib.stream_handle(dev),
-    )
-    _lib.check("gdn_chunk_prefill", rc)
+    ws = _prefill_workspace(lib, q, k, v, cu_seqlens)
+    if ws is not None:
+        rc = lib.gdn_chunk_prefill_split(
+            D(q), D(k), D(v), D(g), D(beta), D(recurrent_state), D(recurrent_state_indices), D(cu_seqlens), D(o), D(ws),
+            float(scale), CHUNK_SIZE, _lib.stream_handle(dev),
+        )
+        _lib.check("gdn_chunk_prefill_split", rc)
+    else:
+        rc = lib.gdn_chunk_prefill(
+            D(q), D(k), D(v), D(g), D(beta), D(recurrent_state), D(recurrent_state_indices), D(cu_seqlens), D(o),
+            float(scale), CHUNK_SIZE, _lib.stream_handle(dev),
+        )
+        _lib.check("gdn_chunk_prefill", rc)
     if out is not None and o is not out:
         out.copy_(o)
         return out
     return o
+
+
+def _prefill_workspace(lib, q, k, v, cu_seqlens):
+    """Workspace of the split prefill when these sizes run split (few sequences),
+    else None: the fused kernel, also where the memory is not to be had."""
+    if q.dim() != 3 or v.dim() != 3 or cu_seqlens.dim() != 1:
+        return None  # (the entry refuses the call)
+    n = lib.gdn_chunk_prefill_workspace_size(q.shape[0], cu_seqlens.shape[0] - 1, q.shape[1], v.shape[1], q.shape[2],
+                                             v.shape[2])
+    if n <= 0:
+        return None
+    try:
+        return torch.empty(n, dtype=torch.float32, device=q.device)
+    except torch.OutOfMemoryError:
+        return None
 
 
 def chunk_prefill_ex(q, k, v, g, beta, state, idx, cu_seqlens, out, scale, flags=0, items_per_wg=-1,
