@@ -9,6 +9,8 @@ fallback: if the library is missing every op raises.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 
@@ -16,6 +18,7 @@ import torch
 
 LIB_PATH = os.environ.get("MYVLLM_AMD_LIB") or os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib",
                                                             "libgdn_hip.so")
+BINDING_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "_gdn_binding.so")
 ABI_VERSION = 1
 MAX_NDIM = 4
 
@@ -79,13 +82,24 @@ class GdnError(RuntimeError):
 
 
 _lib = None
+_fast = None  # the native call path (csrc/binding.cpp), bound to the loaded library
 _lock = threading.Lock()
 _PT = ctypes.POINTER(GdnTensor)
 
 
+def _load_binding(lib: ctypes.CDLL):
+    if not os.path.exists(BINDING_PATH):
+        raise RuntimeError(f"{BINDING_PATH} is missing: build the library first (see load())")
+    loader = importlib.machinery.ExtensionFileLoader("_gdn_binding", BINDING_PATH)
+    mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_gdn_binding", loader))
+    loader.exec_module(mod)
+    mod.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in EXPORTED_SYMBOLS})
+    return mod
+
+
 def load() -> ctypes.CDLL:
     """Load (once) and type the shared library; raises if it has not been built."""
-    global _lib
+    global _lib, _fast
     if _lib is not None:
         return _lib
     with _lock:
@@ -146,8 +160,19 @@ def load() -> ctypes.CDLL:
         lib.paged_attention_decode_noalloc.argtypes = [_PT] * 6 + [ctypes.c_int32, ctypes.c_float, ctypes.c_void_p]
         if lib.gdn_abi_version() != ABI_VERSION:
             raise RuntimeError(f"{LIB_PATH} has ABI {lib.gdn_abi_version()}, expected {ABI_VERSION}; rebuild it")
+        _fast = _load_binding(lib)
         _lib = lib
         return lib
+
+
+def _load_fast():
+    load()
+    return _fast
+
+
+def workspace_size(fn: str, *sizes: int) -> int:
+    """One of the library's ``*_workspace_size`` functions."""
+    return getattr(_fast or _load_fast(), fn)(*sizes)
 
 
 def strerror(code: int) -> str:
@@ -170,6 +195,19 @@ def describe(t: torch.Tensor | None) -> GdnTensor:
     return d
 
 
+def call(fn: str, *args) -> None:
+    """Entry point `fn` on tensors (None: a null descriptor) and scalars, on the
+    current stream of the first tensor's device; raises on a non-zero code.
+    Plain tensors go through the native call path, others through ctypes."""
+    lib = _lib or load()
+    code = getattr(_fast, fn)(*args)
+    if code is None:
+        code = getattr(lib, fn)(*(describe(a) if isinstance(a, torch.Tensor) else a for a in args),
+                                stream_handle(args[0].device))
+    if code:
+        raise GdnError(fn, code, strerror(code))
+
+
 def check(fn: str, code: int) -> None:
     if code != 0:
         raise GdnError(fn, code, strerror(code))
@@ -180,6 +218,9 @@ def vec16(t: torch.Tensor) -> torch.Tensor:
     inner stride, 16-byte aligned data and outer strides), else a contiguous
     copy: the reference passes every stride to its kernels, so any strided
     input is accepted, at the cost of a copy when it is misaligned."""
+    ok = (_fast or _load_fast()).vec16_ok(t)
+    if ok is not None:
+        return t if ok else t.contiguous()
     es = t.element_size()
     if t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all((t.stride(i) * es) % 16 == 0 for i in range(t.dim() - 1)):
         return t
@@ -192,6 +233,8 @@ def vec16_ok(t: torch.Tensor) -> bool:
 
 def require_device(*tensors: torch.Tensor) -> torch.device:
     """All tensors must live on one HIP device (the kernels dereference the pointers)."""
+    if (_fast or _load_fast()).same_device(*tensors) >= 0:
+        return next(t for t in tensors if t is not None).device
     dev = None
     for t in tensors:
         if t is None:

@@ -70,6 +70,33 @@ def _run(cmd: list[str], verbose: bool) -> None:
         print(out, flush=True)
 
 
+BINDING = "_gdn_binding.so"
+
+
+def build_binding(verbose: bool = False) -> str:
+    """Compile the Python call path (csrc/binding.cpp, host code against
+    PyTorch's headers and libraries); returns its path."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    os.makedirs(LIBDIR, exist_ok=True)
+    out = os.path.join(LIBDIR, BINDING)
+    tmp = out + f".tmp{os.getpid()}"
+    tlib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = [_hipcc(), "--offload-host-only", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", INCLUDE,
+           "-I", sysconfig.get_paths()["include"]]
+    for p in include_paths():
+        cmd += ["-isystem", p]
+    cmd += [os.path.join(CSRC, "binding.cpp"), "-o", tmp, "-L", tlib, f"-Wl,-rpath,{tlib}", "-ltorch_python", "-ltorch",
+            "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    _run(cmd, verbose)
+    os.replace(tmp, out)
+    return out
+
+
 def library_path() -> str:
     return os.path.join(LIBDIR, LIBNAME)
 
@@ -87,7 +114,7 @@ def build(verbose: bool = False, jobs: int | None = None) -> str:
         cmds.append([hipcc, *COMMON_FLAGS, *SOURCE_FLAGS.get(src, []), "-c", os.path.join(CSRC, src), "-o", obj])
     jobs = jobs or min(len(cmds), max(1, (os.cpu_count() or 2)))
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as ex:
-        for f in [ex.submit(_run, c, verbose) for c in cmds]:
+        for f in [ex.submit(build_binding, verbose)] + [ex.submit(_run, c, verbose) for c in cmds]:
             f.result()
     out = library_path()
     tmp = out + f".tmp{os.getpid()}"

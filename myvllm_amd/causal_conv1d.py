@@ -35,19 +35,11 @@ def causal_conv1d_fn(
     dev = _lib.require_device(x, weight, conv_state, conv_state_indices, cu_seqlens)
     x = _lib.vec16(x)
     o = torch.empty(x.shape, dtype=x.dtype, device=dev)
-    D = _lib.describe
-    lib = _lib.load()
     if l2norm_channels:
-        rc = lib.causal_conv1d_varlen_qknorm(
-            D(x), D(weight), D(conv_state), D(conv_state_indices), D(cu_seqlens), D(o), int(l2norm_channels),
-            _lib.stream_handle(dev),
-        )
-        _lib.check("causal_conv1d_varlen_qknorm", rc)
+        _lib.call("causal_conv1d_varlen_qknorm", x, weight, conv_state, conv_state_indices, cu_seqlens, o,
+                  int(l2norm_channels))
     else:
-        rc = lib.causal_conv1d_varlen(
-            D(x), D(weight), D(conv_state), D(conv_state_indices), D(cu_seqlens), D(o), _lib.stream_handle(dev)
-        )
-        _lib.check("causal_conv1d_varlen", rc)
+        _lib.call("causal_conv1d_varlen", x, weight, conv_state, conv_state_indices, cu_seqlens, o)
     return o
 
 
@@ -62,9 +54,5 @@ def causal_conv1d_update(
     if x.stride(-1) != 1:
         x = x.contiguous()
     o = torch.empty(x.shape, dtype=x.dtype, device=dev)
-    D = _lib.describe
-    rc = _lib.load().causal_conv1d_step(
-        D(x), D(weight), D(conv_state), D(conv_state_indices), D(o), _lib.stream_handle(dev)
-    )
-    _lib.check("causal_conv1d_step", rc)
+    _lib.call("causal_conv1d_step", x, weight, conv_state, conv_state_indices, o)
     return o

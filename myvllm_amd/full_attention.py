@@ -76,13 +76,8 @@ def flash_attention_prefill(
         return _padded_prefill(q, k, v, cu_seqlens, scale, head_dim, head_v_dim, is_causal, max_seqlen, out)
     q, k, v = _lib.vec16(q), _lib.vec16(k), _lib.vec16(v)
     o = _out_for(out, (q.shape[0], q.shape[1], head_v_dim), q.dtype, dev)
-    D = _lib.describe
-    name = "flash_attention_varlen" if own else "flash_attention_varlen_any_dim"
-    rc = getattr(_lib.load(), name)(
-        D(q), D(k), D(v), D(cu_seqlens), D(o), int(max_seqlen), float(scale), int(bool(is_causal)),
-        _lib.stream_handle(dev),
-    )
-    _lib.check(name, rc)
+    _lib.call("flash_attention_varlen" if own else "flash_attention_varlen_any_dim", q, k, v, cu_seqlens, o,
+              int(max_seqlen), float(scale), int(bool(is_causal)))
     return _finish(out, o)
 
 
@@ -158,19 +153,14 @@ def paged_flash_attention_decode(
     B, Hq, Dh = q.shape
     if num_splits is None:
         num_splits = decode_num_splits(B, Hq, k_cache.shape[2], block_tables.shape[1] * block_size)
-    lib = _lib.load()
     ws = None
-    n_ws = lib.paged_attention_decode_workspace_size(B, Hq, Dh, int(num_splits))
+    n_ws = _lib.workspace_size("paged_attention_decode_workspace_size", B, Hq, Dh, int(num_splits))
     if n_ws > 0:
         ws = torch.empty(n_ws, dtype=torch.float32, device=dev)
     q, k_cache, v_cache = _lib.vec16(q), _lib.vec16(k_cache), _lib.vec16(v_cache)
     o = _out_for(out, (B, Hq, v_cache.shape[-1]), q.dtype, dev)
-    D = _lib.describe
-    rc = lib.paged_attention_decode(
-        D(q), D(k_cache), D(v_cache), D(block_tables), D(context_lens), D(o),
-        D(ws) if ws is not None else None, int(num_splits), float(scale), _lib.stream_handle(dev),
-    )
-    _lib.check("paged_attention_decode", rc)
+    _lib.call("paged_attention_decode", q, k_cache, v_cache, block_tables, context_lens, o, ws, int(num_splits),
+              float(scale))
     return _finish(out, o)
 
 
@@ -193,13 +183,9 @@ def paged_flash_attention_decode_noalloc(
     share that array and race; order them on one stream."""
     if k_cache.shape[1] != block_size:
         raise ValueError(f"block_size {block_size} != k_cache.shape[1] {k_cache.shape[1]}")
-    dev = _lib.require_device(q, k_cache, v_cache, block_tables, context_lens, out)
-    D = _lib.describe
-    rc = _lib.load().paged_attention_decode_noalloc(
-        D(q), D(k_cache), D(v_cache), D(block_tables), D(context_lens), D(out), int(num_splits), float(scale),
-        _lib.stream_handle(dev),
-    )
-    _lib.check("paged_attention_decode_noalloc", rc)
+    _lib.require_device(q, k_cache, v_cache, block_tables, context_lens, out)
+    _lib.call("paged_attention_decode_noalloc", q, k_cache, v_cache, block_tables, context_lens, out, int(num_splits),
+              float(scale))
     return out
 
 
@@ -230,21 +216,13 @@ def paged_flash_attention_prefill(
         max_seqlen = _max_seqlen(cu_seqlens)
     q, k_cache, v_cache = _lib.vec16(q), _lib.vec16(k_cache), _lib.vec16(v_cache)
     o = _out_for(out, (q.shape[0], q.shape[1], v_cache.shape[-1]), q.dtype, dev)
-    D = _lib.describe
-    lib = _lib.load()
-    n_ws = lib.paged_attention_prefill_workspace_size(q.shape[0], cu_seqlens.numel() - 1, q.shape[1],
-                                                      k_cache.shape[2], q.shape[2],
-                                                      page_block_tables.shape[1] * page_block_size)
+    n_ws = _lib.workspace_size("paged_attention_prefill_workspace_size", q.shape[0], cu_seqlens.numel() - 1, q.shape[1],
+                               k_cache.shape[2], q.shape[2], page_block_tables.shape[1] * page_block_size)
     if n_ws > 0:
         ws = torch.empty(n_ws, dtype=torch.float32, device=dev)
-        rc = lib.paged_attention_prefill_split(
-            D(q), D(k_cache), D(v_cache), D(page_block_tables), D(context_lens), D(cu_seqlens), D(o), D(ws),
-            int(max_seqlen), float(scale), _lib.stream_handle(dev),
-        )
+        _lib.call("paged_attention_prefill_split", q, k_cache, v_cache, page_block_tables, context_lens, cu_seqlens, o,
+                  ws, int(max_seqlen), float(scale))
     else:
-        rc = lib.paged_attention_prefill(
-            D(q), D(k_cache), D(v_cache), D(page_block_tables), D(context_lens), D(cu_seqlens), D(o),
-            int(max_seqlen), float(scale), _lib.stream_handle(dev),
-        )
-    _lib.check("paged_attention_prefill", rc)
+        _lib.call("paged_attention_prefill", q, k_cache, v_cache, page_block_tables, context_lens, cu_seqlens, o,
+                  int(max_seqlen), float(scale))
     return _finish(out, o)

@@ -54,34 +54,26 @@ def chunk_gated_delta_rule(
                                             scale, out)
     # (an out the kernel cannot write with 16-byte stores is filled through a temporary)
     o = torch.empty(v.shape, dtype=v.dtype, device=dev) if out is None or not _lib.vec16_ok(out) else out
-    lib = _lib.load()
-    D = _lib.describe
-    ws = _prefill_workspace(lib, q, k, v, cu_seqlens)
+    ws = _prefill_workspace(q, v, cu_seqlens)
     if ws is not None:
-        rc = lib.gdn_chunk_prefill_split(
-            D(q), D(k), D(v), D(g), D(beta), D(recurrent_state), D(recurrent_state_indices), D(cu_seqlens), D(o), D(ws),
-            float(scale), CHUNK_SIZE, _lib.stream_handle(dev),
-        )
-        _lib.check("gdn_chunk_prefill_split", rc)
+        _lib.call("gdn_chunk_prefill_split", q, k, v, g, beta, recurrent_state, recurrent_state_indices, cu_seqlens, o,
+                  ws, float(scale), CHUNK_SIZE)
     else:
-        rc = lib.gdn_chunk_prefill(
-            D(q), D(k), D(v), D(g), D(beta), D(recurrent_state), D(recurrent_state_indices), D(cu_seqlens), D(o),
-            float(scale), CHUNK_SIZE, _lib.stream_handle(dev),
-        )
-        _lib.check("gdn_chunk_prefill", rc)
+        _lib.call("gdn_chunk_prefill", q, k, v, g, beta, recurrent_state, recurrent_state_indices, cu_seqlens, o,
+                  float(scale), CHUNK_SIZE)
     if out is not None and o is not out:
         out.copy_(o)
         return out
     return o
 
 
-def _prefill_workspace(lib, q, k, v, cu_seqlens):
+def _prefill_workspace(q, v, cu_seqlens):
     """Workspace of the split prefill when these sizes run split (few sequences),
     else None: the fused kernel, also where the memory is not to be had."""
-    if q.dim() != 3 or v.dim() != 3 or cu_seqlens.dim() != 1:
+    qs, vs, cs = q.shape, v.shape, cu_seqlens.shape
+    if len(qs) != 3 or len(vs) != 3 or len(cs) != 1:
         return None  # (the entry refuses the call)
-    n = lib.gdn_chunk_prefill_workspace_size(q.shape[0], cu_seqlens.shape[0] - 1, q.shape[1], v.shape[1], q.shape[2],
-                                             v.shape[2])
+    n = _lib.workspace_size("gdn_chunk_prefill_workspace_size", qs[0], cs[0] - 1, qs[1], vs[1], qs[2], vs[2])
     if n <= 0:
         return None
     try:
@@ -96,13 +88,9 @@ def chunk_prefill_ex(q, k, v, g, beta, state, idx, cu_seqlens, out, scale, flags
     ``_lib.PREFILL_*``, the schedule and the bound of the kernel's internal
     waits; include/gdn_hip.h).  q, k, v bf16 or fp16, last stride 1; out
     v's dtype, or fp32 for fp16 inputs; nothing is converted or allocated."""
-    dev = _lib.require_device(q, k, v, g, beta, state, idx, cu_seqlens, out)
-    D = _lib.describe
-    rc = _lib.load().gdn_chunk_prefill_ex(
-        D(q), D(k), D(v), D(g), D(beta), D(state), D(idx), D(cu_seqlens), D(out), float(scale), CHUNK_SIZE,
-        int(flags), int(items_per_wg), int(spin_limit), _lib.stream_handle(dev),
-    )
-    _lib.check("gdn_chunk_prefill_ex", rc)
+    _lib.require_device(q, k, v, g, beta, state, idx, cu_seqlens, out)
+    _lib.call("gdn_chunk_prefill_ex", q, k, v, g, beta, state, idx, cu_seqlens, out, float(scale), CHUNK_SIZE,
+              int(flags), int(items_per_wg), int(spin_limit))
     return out
 
 
@@ -148,13 +136,7 @@ def recurrent_gated_delta_rule(
     if scale is None:
         scale = k.shape[-1] ** -0.5
     o = torch.empty(v.shape, dtype=v.dtype, device=dev)
-    lib = _lib.load()
-    D = _lib.describe
-    rc = lib.gdn_recurrent_step(
-        D(q), D(k), D(v), D(g), D(beta), D(recurrent_state), D(recurrent_state_indices), D(o),
-        float(scale), _lib.stream_handle(dev),
-    )
-    _lib.check("gdn_recurrent_step", rc)
+    _lib.call("gdn_recurrent_step", q, k, v, g, beta, recurrent_state, recurrent_state_indices, o, float(scale))
     return o
 
 
@@ -216,12 +198,6 @@ def gated_delta_net_decode_step(
     if scale is None:
         scale = K ** -0.5
     o = torch.empty((mixed_qkv.shape[0], Hv, V), dtype=mixed_qkv.dtype, device=dev) if out is None else out
-    lib = _lib.load()
-    D = _lib.describe
-    rc = lib.gdn_decode_step_fused(
-        D(mixed_qkv), D(conv_weight), D(conv_state), D(conv_state_indices), D(a), D(b), D(A_log), D(dt_bias),
-        D(recurrent_state), D(recurrent_state_indices), D(o), int(num_k_heads), float(scale),
-        _lib.stream_handle(dev),
-    )
-    _lib.check("gdn_decode_step_fused", rc)
+    _lib.call("gdn_decode_step_fused", mixed_qkv, conv_weight, conv_state, conv_state_indices, a, b, A_log, dt_bias,
+              recurrent_state, recurrent_state_indices, o, int(num_k_heads), float(scale))
     return o

@@ -32,9 +32,7 @@ def rms_norm_gated(x: torch.Tensor, gate: torch.Tensor, weight: torch.Tensor, ep
     if g3.stride(-1) != 1:
         g3 = g3.contiguous()
     out = torch.empty(x3.shape, dtype=x.dtype, device=dev)
-    D = _lib.describe
-    rc = _lib.load().gdn_rms_norm_gated(D(x3), D(g3), D(weight), D(out), float(eps), _lib.stream_handle(dev))
-    _lib.check("gdn_rms_norm_gated", rc)
+    _lib.call("gdn_rms_norm_gated", x3, g3, weight, out, float(eps))
     return out.reshape(shape)
 
 
@@ -61,7 +59,5 @@ def gdn_gating(a: torch.Tensor, b: torch.Tensor, A_log: torch.Tensor, dt_bias: t
     dev = _lib.require_device(a, b, A_log, dt_bias)
     g = torch.empty(a.shape, dtype=torch.float32, device=dev)
     beta = torch.empty(a.shape, dtype=torch.float32, device=dev)
-    D = _lib.describe
-    rc = _lib.load().gdn_gating(D(a), D(b), D(A_log), D(dt_bias), D(g), D(beta), _lib.stream_handle(dev))
-    _lib.check("gdn_gating", rc)
+    _lib.call("gdn_gating", a, b, A_log, dt_bias, g, beta)
     return g, beta
