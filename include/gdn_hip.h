@@ -246,6 +246,26 @@ int gdn_decode_step_fused(const gdn_tensor* mixed_qkv, const gdn_tensor* conv_we
                           void* stream);
 
 /*
+ * The same with the layer's gated RMSNorm (layers/linear_attention.py:121) on
+ * the output before it is rounded:
+ *   out = o * rsqrt(mean(o^2) + eps) * norm_weight * silu(gate), per v-head.
+ * gate: out's shape and dtype, unit inner stride; norm_weight: (V,) float.
+ */
+int gdn_decode_step_fused_norm(const gdn_tensor* mixed_qkv, const gdn_tensor* conv_weight, gdn_tensor* conv_state,
+                               const gdn_tensor* conv_state_indices, const gdn_tensor* a, const gdn_tensor* b,
+                               const gdn_tensor* A_log, const gdn_tensor* dt_bias, gdn_tensor* state,
+                               const gdn_tensor* state_indices, const gdn_tensor* gate,
+                               const gdn_tensor* norm_weight, gdn_tensor* out, int32_t num_k_heads, float scale,
+                               float eps, void* stream);
+
+/*
+ * Linear layer of at most 16 tokens: out (M, N) = x (M, K) weight (N, K)^T,
+ * bf16 or fp16 throughout with fp32 sums; K a multiple of 256; unit inner
+ * strides, 16-byte aligned rows of x and weight, 8-byte aligned rows of out.
+ */
+int gdn_linear(const gdn_tensor* x, const gdn_tensor* weight, gdn_tensor* out, void* stream);
+
+/*
  * causal_conv1d_varlen, and the per-head L2 norm of the layer
  * (layers/linear_attention.py:113-114, y * rsqrt(sum y^2 + 1e-6) over each
  * 128-channel head) applied in fp32 to output channels [0, norm_channels)

@@ -44,6 +44,8 @@ EXPORTED_SYMBOLS = (
     "causal_conv1d_varlen",
     "causal_conv1d_step",
     "gdn_decode_step_fused",
+    "gdn_decode_step_fused_norm",
+    "gdn_linear",
     "causal_conv1d_varlen_qknorm",
     "gdn_rms_norm_gated",
     "gdn_gating",
@@ -131,6 +133,11 @@ def load() -> ctypes.CDLL:
         lib.causal_conv1d_step.argtypes = [_PT] * 5 + [ctypes.c_void_p]
         lib.gdn_decode_step_fused.restype = ctypes.c_int
         lib.gdn_decode_step_fused.argtypes = [_PT] * 11 + [ctypes.c_int32, ctypes.c_float, ctypes.c_void_p]
+        lib.gdn_decode_step_fused_norm.restype = ctypes.c_int
+        lib.gdn_decode_step_fused_norm.argtypes = [_PT] * 13 + [ctypes.c_int32, ctypes.c_float, ctypes.c_float,
+                                                                ctypes.c_void_p]
+        lib.gdn_linear.restype = ctypes.c_int
+        lib.gdn_linear.argtypes = [_PT] * 3 + [ctypes.c_void_p]
         lib.causal_conv1d_varlen_qknorm.restype = ctypes.c_int
         lib.causal_conv1d_varlen_qknorm.argtypes = [_PT] * 6 + [ctypes.c_int64, ctypes.c_void_p]
         lib.gdn_rms_norm_gated.restype = ctypes.c_int

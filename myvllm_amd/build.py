@@ -26,6 +26,7 @@ SOURCES = [
     "gdn_prefill_split.hip",
     "causal_conv1d.hip",
     "gdn_norm.hip",
+    "linear.hip",
     "attention.hip",
     "hbm_copy.hip",
     "gdn_capi.cpp",

@@ -177,6 +177,8 @@ typedef Entry<12, 7, int64_t, float> PagedPrefill;
 typedef Entry<13, 8, int64_t, float> PagedPrefillSplit;
 typedef Entry<14, 7, int32_t, float> PagedDecode;
 typedef Entry<15, 6, int32_t, float> PagedDecodeNoalloc;
+typedef Entry<16, 13, int32_t, float, float> DecodeFusedNorm;
+typedef Entry<17, 3> Linear;
 typedef Size<0, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t> ChunkPrefillSize;
 typedef Size<1, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t> PagedPrefillSize;
 typedef Size<2, int64_t, int64_t, int64_t, int32_t> PagedDecodeSize;
@@ -196,6 +198,8 @@ const Bound kBound[] = {
     GDN_BOUND("causal_conv1d_varlen_qknorm", ConvVarlenNorm),
     GDN_BOUND("causal_conv1d_step", ConvStep),
     GDN_BOUND("gdn_decode_step_fused", DecodeFused),
+    GDN_BOUND("gdn_decode_step_fused_norm", DecodeFusedNorm),
+    GDN_BOUND("gdn_linear", Linear),
     GDN_BOUND("gdn_rms_norm_gated", RmsNorm),
     GDN_BOUND("gdn_gating", Gating),
     GDN_BOUND("flash_attention_varlen", AttnVarlen),

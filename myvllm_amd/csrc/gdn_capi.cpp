@@ -35,7 +35,9 @@ hipError_t causal_conv1d_step_launch(const gdn_tensor* x, const gdn_tensor* w, g
 hipError_t gdn_decode_fused_launch(const gdn_tensor* x, const gdn_tensor* w, gdn_tensor* cs, const gdn_tensor* cidx,
                                    const gdn_tensor* ga, const gdn_tensor* gb, const gdn_tensor* A_log,
                                    const gdn_tensor* dt_bias, gdn_tensor* state, const gdn_tensor* sidx,
-                                   gdn_tensor* out, int32_t Hk, float scale, hipStream_t st);
+                                   const gdn_tensor* gate, const gdn_tensor* nw, gdn_tensor* out, int32_t Hk,
+                                   float scale, float eps, hipStream_t st);
+hipError_t linear_launch(const gdn_tensor* x, const gdn_tensor* w, gdn_tensor* out, hipStream_t st);
 
 hipError_t attn_varlen_prefill_launch(const gdn_tensor* q, const gdn_tensor* k, const gdn_tensor* v,
                                       const gdn_tensor* cu, gdn_tensor* out, int64_t max_seqlen, float scale,
@@ -421,8 +423,44 @@ GDN_EXPORT int gdn_decode_step_fused(const gdn_tensor* mixed_qkv, const gdn_tens
   GDN_TRY(check_fused(mixed_qkv, conv_weight, conv_state, conv_state_indices, a, b, A_log, dt_bias, state,
                       state_indices, out, num_k_heads));
   return launch_rc(gdn_decode_fused_launch(mixed_qkv, conv_weight, conv_state, conv_state_indices, a, b, A_log,
-                                           dt_bias, state, state_indices, out, num_k_heads, scale,
-                                           reinterpret_cast<hipStream_t>(stream)));
+                                           dt_bias, state, state_indices, nullptr, nullptr, out, num_k_heads, scale,
+                                           0.f, reinterpret_cast<hipStream_t>(stream)));
+}
+
+GDN_EXPORT int gdn_decode_step_fused_norm(const gdn_tensor* mixed_qkv, const gdn_tensor* conv_weight,
+                                          gdn_tensor* conv_state, const gdn_tensor* conv_state_indices,
+                                          const gdn_tensor* a, const gdn_tensor* b, const gdn_tensor* A_log,
+                                          const gdn_tensor* dt_bias, gdn_tensor* state,
+                                          const gdn_tensor* state_indices, const gdn_tensor* gate,
+                                          const gdn_tensor* norm_weight, gdn_tensor* out, int32_t num_k_heads,
+                                          float scale, float eps, void* stream) {
+  GDN_TRY(check_fused(mixed_qkv, conv_weight, conv_state, conv_state_indices, a, b, A_log, dt_bias, state,
+                      state_indices, out, num_k_heads));
+  GDN_TRY(check_desc(gate, 3));
+  GDN_TRY(check_desc(norm_weight, 1));
+  for (int i = 0; i < 3; ++i)
+    if (gate->shape[i] != out->shape[i]) return GDN_ERR_SHAPE;
+  if (norm_weight->shape[0] != out->shape[2]) return GDN_ERR_SHAPE;
+  if (gate->dtype != out->dtype || !is_float(norm_weight->dtype)) return GDN_ERR_DTYPE;
+  if (gate->stride[2] != 1 || norm_weight->stride[0] != 1) return GDN_ERR_STRIDE;
+  return launch_rc(gdn_decode_fused_launch(mixed_qkv, conv_weight, conv_state, conv_state_indices, a, b, A_log,
+                                           dt_bias, state, state_indices, gate, norm_weight, out, num_k_heads, scale,
+                                           eps, reinterpret_cast<hipStream_t>(stream)));
+}
+
+GDN_EXPORT int gdn_linear(const gdn_tensor* x, const gdn_tensor* weight, gdn_tensor* out, void* stream) {
+  GDN_TRY(check_desc(x, 2));
+  GDN_TRY(check_desc(weight, 2));
+  GDN_TRY(check_desc(out, 2));
+  const int64_t M = x->shape[0], K = x->shape[1], N = weight->shape[0];
+  if (weight->shape[1] != K || out->shape[0] != M || out->shape[1] != N) return GDN_ERR_SHAPE;
+  if (K <= 0 || K % 256 != 0) return GDN_ERR_SHAPE;
+  if (M > 16 || N > kMaxGrid / 2 || K > kMaxGrid) return GDN_ERR_RANGE;
+  if ((x->dtype != GDN_DTYPE_BF16 && x->dtype != GDN_DTYPE_F16) || weight->dtype != x->dtype || out->dtype != x->dtype)
+    return GDN_ERR_DTYPE;
+  if (x->stride[1] != 1 || weight->stride[1] != 1 || out->stride[1] != 1) return GDN_ERR_STRIDE;
+  if (M > 0 && N > 0 && (!vec_ok(x, 16) || !vec_ok(weight, 16) || !vec_ok(out, 8))) return GDN_ERR_ALIGN;
+  return launch_rc(linear_launch(x, weight, out, reinterpret_cast<hipStream_t>(stream)));
 }
 
 GDN_EXPORT int causal_conv1d_varlen_qknorm(const gdn_tensor* x, const gdn_tensor* weight, gdn_tensor* conv_state,

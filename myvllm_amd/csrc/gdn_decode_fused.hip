@@ -30,6 +30,11 @@ struct FusedArgs {
   int32_t w_dtype, cs_dtype, a_dtype, b_dtype, al_dtype, dt_dtype;
   float scale;
   bool cidx64, sidx64;
+  // gated norm of the output (gate null: none)
+  const void* gate; const void* nw;
+  int64_t g_s0, g_s1;
+  int32_t nw_dtype;
+  float eps;
 };
 
 constexpr int kThreads = 1024;
@@ -214,8 +219,29 @@ void gdn_decode_fused_kernel(FusedArgs a) {
     for (int j = 0; j < 4; ++j) d[j] = bn * (sv[n][4 * cc + j] - eg * kS[j]);
     sd[n][cc] = d;
     TX* o = reinterpret_cast<TX*>(a.out) + b * a.o_s0 + (h0 + n) * a.o_s1;
+    float y[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) o[4 * cc + j] = from_f32<TX>(fmaf(eg, qS[j], qkn * d[j]));
+    for (int j = 0; j < 4; ++j) y[j] = fmaf(eg, qS[j], qkn * d[j]);
+    if (a.gate) {
+      // the head's gated RMSNorm (rms_norm_gated_kernel's), before o is
+      // rounded: its CG = 32 threads are one half of a wave
+      static_assert(CG == 32, "a head's finishers are half a wave");
+      const TX* z = reinterpret_cast<const TX*>(a.gate) + b * a.g_s0 + (h0 + n) * a.g_s1;
+      float ss = 0.f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) ss = fmaf(y[j], y[j], ss);
+#pragma unroll
+      for (int off = 1; off < CG; off <<= 1) ss += __shfl_xor(ss, off, 64);
+      const float rn = rsqrtf(ss * (1.f / V) + a.eps);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float g = to_f32(z[4 * cc + j]);
+        y[j] = y[j] * rn * scalar_raw_f32(load_scalar_raw(a.nw, 4 * cc + j, a.nw_dtype), a.nw_dtype) *
+               (g / (1.f + __expf(-g)));
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[4 * cc + j] = from_f32<TX>(y[j]);
   }
   __syncthreads();
 #pragma unroll
@@ -250,8 +276,14 @@ hipError_t launch_heads(const FusedArgs& a, int nh, int64_t nblocks, hipStream_t
 hipError_t gdn_decode_fused_launch(const gdn_tensor* x, const gdn_tensor* w, gdn_tensor* cs, const gdn_tensor* cidx,
                                    const gdn_tensor* ga, const gdn_tensor* gb, const gdn_tensor* A_log,
                                    const gdn_tensor* dt_bias, gdn_tensor* state, const gdn_tensor* sidx,
-                                   gdn_tensor* out, int32_t Hk, float scale, hipStream_t st) {
-  FusedArgs a;
+                                   const gdn_tensor* gate, const gdn_tensor* nw, gdn_tensor* out, int32_t Hk,
+                                   float scale, float eps, hipStream_t st) {
+  FusedArgs a{};
+  if (gate) {
+    a.gate = gate->data; a.g_s0 = gate->stride[0]; a.g_s1 = gate->stride[1];
+    a.nw = nw->data; a.nw_dtype = nw->dtype;
+    a.eps = eps;
+  }
   a.x = x->data; a.w = w->data; a.cs = cs->data; a.cidx = cidx->data;
   a.ga = ga->data; a.gb = gb->data; a.A_log = A_log->data; a.dt_bias = dt_bias->data;
   a.state = reinterpret_cast<float*>(state->data); a.sidx = sidx->data; a.out = out->data;

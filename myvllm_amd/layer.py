@@ -15,8 +15,11 @@ wrong shapes and projects ``z``, ``:93``, ``:95``, ``:121-122``):
   out = o W_out^T                                                (:122)
 
 The four input projections are one GEMM (rows q|k|v|z|b|a; measured faster
-than separate q|k|v|z and b|a GEMMs on this device) and every GEMM is
-torch's (hipBLASLt); the gates are one small kernel.  One call takes a mixed batch: the prefill
+than separate q|k|v|z and b|a GEMMs on this device) and a GEMM is
+torch's (hipBLASLt), or for the few tokens of a small decode step the linear
+kernel's; the gates are one small kernel.  A step of decode tokens only is
+three launches: in_proj, the fused decode step with the gated norm, out_proj
+(one sequence 78 -> 33 us).  One call takes a mixed batch: the prefill
 sequences' tokens first (``cu_seqlens`` covers them), then
 ``num_decode_tokens`` decode tokens, one per sequence, whose slot ids follow
 the prefill ones in the index tensors (the reference takes one
@@ -37,6 +40,7 @@ import math
 import torch
 from torch import nn
 
+from . import _lib
 from .causal_conv1d import causal_conv1d_fn
 from .gated_delta_rule import chunk_gated_delta_rule, gated_delta_net_decode_step
 from .norm import gdn_gating, rms_norm_gated
@@ -51,6 +55,26 @@ def _side_stream(dev: torch.device) -> torch.cuda.Stream:
     if st is None:
         st = _side_streams[idx] = torch.cuda.Stream(device=idx)
     return st
+
+
+def _linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """x w^T of a decode step's few tokens."""
+    M, K = x.shape
+    N = w.shape[0]
+    if not _own_linear(M, N, K) or _lib.vec16(x) is not x or _lib.vec16(w) is not w:
+        return x @ w.t()
+    out = torch.empty(M, N, dtype=x.dtype, device=x.device)
+    _lib.call("gdn_linear", x, w, out)
+    return out
+
+
+def _own_linear(M: int, N: int, K: int) -> bool:
+    """Where ``gdn_linear`` beats the library's product: up to 16 tokens, while
+    the tokens that each tile of 16 weight rows reads stay few beside the
+    weights (12,352 rows of 2,048: 13.7 against 16.6 us at 4 tokens, 17.7 against
+    16.5 at 16; 6,176 rows 9.9 against 9.6 at 16; 2,048 rows of 4,096 9.4 against
+    11.5).  K in whole k-steps of the kernel's eight waves, 8-byte rows of out."""
+    return 0 < M <= 16 and M * N <= 98304 and K > 0 and K % 256 == 0 and N % 4 == 0
 
 
 class GatedDeltaNet(nn.Module):
@@ -151,6 +175,38 @@ class GatedDeltaNet(nn.Module):
                              "(the fused decode step)")
         return Np
 
+    def _native_decode(self, x: torch.Tensor) -> bool:
+        """Whether a decode step runs as three launches (:meth:`_forward_decode`):
+        plain 16-bit tensors in one dtype with nothing recording the torch
+        products that the general path makes (autograd, autocast, a dispatch
+        or function mode, a compiler)."""
+        if not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16) or x.shape[0] == 0:
+            return False
+        if torch.is_grad_enabled() and (x.requires_grad or self.in_proj.requires_grad or self.out_proj.requires_grad):
+            return False
+        if torch.is_autocast_enabled() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0 or \
+                torch._C._len_torch_function_stack() > 0:
+            return False
+        if torch.autograd.forward_ad._current_level >= 0:
+            return False
+        return (type(x) is torch.Tensor and type(self.in_proj) is nn.Parameter and type(self.out_proj) is nn.Parameter
+                and self.in_proj.dtype == x.dtype and self.out_proj.dtype == x.dtype
+                and self.norm_weight.dim() == 1)
+
+    def _forward_decode(self, x, conv_state_indices, recurrent_state_indices) -> torch.Tensor:
+        """A decode step: in_proj, the fused step with the gated norm, out_proj."""
+        T, Hv, V = x.shape[0], self.num_v_heads, self.v_head_dim
+        proj = _linear(x, self.in_proj)
+        cz = self.conv_dim + self.v_size
+        o = torch.empty(T, Hv, V, dtype=x.dtype, device=x.device)
+        _lib.require_device(x, self.in_proj, self.conv1d_weight, self.A_log, self.dt_bias, self.norm_weight,
+                            self.out_proj)
+        _lib.call("gdn_decode_step_fused_norm", proj[:, : self.conv_dim], self.conv1d_weight, self.conv_state,
+                  conv_state_indices, proj[:, cz + Hv:], proj[:, cz: cz + Hv], self.A_log, self.dt_bias,
+                  self.recurrent_state, recurrent_state_indices, proj[:, self.conv_dim: cz].view(T, Hv, V),
+                  self.norm_weight, o, self.num_k_heads, self.k_head_dim ** -0.5, float(self.rms_norm_eps))
+        return _linear(o.view(T, self.v_size), self.out_proj)
+
     def forward(
         self,
         x: torch.Tensor,  # (T, hidden)
@@ -176,6 +232,8 @@ class GatedDeltaNet(nn.Module):
         num_decode_tokens = self._decode_count(T, is_prefill, num_decode_tokens)
         Tp = T - num_decode_tokens
         Np = self._check_inputs(x, cu_seqlens, conv_state_indices, recurrent_state_indices, Tp, num_decode_tokens)
+        if Tp == 0 and self._native_decode(x):
+            return self._forward_decode(x, conv_state_indices, recurrent_state_indices)
         Hk, Hv, K, V = self.num_k_heads, self.num_v_heads, self.k_head_dim, self.v_head_dim
         proj = x @ self.in_proj.t()
         cz = self.conv_dim + self.v_size
