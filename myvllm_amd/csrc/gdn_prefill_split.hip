@@ -798,11 +798,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
 
 // Floats of the workspace with which a prefill of these sizes runs split, 0
 // when the fused kernel serves it.  Split wins where the fused kernel's items
-// leave most CUs idle for many chunks.  Measured, fused -> split, prompts x
-// tokens at 16 / 32 heads: 1 x 256 33 -> 36 us (two launches and the
-// workspace), 1 x 512 51 -> 36, 1 x 1,024 88 -> 45, 1 x 2,943 225 -> 106, 1 x
-// 16,384 1,186 -> 618, 2 x 512 53 -> 44, 2 x 1,500 126 -> 95, 2 x 2,943 226 ->
-// 202, and past 64 items 3 x 1,000 91 -> 104, 4 x 2,048 164 -> 276: the records
+// leave most CUs idle for a few chunks.  Measured, fused -> split, prompts x
+// tokens at 16 / 32 heads: 1 x 128 21 -> 20 us, 1 x 192 27 -> 22, 1 x 384 40 ->
+// 26, 1 x 1,024 88 -> 45, 1 x 2,943 225 -> 106, 1 x 16,384 1,186 -> 618, 2 x
+// 256 32 -> 28, 2 x 512 51 -> 41, 2 x 1,500 126 -> 95, 2 x 2,943 226 -> 202,
+// and past 64 items 3 x 1,000 91 -> 104, 4 x 2,048 164 -> 276: the records
 // (91 KB per chunk and head, written and read once) then cost more than the
 // idle CUs.  Up to 32 items a scan workgroup takes 16 columns (256 workgroups;
 // 32 columns: 2,943 tokens at 16 heads 74 -> 102 us), past that 32 (each record
@@ -811,7 +811,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
 int64_t gdn_chunk_prefill_split_floats(int64_t T, int64_t nseq, int64_t Hk, int64_t Hv, int64_t kd, int64_t vd) {
   if (T <= 0 || nseq <= 0 || nseq > kMaxSplitSeqs || Hk <= 0 || Hv <= 0 || kd != KD || vd != VD) return 0;
   const int64_t items = nseq * Hv;
-  if (items > 2 * kOneGroupItems || T < (items <= kOneGroupItems ? 384 : 512) * nseq) return 0;
+  if (items > 2 * kOneGroupItems || T < (items <= kOneGroupItems ? 192 : 256) * nseq) return 0;
   const int64_t bytes = (T / C + nseq) * (Hv * kRecBytes + Hk * kKRecBytes);
   return bytes <= (int64_t(1) << 30) ? bytes / 4 : 0;
 }

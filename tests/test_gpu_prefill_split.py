@@ -17,8 +17,8 @@ def _floats(T, N, Hk, Hv, K=128, V=128):
 
 def test_split_rule():
     """Few items with many chunks each are split, within 1 GiB of records; the rest is not."""
-    assert _floats(384, 1, 16, 32) > 0 and _floats(383, 1, 16, 32) == 0
-    assert _floats(1024, 2, 16, 32) > 0 and _floats(1023, 2, 16, 32) == 0
+    assert _floats(192, 1, 16, 32) > 0 and _floats(191, 1, 16, 32) == 0
+    assert _floats(512, 2, 16, 32) > 0 and _floats(511, 2, 16, 32) == 0
     assert _floats(30000, 3, 16, 32) == 0 and _floats(40000, 64, 1, 1) > 0 and _floats(40000, 65, 1, 1) == 0
     for args in ((0, 1, 16, 32), (-5, 1, 16, 32), (400, 0, 16, 32), (400, -1, 16, 32), (400, 1, 0, 32), (400, 1, 3, 32),
                  (400, 1, 16, 32, 64, 128), (400, 1, 16, 32, 128, 64), (2**31, 1, 16, 32)):
@@ -48,7 +48,8 @@ def test_split_workspace_checks(bad, code):
 @pytest.mark.parametrize(
     "lengths, Hk, Hv, dtype, g_scale",
     [
-        ([384], 2, 4, torch.bfloat16, 1.0),  # whole chunks, an even number
+        ([192], 2, 4, torch.bfloat16, 1.0),  # whole chunks
+        ([384], 2, 4, torch.float16, 1.0),  # an even number of them
         ([449], 1, 1, torch.bfloat16, 1.0),  # one token past a chunk, an odd number of chunks
         ([1100, 1, 64], 2, 4, torch.float16, 1.0),  # sequences of one chunk beside a long one
         ([600, 0, 900, 63, 1000], 2, 8, torch.bfloat16, 0.05),  # 40 items: two column groups per workgroup; weak decay
