@@ -20,9 +20,15 @@
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kTile = 64;  // tokens per prefill tile (>= W - 1, see the state-ownership note)
+// Tokens per prefill tile (>= W - 1, see the state-ownership note).  A tile is
+// one thread's chain of row batches: short ones fill the chip in small calls
+// and leave a shorter tail in large ones, at W - 1 rows read again per tile.
+// With batches of 4 rows (below), us for 8,192 channels at 64 / 1,000 / 2,500 /
+// 8,000 / 22,700 tokens: tile 24 10 / 11 / 19 / 48 / 146, 16 9 / 10 / 21 / 48 /
+// 147, 32 12 / 13 / 21 / 47 / 150-170, 64 with batches of 8 19 / 20 / 21 / 55 / 159.
+constexpr int kTile = 24;
 constexpr int kCh = 8;     // channels per thread
-constexpr int kBatch = 8;  // token rows loaded together
+constexpr int kBatch = 4;  // token rows loaded together (113 registers at W = 4: four waves per SIMD)
 
 struct ConvArgs {
   const void* x; const void* w; void* state; const void* idx; const void* cu; void* out;
@@ -182,7 +188,8 @@ GDN_DEVICE void conv_tile(const ConvArgs& a, int64_t seq, int64_t tile, int64_t 
 
 // One workgroup per (tile, channel block); blockIdx.x is the linear tile id.
 template <typename TX, typename TW, typename TS, int W>
-__global__ __launch_bounds__(kThreads) void causal_conv1d_varlen_kernel(ConvArgs a) {
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W <= 4 && sizeof(TX) == 2 ? 4 : 1)))
+void causal_conv1d_varlen_kernel(ConvArgs a) {
   __shared__ int32_t lds[8];
   // output rows no sequence covers are zero, as the reference allocates y
   // zero-filled (ops/causal_conv1d.py:241)

@@ -97,3 +97,12 @@ def test_conv_strided_weight(dev):
     y2_ref = causal_conv1d_update_ref(case.x[:2], case.weight, st2_ref, case.idx)
     assert_out_close(y2.cpu(), y2_ref)
     assert torch.equal(st2.cpu(), st2_ref)
+
+
+@pytest.mark.parametrize("W", [2, 4, 6])
+def test_conv_tile_edges(dev, W):
+    """Lengths around the kernel's 24-token tiles and 4-row batches; the states are exact copies."""
+    case = conv_prefill_case([23, 24, 25, 4, 47, 48, 49, 5, 73, 96], seed=10 + W, D=136, W=W, num_slots=12)
+    y, st, y_ref, st_ref = _prefill(case, dev)
+    assert_out_close(y, y_ref)
+    assert torch.equal(st, st_ref)
