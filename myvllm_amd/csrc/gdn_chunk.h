@@ -323,10 +323,14 @@ GDN_DEVICE void invert_diag16(const Scratch& A, int lane) {
 #pragma unroll
   for (int i = 0; i < 16; ++i) y[i] = i == c ? 1.f : 0.f;
 #pragma unroll
-  for (int kk = 0; kk < 15; ++kk) {
-    const float xk = y[kk];
+  for (int kk = 0; kk < 16; kk += 2) {  // two columns of A per read
+    f32x2 ak[16];
 #pragma unroll
-    for (int i = kk + 1; i < 16; ++i) y[i] = fmaf(-A.row(16 * b + i, b)[kk], xk, y[i]);
+    for (int i = kk + 1; i < 16; ++i) ak[i] = *reinterpret_cast<const f32x2*>(A.row(16 * b + i, b) + kk);
+#pragma unroll
+    for (int i = kk + 1; i < 16; ++i) y[i] = fmaf(-ak[i][0], y[kk], y[i]);
+#pragma unroll
+    for (int i = kk + 2; i < 16; ++i) y[i] = fmaf(-ak[i][1], y[kk + 1], y[i]);
   }
   if (lane < 32) {
 #pragma unroll
@@ -534,6 +538,28 @@ GDN_DEVICE f32x16 gram_regs(const bf16x8 (&kf)[8]) {
   return G;
 }
 
+// e^(gamma_i - gamma_j) for token i of the lane and the tokens j = j0 + 8 i4 + 4g + r of its registers
+GDN_DEVICE void row_decays(float (&d)[16], const float* gam, const float* eg, const float* ieg, bool fact, int i, int j0,
+                           int lane) {
+  if (fact) {
+    const float ei = eg[i];
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4) {
+      const f32x4 ej = rows4(ieg, j0, i4, lane);
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) d[4 * i4 + rr] = ei * ej[rr];
+    }
+  } else {
+    const float gi = gam[i];
+#pragma unroll
+    for (int i4 = 0; i4 < 4; ++i4) {
+      const f32x4 gj = rows4(gam, j0, i4, lane);
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) d[4 * i4 + rr] = __expf(gi - gj[rr]);
+    }
+  }
+}
+
 // Diagonal block `blk` of T: A_bb = strict_lower(beta_i k_i.k_j e^(g_i - g_j))
 // from its kk^T tile, solved in fp32 in the off-diagonal block of the same
 // T buffer (16x16 substitution + one MFMA merge), then T_bb written as fp16
@@ -543,30 +569,20 @@ GDN_DEVICE void solve_diag_block(TBuf& tb, const float* gam, const float* beta, 
                                  bool fact, const f32x16& G, int blk, int lane) {
   const int n = lane & 31, gq = lane >> 5, o = 32 * blk;
   const Scratch A = scratch_of(tb, blk);
-  if (fact) {
-    const float ej = ieg[o + n];
+  // (kk^T is symmetric to the bit, so the lane's column is taken as row n and
+  // its registers as four consecutive columns at a time: two 8-byte writes)
+  const float bn = beta[o + n];
+  float d[16];
+  row_decays(d, gam, eg, ieg, fact, o + n, o, lane);
 #pragma unroll
-    for (int i4 = 0; i4 < 4; ++i4) {
-      const f32x4 ei = rows4(eg, o, i4, lane);
-      const f32x4 bi = rows4(beta, o, i4, lane);
+  for (int i4 = 0; i4 < 4; ++i4) {
+    const int j = 8 * i4 + 4 * gq;
+    float x[4];
 #pragma unroll
-      for (int rr = 0; rr < 4; ++rr) {
-        const int i = 8 * i4 + 4 * gq + rr;
-        A.at(i, n) = i > n ? bi[rr] * G[4 * i4 + rr] * (ei[rr] * ej) : 0.f;
-      }
-    }
-  } else {
-    const float gj = gam[o + n];
-#pragma unroll
-    for (int i4 = 0; i4 < 4; ++i4) {
-      const f32x4 gi = rows4(gam, o, i4, lane);
-      const f32x4 bi = rows4(beta, o, i4, lane);
-#pragma unroll
-      for (int rr = 0; rr < 4; ++rr) {
-        const int i = 8 * i4 + 4 * gq + rr;
-        A.at(i, n) = i > n ? bi[rr] * G[4 * i4 + rr] * __expf(gi[rr] - gj) : 0.f;
-      }
-    }
+    for (int rr = 0; rr < 4; ++rr) x[rr] = n > j + rr ? bn * G[4 * i4 + rr] * d[4 * i4 + rr] : 0.f;
+    float* p = &A.at(n, j);
+    *reinterpret_cast<f32x2*>(p) = (f32x2){x[0], x[1]};
+    *reinterpret_cast<f32x2*>(p + 2) = (f32x2){x[2], x[3]};
   }
   invert_diag16(A, lane);
   merge16(A, lane);
@@ -596,39 +612,23 @@ GDN_DEVICE void solve_diag_block(TBuf& tb, const float* gam, const float* beta, 
 template <typename Tiles>
 GDN_DEVICE void b10_block(const Tiles& ct, TBuf& tb, int lane) {
   const int n = lane & 31, gq = lane >> 5;
-  const f32x16 G = gram_tile(ct.k, ct.k, 1, 0, lane);
-  float d[16];  // e^(gamma_i - gamma_j) for this lane's 16 entries
-  if (__builtin_amdgcn_readfirstlane(ct.fact)) {
-    const float ej = ct.ieg[n];
-#pragma unroll
-    for (int i4 = 0; i4 < 4; ++i4) {
-      const f32x4 ei = rows4(ct.eg, 32, i4, lane);
-#pragma unroll
-      for (int rr = 0; rr < 4; ++rr) d[4 * i4 + rr] = ei[rr] * ej;
-    }
-  } else {
-    const float gj = ct.gam[n];
-#pragma unroll
-    for (int i4 = 0; i4 < 4; ++i4) {
-      const f32x4 gi = rows4(ct.gam, 32, i4, lane);
-#pragma unroll
-      for (int rr = 0; rr < 4; ++rr) d[4 * i4 + rr] = __expf(gi[rr] - gj);
-    }
-  }
+  // (the transposed tile: lane column = token 32 + n, registers = four
+  // consecutive tokens j at a time)
+  const f32x16 G = gram_tile(ct.k, ct.k, 0, 1, lane);
+  const bool fact = __builtin_amdgcn_readfirstlane(ct.fact) != 0;
+  const float bn = ct.beta[32 + n];
+  float d[16];
+  row_decays(d, ct.gam, ct.eg, ct.ieg, fact, 32 + n, 0, lane);
 #pragma unroll
   for (int i4 = 0; i4 < 4; ++i4) {
-    const f32x4 bi = rows4(ct.beta, 32, i4, lane);
+    float x[4];
 #pragma unroll
-    for (int rr = 0; rr < 4; rr += 2) {
-      const int i = 8 * i4 + 4 * gq + rr;
-      f16_t h0, h1, l0, l1;
-      split_pair(G[4 * i4 + rr] * (d[4 * i4 + rr] * bi[rr]), G[4 * i4 + rr + 1] * (d[4 * i4 + rr + 1] * bi[rr + 1]),
-                 h0, h1, l0, l1);
-      tb.hi[i * LDH + 32 + n] = h0;
-      tb.hi[(i + 1) * LDH + 32 + n] = h1;
-      tb.lo[i * LDH + 32 + n] = l0;
-      tb.lo[(i + 1) * LDH + 32 + n] = l1;
-    }
+    for (int rr = 0; rr < 4; ++rr) x[rr] = G[4 * i4 + rr] * (d[4 * i4 + rr] * bn);
+    f16_t hi[4], lo[4];
+    split_vec<4>(x, hi, lo);
+    const int off = n * LDH + 32 + 8 * i4 + 4 * gq;
+    *reinterpret_cast<f16x4*>(tb.hi + off) = (f16x4){hi[0], hi[1], hi[2], hi[3]};
+    *reinterpret_cast<f16x4*>(tb.lo + off) = (f16x4){lo[0], lo[1], lo[2], lo[3]};
   }
 }
 
@@ -647,26 +647,29 @@ GDN_DEVICE void merge_offdiag(TBuf& tb, int lane) {
     M = mfma32(bh, cl, M);
     M = mfma32(bl, ch, M);
   }
-  // -T_11 M: A operand = rows of T_11, B operand = M (C layout rows == k)
+  // (T_11 M)^T = M^T T_11^T: A operand = M^T (M's C layout as it lies), B
+  // operand = rows of T_11; lane column = row of T_10, registers = four
+  // consecutive columns at a time
   f32x16 R = zero16();
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks) {
     const f16x8 ah = frag_rows(th, LDH, 32, 32 + 16 * ks, lane), al = frag_rows(tl, LDH, 32, 32 + 16 * ks, lane);
     f16x8 mh, ml;
     split8(M, ks, 1.f, mh, ml);
-    R = mfma32(ah, mh, R);
-    R = mfma32(ah, ml, R);
-    R = mfma32(al, mh, R);
+    R = mfma32(mh, ah, R);
+    R = mfma32(ml, ah, R);
+    R = mfma32(mh, al, R);
   }
 #pragma unroll
-  for (int j = 0; j < 16; j += 2) {
-    const int i = 32 + 8 * (j >> 2) + 4 * gq + (j & 3);
-    f16_t h0, h1, l0, l1;
-    split_pair(-R[j], -R[j + 1], h0, h1, l0, l1);
-    tb.hi[i * LDH + n] = h0;
-    tb.hi[(i + 1) * LDH + n] = h1;
-    tb.lo[i * LDH + n] = l0;
-    tb.lo[(i + 1) * LDH + n] = l1;
+  for (int i4 = 0; i4 < 4; ++i4) {
+    float x[4];
+    f16_t hi[4], lo[4];
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr) x[rr] = -R[4 * i4 + rr];
+    split_vec<4>(x, hi, lo);
+    const int off = (32 + n) * LDH + 8 * i4 + 4 * gq;
+    *reinterpret_cast<f16x4*>(tb.hi + off) = (f16x4){hi[0], hi[1], hi[2], hi[3]};
+    *reinterpret_cast<f16x4*>(tb.lo + off) = (f16x4){lo[0], lo[1], lo[2], lo[3]};
   }
 }
 

@@ -94,13 +94,15 @@ GDN_DEVICE void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+constexpr int kLdt = 72;  // row stride of the terms of T diag(..)
+
 // The tile members of ChunkTiles that the prepare kernel has (its helpers take
 // K and the decay vectors only).
 struct PrepSmem {
   alignas(16) f16_t k[C * LDK];  // K, later V
   union {
     TBuf tb;
-    f16_t terms[3 * C * LDH];  // later the terms of T diag(..)
+    alignas(16) f16_t terms[3 * C * kLdt];  // later the terms of T diag(..), quads swapped like K's
   };
   alignas(16) float gam[C];
   alignas(16) float eg[C];
@@ -135,20 +137,27 @@ GDN_DEVICE void put_split16(f16_t* dst, int i, int j0, const float (&x)[16], flo
   for (int m = 0; m < 16; ++m) y[m] = x[m] * sc;
   split_vec<16>(y, hi, lo);
 #pragma unroll
-  for (int m = 0; m < 16; m += 4) {
-    *reinterpret_cast<f16x4*>(dst + i * LDH + j0 + m) = (f16x4){hi[m], hi[m + 1], hi[m + 2], hi[m + 3]};
-    *reinterpret_cast<f16x4*>(dst + C * LDH + i * LDH + j0 + m) = (f16x4){lo[m], lo[m + 1], lo[m + 2], lo[m + 3]};
+  for (int m = 0; m < 2; ++m) {  // stored quads 0, 2 and 1, 3 of the 16 columns
+    const int a = 4 * m, b = a + 8;
+    f16_t* p = dst + i * kLdt + j0 + 8 * m;
+    *reinterpret_cast<f16x8*>(p) =
+        (f16x8){hi[a], hi[a + 1], hi[a + 2], hi[a + 3], hi[b], hi[b + 1], hi[b + 2], hi[b + 3]};
+    *reinterpret_cast<f16x8*>(p + C * kLdt) =
+        (f16x8){lo[a], lo[a + 1], lo[a + 2], lo[a + 3], lo[b], lo[b + 1], lo[b + 2], lo[b + 3]};
   }
+}
+GDN_DEVICE f16x8 term_rows(const f16_t* M, int r0, int kbase, int lane) {
+  return *reinterpret_cast<const f16x8*>(M + (r0 + (lane & 31)) * kLdt + kbase + 8 * (lane >> 5));
 }
 
 // The same as three bf16 terms (24 bits, fp32's range) in three arrays
 GDN_DEVICE void put_bf16x3(f16_t* dst, int i, int j0, const float (&x)[16]) {
 #pragma unroll
-  for (int m = 0; m < 16; m += 4) {
-    bf16x4 t[3];
+  for (int m = 0; m < 2; ++m) {
+    bf16x8 t[3];
 #pragma unroll
-    for (int z = 0; z < 4; ++z) {
-      float r = x[m + z];
+    for (int z = 0; z < 8; ++z) {
+      float r = x[4 * m + (z & 3) + 8 * (z >> 2)];
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
         t[k][z] = (bf16_t)r;
@@ -156,7 +165,7 @@ GDN_DEVICE void put_bf16x3(f16_t* dst, int i, int j0, const float (&x)[16]) {
       }
     }
 #pragma unroll
-    for (int k = 0; k < 3; ++k) *reinterpret_cast<bf16x4*>(dst + k * C * LDH + i * LDH + j0 + m) = t[k];
+    for (int k = 0; k < 3; ++k) *reinterpret_cast<bf16x8*>(dst + k * C * kLdt + i * kLdt + j0 + 8 * m) = t[k];
   }
 }
 
@@ -208,13 +217,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void g
   PrepSmem& ct = sm;
   const int n = lane & 31, g2 = lane >> 5, l16 = lane & 15, q4 = lane >> 4;
 
-  // V rows 16w + lane / 16 + 4u, held in registers until the K tile is done with
-  bf16x8 vr[4];
-  {
-    const bf16_t* vb = src.vg + c0 * a.v_s0;
-#pragma unroll
-    for (int u = 0; u < 4; ++u) vr[u] = load_row_piece(vb, (uint32_t)a.v_s0, 16 * w + q4 + 4 * u, 8 * l16, L);
-  }
   f16x8 qf[2][8];  // wave 3: Q
   if (w < 2) {
     DiagLoad dl;
@@ -306,6 +308,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void g
     }
   }
   __syncthreads();
+  // V rows 16w + lane / 16 + 4u, in flight until the K tile is done with
+  bf16x8 vr[4];
+  {
+    const bf16_t* vb = src.vg + c0 * a.v_s0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) vr[u] = load_row_piece(vb, (uint32_t)a.v_s0, 16 * w + q4 + 4 * u, 8 * l16, L);
+  }
   // this lane's 16 entries of T (row ti, columns tj..)
   const int ti = 16 * w + (lane >> 2), tj = 16 * (lane & 3);
   float tbeta[16], tw[16];
@@ -347,7 +356,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void g
     for (int t = 0; t < 2; ++t) {
 #pragma unroll
       for (int nt = ks >> 1; nt < 2; ++nt)
-        acc[nt] = mfma32(kf, frag_rows(terms + t * C * LDH, LDH, 32 * nt, 16 * ks, lane), acc[nt]);
+        acc[nt] = mfma32(kf, term_rows(terms + t * C * kLdt, 32 * nt, 16 * ks, lane), acc[nt]);
     }
   }
   float mx = 0.f;
@@ -404,7 +413,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void g
     for (int t = 0; t < (F16 ? 2 : 3); ++t) {
 #pragma unroll
       for (int mt = ks >> 1; mt < 2; ++mt) {
-        const f16x8 tf = frag_rows(terms + t * C * LDH, LDH, 32 * mt, 16 * ks, lane);
+        const f16x8 tf = term_rows(terms + t * C * kLdt, 32 * mt, 16 * ks, lane);
         if constexpr (F16) U[mt] = mfma32(tf, vf, U[mt]);
         else
           U[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, tf), __builtin_bit_cast(bf16x8, vf),
