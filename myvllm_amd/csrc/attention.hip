@@ -157,6 +157,7 @@ GDN_DEVICE const char* kv_row(const KvSource& s, const PagedTable& tb, int64_t n
 // tiles before it, with no barrier.  Six images of 450 to 2,900 patches 143 ->
 // 137 us, eight causal prompts of 512 to 4,096 tokens 171 -> 159 (D = 64) and
 // 259 -> 247 (128), eight chunks over up to 4,096 cached keys 340 -> 331 (128).
+// Past the last tile seq is -1 and tile counts from there.
 // Larger batches, and D = 256 (sixteen prompts: 974 in index order, 985
 // ranked), are taken in index order by a scan over the workgroup.
 struct SeqTile {
@@ -174,19 +175,40 @@ GDN_DEVICE SeqTile attn_tile_lookup(const AttnArgs& a, int tile_len, int64_t tar
       nt = (int)((e - s + tile_len - 1) >> sh);
       key = PAGED ? (int)clamp64(load_index(a.ctx, lane, a.ctx64), 0, 0x7fffffff) : (int)(e - s);
     }
-    int base = 0;
+    int base = 0, total = 0;
     for (int j = 0; j < (int)a.nseq; ++j) {
       const int kj = __builtin_amdgcn_readlane(key, j), tj = __builtin_amdgcn_readlane(nt, j);
       base += kj > key || (kj == key && j < lane) ? tj : 0;
+      total += tj;
     }
     const int t = (int)target - base;
     const uint64_t own = __builtin_amdgcn_ballot_w64(t >= 0 && t < nt);
     r.seq = own ? __builtin_ctzll(own) : -1;
-    r.tile = own ? __builtin_amdgcn_readlane(t, (int)r.seq) : 0;
+    r.tile = own ? __builtin_amdgcn_readlane(t, (int)r.seq) : target - total;
     return r;
   }
   find_seq_tile<256>(a.cu, a.cu64, a.nseq, a.T, tile_len, target, r.seq, r.tile, lds);
   return r;
+}
+
+// Output rows that no sequence covers -- [0, cu[0]) and [cu[N], T), clamped
+// like seq_range -- are zero, as the reference allocates o zero-filled
+// (ops/full_attention.py:467).  The workgroups past the last tile, `wg` of `n`,
+// share them (a kernel of their own, launched first, took 3 to 5 us of every
+// call; the usual batch covers all rows and has nothing to do here).
+template <typename T>
+GDN_DEVICE void zero_rows_tail(const AttnArgs& a, uint32_t wg, uint32_t n) {
+  int64_t first = load_index(a.cu, 0, a.cu64), last = load_index(a.cu, a.nseq, a.cu64);
+  first = clamp64(first, 0, a.T);
+  last = clamp64(last, first, a.T);
+  const int64_t nrows = first + (a.T - last);
+  constexpr int per = 16 / (int)sizeof(T);  // elements of a 16-byte piece
+  const int64_t vph = a.dim / per, vpr = a.Hq * vph;
+  for (int64_t i = (int64_t)wg * 256 + threadIdx.x; i < nrows * vpr; i += (int64_t)n * 256) {
+    const int64_t r = i / vpr, rem = i - r * vpr, h = rem / vph, c = (rem - h * vph) * per;
+    const int64_t t = r < first ? r : last + (r - first);
+    *reinterpret_cast<uint4*>(reinterpret_cast<T*>(a.o) + t * a.o_st + h * a.o_sh + c) = uint4{0, 0, 0, 0};
+  }
 }
 
 // SPLIT: the key range of every (query tile, head group) row is cut into
@@ -258,10 +280,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   // sequence's workgroups run together and share its K/V rows in L2.
   __shared__ int32_t lookup[8];
   const int hg = a.Hq / gh;  // head groups
-  const uint32_t piece = SPLIT ? blockIdx.x / (uint32_t)a.rows : 0u;
-  const uint32_t row_id = SPLIT ? blockIdx.x - piece * (uint32_t)a.rows : blockIdx.x;
+  // (the grid ends with one tile's head groups more than the sequences can
+  // have: a split grid's come after its pieces)
+  const uint32_t srows = SPLIT ? (uint32_t)a.rows : 0u;
+  const bool past = SPLIT && blockIdx.x >= srows * (uint32_t)a.splits;
+  const uint32_t piece = SPLIT && !past ? blockIdx.x / srows : 0u;
+  const uint32_t row_id = past ? srows + (blockIdx.x - srows * (uint32_t)a.splits) : blockIdx.x - piece * srows;
   const SeqTile st = attn_tile_lookup<D, PAGED>(a, 32 * qsubs, row_id / hg, lookup);
-  if (st.seq < 0) return;
+  if (st.seq < 0) {
+    if (piece > 0) return;
+    const uint32_t tiles = (SPLIT ? srows : gridDim.x - hg) / hg + 1;
+    zero_rows_tail<T>(a, (uint32_t)st.tile * hg + row_id % hg, (tiles - (row_id / hg - (uint32_t)st.tile)) * hg);
+    return;
+  }
   const int64_t n = st.seq;
   const int y = (int)(row_id % hg);
   const int kvh = y / groups;
@@ -1262,15 +1293,14 @@ PagedTable paged_table(const gdn_tensor* tab, const gdn_tensor* kc) {
 template <typename T, int D, int BN, bool PAGED, int DQ = 0>
 hipError_t launch_prefill_t(const AttnArgs& a, int64_t nseq, int64_t max_len, hipStream_t st) {
   const int qsubs = 4 / a.gh;
-  // output rows no sequence covers are zero, as the reference allocates o
-  // zero-filled (ops/full_attention.py:467); a kernel of its own, launched
-  // first (a call inside the attention kernel changed its register allocation
-  // and cost it about a fifth of its speed)
-  zero_uncovered_rows_kernel<(int)sizeof(T)><<<dim3(64), dim3(256), 0, st>>>(a.o, a.o_st, a.o_sh, a.Hq, a.dim, a.cu,
+  // without sequences there are only rows to zero
+  if (nseq <= 0 || max_len <= 0)
+    zero_uncovered_rows_kernel<(int)sizeof(T)><<<dim3(64), dim3(256), 0, st>>>(a.o, a.o_st, a.o_sh, a.Hq, a.dim, a.cu,
                                                                              a.cu64, a.nseq, a.T);
   if (nseq <= 0 || max_len <= 0) return hipGetLastError();
-  // query tiles: at most T / tile_len + one partial tile per sequence
-  const int64_t tiles = a.T / (32 * qsubs) + nseq;
+  // query tiles: at most T / tile_len + one partial tile per sequence, and one
+  // that no sequence can have
+  const int64_t tiles = a.T / (32 * qsubs) + nseq + 1;
   const dim3 grid((unsigned)(tiles * (a.Hq / a.gh)));
   if constexpr (!PAGED) {
     hipLaunchKernelGGL((attn_prefill_kernel<T, D, BN, 0, false, DQ>), grid, dim3(256), 0, st, a);
@@ -1278,7 +1308,7 @@ hipError_t launch_prefill_t(const AttnArgs& a, int64_t nseq, int64_t max_len, hi
              a.tab.cols * a.tab.page < (int64_t(1) << 31) && a.tab.num_blocks < (int64_t(1) << 31)) {
     // whole 16-row groups per page, 32-bit table arithmetic
     if (a.splits > 1) {
-      const dim3 sgrid((unsigned)(a.rows * a.splits));
+      const dim3 sgrid((unsigned)(a.rows * a.splits + a.Hq / a.gh));
       constexpr int DG = D == 256 ? 2 : 1;  // 32-dim blocks per combine workgroup
       if (a.tab.is64)
         hipLaunchKernelGGL((attn_prefill_kernel<T, D, BN, 3, true>), sgrid, dim3(256), 0, st, a);

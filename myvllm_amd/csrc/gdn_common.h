@@ -250,7 +250,8 @@ GDN_DEVICE int wave_inclusive_scan_i32(int x) {
 // Block-wide lookup of the (sequence, tile) pair owning linear tile id
 // `target`, where sequence n is cut into ceil(len_n / tile_len) tiles laid
 // out sequence after sequence.  Every thread of the (256-thread) block must
-// call it; all receive the same answer, seq = -1 when target is past the end.
+// call it; all receive the same answer, seq = -1 when target is past the end
+// (tile then counts from the last tile's end).
 // Tile counts are 32-bit (the host bounds T and the grid).  `lds` must hold
 // at least 6 int32 values.
 template <int NT>
@@ -293,5 +294,5 @@ GDN_DEVICE void find_seq_tile(const void* cu, bool cu64, int64_t nseq, int64_t T
     if (lds[4] >= 0 || target < running) break;
   }
   seq = lds[4];
-  tile = lds[5];
+  tile = seq >= 0 ? lds[5] : target - running;
 }

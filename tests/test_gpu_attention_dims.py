@@ -75,3 +75,21 @@ def test_sequence_order(dev, N, Dh):
     got = flash_attention_prefill(case.q.to(dev), case.k.to(dev), case.v.to(dev), case.cu.to(dev), case.scale, 4, 1, Dh,
                                   Dh, True)
     assert_out_close(got, flash_attention_prefill_ref(case.q, case.k, case.v, case.cu, case.scale))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Dh, N", [(256, 3), (72, 3), (128, 70), (64, 1)])
+@pytest.mark.parametrize("first, tail", [(0, 1), (5, 0), (7, 900)])
+def test_uncovered_rows_are_zero(dev, Dh, N, first, tail):
+    """Rows before cu[0] and past cu[N], few and many, are zeroed by the workgroups past the last tile."""
+    lengths = [33 + (7 * n) % 64 for n in range(N)]
+    case = attn_varlen_case(lengths, seed=N + Dh, Hq=4, Hkv=2, D=Dh)
+    T = sum(lengths)
+    pad = lambda t: torch.cat([torch.full_like(t[:1], 9.0).expand(first, -1, -1), t,  # noqa: E731
+                               torch.full_like(t[:1], 9.0).expand(tail, -1, -1)]).contiguous().to(dev)
+    cu = (case.cu + first).to(dev)
+    out = torch.full((first + T + tail, 4, Dh), 5.0, dtype=case.q.dtype, device=dev)
+    print(f"uncovered rows D={Dh} N={N} first={first} tail={tail}", flush=True)
+    flash_attention_prefill(pad(case.q), pad(case.k), pad(case.v), cu, case.scale, 4, 2, Dh, Dh, True, out=out)
+    assert (out[:first] == 0).all() and (out[first + T:] == 0).all()
+    assert_out_close(out[first: first + T], flash_attention_prefill_ref(case.q, case.k, case.v, case.cu, case.scale))

@@ -67,3 +67,18 @@ def test_split_paged_prefill(dev, ctx, new, page, Hq, Hkv, Dh, dtype, tab64):
         assert_out_close(got, want)
         err = (got.double() - want.double()).norm() / want.double().norm().clamp_min(1e-12)
         assert err < 5e-3, f"relative error norm {err:.3e}"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tail", [1, 300])
+def test_split_paged_prefill_uncovered_rows(dev, tail):
+    case = paged_case([3000, 40], [5, 40], page=16, seed=3, Hq=16, Hkv=2, D=256)
+    assert _splits(45 + tail, 2, 16, 2, 256, case.block_tables.shape[1] * 16) > 1
+    q = torch.cat([case.q, torch.full_like(case.q[:1], 9.0).expand(tail, -1, -1)]).contiguous()
+    out = torch.full_like(q, 5.0).to(dev)
+    print(f"split paged prefill, {tail} uncovered rows", flush=True)
+    paged_flash_attention_prefill(q.to(dev), case.k_cache.to(dev), case.v_cache.to(dev), case.block_tables.to(dev),
+                                  case.context_lens.to(dev), case.cu.to(dev), None, case.scale, 16, out=out)
+    assert (out[45:] == 0).all()
+    assert_out_close(out[:45], paged_attention_ref(case.q, case.k_cache, case.v_cache, case.block_tables,
+                                                   case.context_lens, case.cu, case.scale))
