@@ -158,6 +158,12 @@ int gdn_chunk_prefill_split(const gdn_tensor* q, const gdn_tensor* k, const gdn_
                             const gdn_tensor* state_indices, const gdn_tensor* cu_seqlens,
                             gdn_tensor* out, const gdn_tensor* workspace, float scale, int32_t chunk_size,
                             void* stream);
+/* The same with gdn_chunk_prefill_ex's flags and output types (below). */
+int gdn_chunk_prefill_split_ex(const gdn_tensor* q, const gdn_tensor* k, const gdn_tensor* v,
+                               const gdn_tensor* g, const gdn_tensor* beta, gdn_tensor* state,
+                               const gdn_tensor* state_indices, const gdn_tensor* cu_seqlens,
+                               gdn_tensor* out, const gdn_tensor* workspace, float scale, int32_t chunk_size,
+                               int32_t flags, void* stream);
 
 /*
  * gdn_chunk_prefill with options (no counterpart in the reference).  With

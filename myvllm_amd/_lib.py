@@ -41,6 +41,7 @@ EXPORTED_SYMBOLS = (
     "gdn_chunk_prefill_ex",
     "gdn_chunk_prefill_workspace_size",
     "gdn_chunk_prefill_split",
+    "gdn_chunk_prefill_split_ex",
     "causal_conv1d_varlen",
     "causal_conv1d_step",
     "gdn_decode_step_fused",
@@ -127,6 +128,9 @@ def load() -> ctypes.CDLL:
         lib.gdn_chunk_prefill_workspace_size.argtypes = [ctypes.c_int64] * 6
         lib.gdn_chunk_prefill_split.restype = ctypes.c_int
         lib.gdn_chunk_prefill_split.argtypes = [_PT] * 10 + [ctypes.c_float, ctypes.c_int32, ctypes.c_void_p]
+        lib.gdn_chunk_prefill_split_ex.restype = ctypes.c_int
+        lib.gdn_chunk_prefill_split_ex.argtypes = [_PT] * 10 + [ctypes.c_float] + [ctypes.c_int32] * 2 + \
+            [ctypes.c_void_p]
         lib.causal_conv1d_varlen.restype = ctypes.c_int
         lib.causal_conv1d_varlen.argtypes = [_PT] * 6 + [ctypes.c_void_p]
         lib.causal_conv1d_step.restype = ctypes.c_int

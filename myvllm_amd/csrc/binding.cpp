@@ -179,6 +179,7 @@ typedef Entry<14, 7, int32_t, float> PagedDecode;
 typedef Entry<15, 6, int32_t, float> PagedDecodeNoalloc;
 typedef Entry<16, 13, int32_t, float, float> DecodeFusedNorm;
 typedef Entry<17, 3> Linear;
+typedef Entry<18, 10, float, int32_t, int32_t> ChunkPrefillSplitEx;
 typedef Size<0, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t> ChunkPrefillSize;
 typedef Size<1, int64_t, int64_t, int64_t, int64_t, int64_t, int64_t> PagedPrefillSize;
 typedef Size<2, int64_t, int64_t, int64_t, int32_t> PagedDecodeSize;
@@ -193,6 +194,7 @@ const Bound kBound[] = {
     GDN_BOUND("gdn_recurrent_step", RecurrentStep),
     GDN_BOUND("gdn_chunk_prefill", ChunkPrefill),
     GDN_BOUND("gdn_chunk_prefill_split", ChunkPrefillSplit),
+    GDN_BOUND("gdn_chunk_prefill_split_ex", ChunkPrefillSplitEx),
     GDN_BOUND("gdn_chunk_prefill_ex", ChunkPrefillEx),
     GDN_BOUND("causal_conv1d_varlen", ConvVarlen),
     GDN_BOUND("causal_conv1d_varlen_qknorm", ConvVarlenNorm),

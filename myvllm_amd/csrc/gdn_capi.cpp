@@ -22,7 +22,7 @@ int64_t gdn_chunk_prefill_split_floats(int64_t T, int64_t nseq, int64_t Hk, int6
 hipError_t gdn_chunk_prefill_split_launch(const gdn_tensor* q, const gdn_tensor* k, const gdn_tensor* v,
                                           const gdn_tensor* g, const gdn_tensor* beta, gdn_tensor* state,
                                           const gdn_tensor* idx, const gdn_tensor* cu, gdn_tensor* out,
-                                          float* workspace, float scale, hipStream_t st);
+                                          float* workspace, float scale, int32_t flags, hipStream_t st);
 hipError_t causal_conv1d_varlen_launch(const gdn_tensor* x, const gdn_tensor* w, gdn_tensor* cs,
                                        const gdn_tensor* idx, const gdn_tensor* cu, gdn_tensor* out,
                                        int64_t norm_ch, hipStream_t st);
@@ -360,17 +360,21 @@ GDN_EXPORT int64_t gdn_chunk_prefill_workspace_size(int64_t T, int64_t num_seqs,
   return gdn_chunk_prefill_split_floats(T, num_seqs, num_k_heads, num_v_heads, k_head_dim, v_head_dim);
 }
 
-GDN_EXPORT int gdn_chunk_prefill_split(const gdn_tensor* q, const gdn_tensor* k, const gdn_tensor* v,
-                                       const gdn_tensor* g, const gdn_tensor* beta, gdn_tensor* state,
-                                       const gdn_tensor* state_indices, const gdn_tensor* cu_seqlens,
-                                       gdn_tensor* out, const gdn_tensor* workspace, float scale, int32_t chunk_size,
-                                       void* stream) {
+GDN_EXPORT int gdn_chunk_prefill_split_ex(const gdn_tensor* q, const gdn_tensor* k, const gdn_tensor* v,
+                                          const gdn_tensor* g, const gdn_tensor* beta, gdn_tensor* state,
+                                          const gdn_tensor* state_indices, const gdn_tensor* cu_seqlens,
+                                          gdn_tensor* out, const gdn_tensor* workspace, float scale,
+                                          int32_t chunk_size, int32_t flags, void* stream) {
   if (chunk_size != 64) return GDN_ERR_CHUNK;
-  GDN_TRY(check_recurrent(q, k, v, g, beta, state, state_indices, out, cu_seqlens, true));
+  constexpr int32_t kKnown = GDN_PREFILL_ZERO_INIT | GDN_PREFILL_ACCUM_STATE | GDN_PREFILL_ACCUM_OUT;
+  if ((flags & ~kKnown) != 0) return GDN_ERR_ARG;
+  const bool f32_out = out && out->dtype == GDN_DTYPE_F32;
+  if ((flags & GDN_PREFILL_ACCUM_OUT) && !f32_out) return GDN_ERR_DTYPE;
+  GDN_TRY(check_recurrent(q, k, v, g, beta, state, state_indices, out, cu_seqlens, true, f32_out));
   const int64_t need = gdn_chunk_prefill_workspace_size(q->shape[0], cu_seqlens->shape[0] - 1, q->shape[1], v->shape[1],
                                                         q->shape[2], v->shape[2]);
   if (need == 0)
-    return launch_rc(gdn_chunk_prefill_launch(q, k, v, g, beta, state, state_indices, cu_seqlens, out, scale, 0,
+    return launch_rc(gdn_chunk_prefill_launch(q, k, v, g, beta, state, state_indices, cu_seqlens, out, scale, flags,
                                               kPrefillSpinLimit, -1, reinterpret_cast<hipStream_t>(stream)));
   GDN_TRY(check_desc(workspace, 1));
   if (workspace->dtype != GDN_DTYPE_F32) return GDN_ERR_DTYPE;
@@ -378,8 +382,18 @@ GDN_EXPORT int gdn_chunk_prefill_split(const gdn_tensor* q, const gdn_tensor* k,
   if (workspace->shape[0] < need) return GDN_ERR_SHAPE;
   if (!aligned(workspace, 16)) return GDN_ERR_ALIGN;
   return launch_rc(gdn_chunk_prefill_split_launch(q, k, v, g, beta, state, state_indices, cu_seqlens, out,
-                                                  reinterpret_cast<float*>(workspace->data), scale,
+                                                  reinterpret_cast<float*>(workspace->data), scale, flags,
                                                   reinterpret_cast<hipStream_t>(stream)));
+}
+
+GDN_EXPORT int gdn_chunk_prefill_split(const gdn_tensor* q, const gdn_tensor* k, const gdn_tensor* v,
+                                       const gdn_tensor* g, const gdn_tensor* beta, gdn_tensor* state,
+                                       const gdn_tensor* state_indices, const gdn_tensor* cu_seqlens,
+                                       gdn_tensor* out, const gdn_tensor* workspace, float scale, int32_t chunk_size,
+                                       void* stream) {
+  GDN_TRY(check_recurrent(q, k, v, g, beta, state, state_indices, out, cu_seqlens, true));
+  return gdn_chunk_prefill_split_ex(q, k, v, g, beta, state, state_indices, cu_seqlens, out, workspace, scale,
+                                    chunk_size, 0, stream);
 }
 
 GDN_EXPORT int gdn_chunk_prefill_ex(const gdn_tensor* q, const gdn_tensor* k, const gdn_tensor* v,

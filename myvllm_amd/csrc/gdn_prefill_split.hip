@@ -187,14 +187,15 @@ GDN_DEVICE void rows_kq(const bf16x8 (&raw)[8], f16x8 (&out)[8]) {
 // of the chain Gram -> diagonal blocks -> T -> W, U; three workgroups per CU
 // (47 KB of LDS: Q stays in registers and P is formed transposed, so that its
 // accumulators are the scan's fragments).
-template <bool F16>
+template <bool F16, bool OUT32>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void gdn_prepare_kernel(SplitArgs sa) {
   __shared__ PrepSmem sm;
   const PrefillArgs& a = sa.p;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int64_t bid = blockIdx.x;
-  zero_uncovered_rows<2>(a.out, a.o_s0, a.o_s1, a.Hv, VD, a.cu, a.cu64, a.nseq, a.T, bid, gridDim.x, tid, 256);
+  if (!(a.flags & GDN_PREFILL_ACCUM_OUT))
+    zero_uncovered_rows<OUT32 ? 4 : 2>(a.out, a.o_s0, a.o_s1, a.Hv, VD, a.cu, a.cu64, a.nseq, a.T, bid, gridDim.x, tid, 256);
   // the two v-heads of a k-head on one XCD, as in the fused kernel
   const int64_t work = 2 * ((bid >> 4) * 8 + (bid & 7)) + ((bid >> 3) & 1);
   const int64_t slot = work / a.Hv;
@@ -481,7 +482,7 @@ GDN_DEVICE float pow2_biased(int k) { return __builtin_bit_cast(float, (uint32_t
 // chunk against 1.67 with four waves doing both and all loads at the end.
 // An item's column groups run on one XCD (workgroups are dealt
 // round-robin), which reads its chunks' records from HBM once.
-template <bool F16, int NT>
+template <bool F16, int NT, bool OUT32>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void gdn_scan_kernel(SplitArgs sa) {
   __shared__ ScanSmem smt[NT];
   constexpr int kWgs = kGroups / NT;  // workgroups per item
@@ -509,10 +510,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
   seq_range(a.cu, a.cu64, seq, a.T, s0, s1);
   const int64_t st_slot = load_index(a.idx, seq, a.idx64);
   const int c = lane & 15, q = lane >> 4;
-  bf16_t* const ob = a.out + h * a.o_s1 + kCols * cg;
+  // (byte addresses: the output holds 16-bit elements, or fp32 ones with OUT32)
+  constexpr uint32_t kOut = OUT32 ? 4 : 2;
+  char* const ob = reinterpret_cast<char*>(a.out) + (h * a.o_s1 + kCols * cg) * kOut;
   if (st_slot < 0 || st_slot >= a.num_slots) {  // a padding sequence: zero rows, no state
+    if (a.flags & GDN_PREFILL_ACCUM_OUT) return;  // (nothing to add)
     for (int64_t t = s0 + (tid >> 4); t < s1; t += 32)
-      for (int nt = 0; nt < NT; ++nt) ob[t * a.o_s0 + kCols * nt + c] = (bf16_t)0.f;
+      for (int nt = 0; nt < NT; ++nt) {
+        char* p = ob + (t * a.o_s0 + kCols * nt + c) * kOut;
+        if constexpr (OUT32) *reinterpret_cast<float*>(p) = 0.f;
+        else *reinterpret_cast<uint16_t*>(p) = 0;
+      }
     return;
   }
   if (nc == 0) return;
@@ -550,8 +558,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
       d.p[1] = frag(l16b, pr + (w >= 2 ? kPieceBytes : 0));
     };
     // output rows 16w + 4q + r of a chunk, through a descriptor that ends after its last row
-    const uint32_t orow = (uint32_t)a.o_s0 * 2u;
-    const uint32_t ooff = (uint32_t)(16 * w + 4 * q) * orow + 2u * c;
+    const uint32_t orow = (uint32_t)a.o_s0 * kOut;
+    const uint32_t ooff = (uint32_t)(16 * w + 4 * q) * orow + kOut * c;
     // A touch reads one dword of each 128-byte line of a chunk's records into
     // L2, kTouch chunks before they are loaded for use, the lines dealt over
     // the item's output waves.  Without it every one of the item's workgroups
@@ -593,7 +601,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
       lds_barrier();
       const int64_t t0 = s0 + (int64_t)C * ch;
       const uint32_t rows = (uint32_t)(s1 - t0 < C ? s1 - t0 : C);
-      const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(ob + t0 * a.o_s0, 0, rows * orow, 0x00020000);
+      const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(ob + t0 * (int64_t)orow, 0, rows * orow, 0x00020000);
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
         const ScanSmem& sm = smt[nt];
@@ -604,10 +612,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const float o = a.scale * fmaf(d.eg[r], QS[nt][r], O[r] * vu);
-          uint16_t ov;
-          if constexpr (F16) ov = __builtin_bit_cast(uint16_t, (f16_t)o);
-          else ov = __builtin_bit_cast(uint16_t, (bf16_t)o);
-          __builtin_amdgcn_raw_buffer_store_b16(ov, ro, ooff + r * orow, 2 * kCols * nt, 0);
+          if constexpr (OUT32) {
+            float y = o;
+            if (a.flags & GDN_PREFILL_ACCUM_OUT)
+              y += __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ro, ooff + r * orow, kOut * kCols * nt, 0));
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, y), ro, ooff + r * orow, kOut * kCols * nt, 0);
+          } else {
+            uint16_t ov;
+            if constexpr (F16) ov = __builtin_bit_cast(uint16_t, (f16_t)o);
+            else ov = __builtin_bit_cast(uint16_t, (bf16_t)o);
+            __builtin_amdgcn_raw_buffer_store_b16(ov, ro, ooff + r * orow, kOut * kCols * nt, 0);
+          }
         }
       }
       load(dn, next(ch));
@@ -665,7 +680,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) S[nt][mt][r] = sg[(16 * mt + r) * VD + kCols * nt];
+      for (int r = 0; r < 4; ++r)
+        S[nt][mt][r] = a.flags & GDN_PREFILL_ZERO_INIT ? 0.f : sg[(16 * mt + r) * VD + kCols * nt];
   // The next chunk's loads go out in four groups, each behind the LDS reads or
   // MFMAs that the wave is about to wait for (the scheduling barriers keep them
   // there): all at once they held up the chain for as long as they took to issue.
@@ -800,7 +816,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) sg[(16 * mt + r) * VD + kCols * nt] = S[nt][mt][r];
+      for (int r = 0; r < 4; ++r) {
+        float* p = sg + (16 * mt + r) * VD + kCols * nt;
+        *p = a.flags & GDN_PREFILL_ACCUM_STATE ? *p + S[nt][mt][r] : S[nt][mt][r];
+      }
 }
 
 }  // namespace
@@ -826,16 +845,16 @@ int64_t gdn_chunk_prefill_split_floats(int64_t T, int64_t nseq, int64_t Hk, int6
 }
 
 namespace {
-template <bool F16>
+template <bool F16, bool OUT32>
 hipError_t launch_split(const SplitArgs& sa, int nt, hipStream_t st) {
   // (the work maps cover whole groups of 16)
   const dim3 pgrid((unsigned)((sa.slots * sa.p.Hv + 15) / 16 * 16));
   const dim3 sgrid((unsigned)((sa.p.nseq * sa.p.Hv + 15) / 16 * 16 * (kGroups / nt)));
-  gdn_prepare_kernel<F16><<<pgrid, dim3(256), 0, st>>>(sa);
+  gdn_prepare_kernel<F16, OUT32><<<pgrid, dim3(256), 0, st>>>(sa);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  if (nt == 1) gdn_scan_kernel<F16, 1><<<sgrid, dim3(512), 0, st>>>(sa);
-  else gdn_scan_kernel<F16, 2><<<sgrid, dim3(512), 0, st>>>(sa);
+  if (nt == 1) gdn_scan_kernel<F16, 1, OUT32><<<sgrid, dim3(512), 0, st>>>(sa);
+  else gdn_scan_kernel<F16, 2, OUT32><<<sgrid, dim3(512), 0, st>>>(sa);
   return hipGetLastError();
 }
 }  // namespace
@@ -843,12 +862,14 @@ hipError_t launch_split(const SplitArgs& sa, int nt, hipStream_t st) {
 hipError_t gdn_chunk_prefill_split_launch(const gdn_tensor* q, const gdn_tensor* k, const gdn_tensor* v,
                                           const gdn_tensor* g, const gdn_tensor* beta, gdn_tensor* state,
                                           const gdn_tensor* idx, const gdn_tensor* cu, gdn_tensor* out,
-                                          float* workspace, float scale, hipStream_t st) {
+                                          float* workspace, float scale, int32_t flags, hipStream_t st) {
   SplitArgs sa;
   sa.p = prefill_args(q, k, v, g, beta, state, idx, cu, out, scale);
+  sa.p.flags = flags;
   sa.ws = reinterpret_cast<char*>(workspace);
   sa.slots = sa.p.T / C + sa.p.nseq;
   sa.Hk = (int32_t)q->shape[1];
   const int nt = sa.p.nseq * sa.p.Hv <= kOneGroupItems ? 1 : 2;
-  return q->dtype == GDN_DTYPE_F16 ? launch_split<true>(sa, nt, st) : launch_split<false>(sa, nt, st);
+  if (out->dtype == GDN_DTYPE_F32) return launch_split<true, true>(sa, nt, st);  // (q, k, v fp16: checked by the caller)
+  return q->dtype == GDN_DTYPE_F16 ? launch_split<true, false>(sa, nt, st) : launch_split<false, false>(sa, nt, st);
 }

@@ -111,9 +111,13 @@ def _chunk_gated_delta_rule_fp32(q, k, v, g, beta, state, idx, cu_seqlens, scale
     v_hi = v.to(torch.float16)
     v_lo = (v - v_hi.float()).to(torch.float16)
     o = torch.empty(v.shape, dtype=torch.float32, device=dev) if out is None or not _lib.vec16_ok(out) else out
-    chunk_prefill_ex(qh, kh, v_hi, g, beta, state, idx, cu_seqlens, o, scale)
-    chunk_prefill_ex(qh, kh, v_lo, g, beta, state, idx, cu_seqlens, o, scale,
-                     flags=_lib.PREFILL_ZERO_INIT | _lib.PREFILL_ACCUM_STATE | _lib.PREFILL_ACCUM_OUT)
+    ws = _prefill_workspace(qh, v_hi, cu_seqlens)  # (both passes use it in turn, on one stream)
+    for vp, flags in ((v_hi, 0), (v_lo, _lib.PREFILL_ZERO_INIT | _lib.PREFILL_ACCUM_STATE | _lib.PREFILL_ACCUM_OUT)):
+        if ws is not None:
+            _lib.call("gdn_chunk_prefill_split_ex", qh, kh, vp, g, beta, state, idx, cu_seqlens, o, ws, float(scale),
+                      CHUNK_SIZE, flags)
+        else:
+            chunk_prefill_ex(qh, kh, vp, g, beta, state, idx, cu_seqlens, o, scale, flags=flags)
     if out is not None and o is not out:
         out.copy_(o)
         return out

@@ -115,3 +115,33 @@ def test_split_prefill_padding_strides_and_graph(dev):
         assert_out_close(out, o_ref)
         assert (out[500:800] == 0).all() and (out[T - 9:] == 0).all()
         assert_state_close(st, st_ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lengths, Hk, Hv", [([200, 333], 2, 4), ([450, 700, 64], 4, 16)])
+def test_split_prefill_fp32(dev, lengths, Hk, Hv):
+    """fp32 q, k, v: both passes (v hi from the slot's state, v lo added from zero) run split, with
+    a padding sequence and an uncovered row; against the fused kernel's passes on the same inputs."""
+    c = _case(lengths, Hk, Hv, dtype=torch.float32)
+    T = sum(lengths)
+    assert _floats(T + 1, len(lengths), Hk, Hv) > 0
+    pad = lambda t: torch.cat([t, t[:1]]).contiguous().to(dev)  # noqa: E731
+    d = [pad(t) for t in (c.q, c.k, c.v, c.g, c.beta)]
+    idx = c.idx.clone()
+    idx[-1] = -1
+    print(f"split prefill fp32 {lengths} Hk={Hk} Hv={Hv}", flush=True)
+    st = c.state.to(dev)
+    o = chunk_gated_delta_rule(*d, st, idx.to(dev), c.cu.to(dev), out=torch.full_like(d[2], 7.0))
+    assert o.dtype == torch.float32 and (o[T:] == 0).all() and (o[T - lengths[-1]: T] == 0).all()
+    st2, o2 = c.state.to(dev), torch.full_like(d[2], 7.0)
+    qh, kh, vh = d[0].half(), d[1].half(), d[2].half()
+    args = (d[3], d[4], st2, idx.to(dev), c.cu.to(dev), o2, 128 ** -0.5)
+    chunk_prefill_ex(qh, kh, vh, *args)
+    chunk_prefill_ex(qh, kh, (d[2] - vh.float()).half(), *args,
+                     flags=_lib.PREFILL_ZERO_INIT | _lib.PREFILL_ACCUM_STATE | _lib.PREFILL_ACCUM_OUT)
+    # (the splits of either keep 22 bits; P and the hi parts that feed o only keep 11)
+    assert (st - st2).norm() < 3e-6 * st2.norm()
+    assert (o - o2).norm() < 2e-3 * o2.norm()
+    st_ref = c.state.clone()
+    o_ref = chunk_gated_delta_rule_ref(c.q, c.k, c.v, c.g, c.beta, st_ref, idx, c.cu)
+    assert_out_close(o[:T], o_ref, rtol=2e-3, atol=1e-3)
