@@ -54,7 +54,7 @@ GDN_DEVICE float softplus_f32(float x) { return x > 20.f ? x : log1pf(__expf(x))
 // states alone take 32+ VGPRs per thread; forcing two workgroups per CU there
 // spills freshly loaded state registers (measured 267 us against 203 us for
 // batch 256 with two heads), so the register budget is left to the compiler.
-template <typename TX, int W, int K, int V, int NH>
+template <typename TX, int W, int K, int V, int NH, bool NORM>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(NH <= 1 ? 8 : 4, 8)))
 void gdn_decode_fused_kernel(FusedArgs a) {
   constexpr int CG = V / 4;             // float4 column groups per state row
@@ -194,6 +194,7 @@ void gdn_decode_fused_kernel(FusedArgs a) {
   // softplus(a + dt_bias), beta = sigmoid(b); loaded only now, when the state
   // loads they would otherwise wait behind have landed), sum the waves'
   // partials and form d and the output
+  float fo[4] = {0.f, 0.f, 0.f, 0.f};  // a finisher's outputs
   if (tid < CG * NH) {
     const int n = tid / CG, cc = tid % CG;
     const int h = h0 + n;
@@ -218,32 +219,40 @@ void gdn_decode_fused_kernel(FusedArgs a) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) d[j] = bn * (sv[n][4 * cc + j] - eg * kS[j]);
     sd[n][cc] = d;
-    TX* o = reinterpret_cast<TX*>(a.out) + b * a.o_s0 + (h0 + n) * a.o_s1;
-    float y[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) y[j] = fmaf(eg, qS[j], qkn * d[j]);
-    if (a.gate) {
-      // the head's gated RMSNorm (rms_norm_gated_kernel's), before o is
-      // rounded: its CG = 32 threads are one half of a wave
-      static_assert(CG == 32, "a head's finishers are half a wave");
+    for (int j = 0; j < 4; ++j) fo[j] = fmaf(eg, qS[j], qkn * d[j]);
+    if constexpr (!NORM) {
+      TX* o = reinterpret_cast<TX*>(a.out) + b * a.o_s0 + (h0 + n) * a.o_s1;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) o[4 * cc + j] = from_f32<TX>(fo[j]);
+    }
+  }
+  __syncthreads();
+  if constexpr (NORM) {
+    // the heads' gated RMSNorm (rms_norm_gated_kernel's), before o is rounded,
+    // while the other waves store their states: a head's CG = 32 finishers are
+    // one half of a wave
+    static_assert(CG == 32, "a head's finishers are half a wave");
+    if (tid < CG * NH) {
+      const int n = tid / CG, cc = tid % CG;
       const TX* z = reinterpret_cast<const TX*>(a.gate) + b * a.g_s0 + (h0 + n) * a.g_s1;
+      TX* o = reinterpret_cast<TX*>(a.out) + b * a.o_s0 + (h0 + n) * a.o_s1;
       float ss = 0.f;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) ss = fmaf(y[j], y[j], ss);
+      for (int j = 0; j < 4; ++j) ss = fmaf(fo[j], fo[j], ss);
 #pragma unroll
       for (int off = 1; off < CG; off <<= 1) ss += __shfl_xor(ss, off, 64);
       const float rn = rsqrtf(ss * (1.f / V) + a.eps);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const float g = to_f32(z[4 * cc + j]);
-        y[j] = y[j] * rn * scalar_raw_f32(load_scalar_raw(a.nw, 4 * cc + j, a.nw_dtype), a.nw_dtype) *
-               (g / (1.f + __expf(-g)));
+        o[4 * cc + j] = from_f32<TX>(fo[j] * rn *
+                                     scalar_raw_f32(load_scalar_raw(a.nw, 4 * cc + j, a.nw_dtype), a.nw_dtype) *
+                                     (g / (1.f + __expf(-g))));
       }
     }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) o[4 * cc + j] = from_f32<TX>(y[j]);
+    __builtin_amdgcn_sched_barrier(0);
   }
-  __syncthreads();
 #pragma unroll
   for (int n = 0; n < NH; ++n) {
     const float eg = seg[n];
@@ -259,14 +268,20 @@ void gdn_decode_fused_kernel(FusedArgs a) {
   }
 }
 
-template <typename TX>
+template <typename TX, bool NORM>
 hipError_t launch_heads(const FusedArgs& a, int nh, int64_t nblocks, hipStream_t st) {
+  const dim3 grid((unsigned)nblocks), block(kThreads);
   switch (nh) {
-    case 1: gdn_decode_fused_kernel<TX, 4, 128, 128, 1><<<dim3((unsigned)nblocks), dim3(kThreads), 0, st>>>(a); break;
-    case 2: gdn_decode_fused_kernel<TX, 4, 128, 128, 2><<<dim3((unsigned)nblocks), dim3(kThreads), 0, st>>>(a); break;
-    default: gdn_decode_fused_kernel<TX, 4, 128, 128, 4><<<dim3((unsigned)nblocks), dim3(kThreads), 0, st>>>(a); break;
+    case 1: gdn_decode_fused_kernel<TX, 4, 128, 128, 1, NORM><<<grid, block, 0, st>>>(a); break;
+    case 2: gdn_decode_fused_kernel<TX, 4, 128, 128, 2, NORM><<<grid, block, 0, st>>>(a); break;
+    default: gdn_decode_fused_kernel<TX, 4, 128, 128, 4, NORM><<<grid, block, 0, st>>>(a); break;
   }
   return hipGetLastError();
+}
+
+template <typename TX>
+hipError_t launch_typed(const FusedArgs& a, int nh, int64_t nblocks, hipStream_t st) {
+  return a.gate ? launch_heads<TX, true>(a, nh, nblocks, st) : launch_heads<TX, false>(a, nh, nblocks, st);
 }
 
 }  // namespace
@@ -306,8 +321,8 @@ hipError_t gdn_decode_fused_launch(const gdn_tensor* x, const gdn_tensor* w, gdn
   const int64_t nblocks = x->shape[0] * (int64_t)Hk;
   if (nblocks == 0) return hipSuccess;
   switch (x->dtype) {
-    case GDN_DTYPE_BF16: return launch_heads<bf16_t>(a, nh, nblocks, st);
-    case GDN_DTYPE_F16: return launch_heads<f16_t>(a, nh, nblocks, st);
-    default: return launch_heads<float>(a, nh, nblocks, st);
+    case GDN_DTYPE_BF16: return launch_typed<bf16_t>(a, nh, nblocks, st);
+    case GDN_DTYPE_F16: return launch_typed<f16_t>(a, nh, nblocks, st);
+    default: return launch_typed<float>(a, nh, nblocks, st);
   }
 }

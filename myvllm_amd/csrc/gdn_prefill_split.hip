@@ -7,8 +7,8 @@
 // not depend on the state is computed by one workgroup per (chunk, v-head)
 // first, into a workspace, and the walk over the chunks that is left runs one
 // workgroup per (item, 16 or 32 value columns): no product mixes value columns,
-// so an item's column groups are independent.  That prompt takes 106 us: 44 to
-// prepare 1,472 (chunk, v-head) pairs, 59 to scan 46 chunks.
+// so an item's column groups are independent.  That prompt takes 95 us: 37 to
+// prepare 1,472 (chunk, v-head) pairs, 56 to scan 46 chunks.
 //
 // gdn_prepare_kernel, per chunk (notation of gdn_prefill.hip):
 //   T = (I + A)^-1,  P                     as in the fused kernel
@@ -828,7 +828,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
 // when the fused kernel serves it.  Split wins where the fused kernel's items
 // leave most CUs idle for a few chunks.  Measured, fused -> split, prompts x
 // tokens at 16 / 32 heads: 1 x 128 21 -> 20 us, 1 x 192 27 -> 22, 1 x 384 40 ->
-// 26, 1 x 1,024 88 -> 45, 1 x 2,943 225 -> 106, 1 x 16,384 1,186 -> 618, 2 x
+// 26, 1 x 1,024 88 -> 45, 1 x 2,943 223 -> 95, 1 x 16,384 1,186 -> 618, 2 x
 // 256 32 -> 28, 2 x 512 51 -> 41, 2 x 1,500 126 -> 95, 2 x 2,943 226 -> 202,
 // and past 64 items 3 x 1,000 91 -> 104, 4 x 2,048 164 -> 276: the records
 // (91 KB per chunk and head, written and read once) then cost more than the
