@@ -242,9 +242,14 @@ def vec16_ok(t: torch.Tensor) -> bool:
     return vec16(t) is t
 
 
+def same_device(*tensors: torch.Tensor) -> bool:
+    """Whether all of them are plain tensors on one HIP device."""
+    return (_fast or _load_fast()).same_device(*tensors) >= 0
+
+
 def require_device(*tensors: torch.Tensor) -> torch.device:
     """All tensors must live on one HIP device (the kernels dereference the pointers)."""
-    if (_fast or _load_fast()).same_device(*tensors) >= 0:
+    if same_device(*tensors):
         return next(t for t in tensors if t is not None).device
     dev = None
     for t in tensors:

@@ -177,9 +177,12 @@ class GatedDeltaNet(nn.Module):
 
     def _native_decode(self, x: torch.Tensor) -> bool:
         """Whether a decode step runs as three launches (:meth:`_forward_decode`):
-        plain 16-bit tensors in one dtype with nothing recording the torch
-        products that the general path makes (autograd, autocast, a dispatch
-        or function mode, a compiler)."""
+        plain 16-bit tensors in one dtype and on one device, with nothing
+        recording the torch products that the general path makes (autograd,
+        autocast, a dispatch or function mode, a compiler).  The caches and
+        indices are on x's device already (:meth:`_check_inputs`); a parameter
+        that is not goes to the general path, whose ops refuse it: the kernels
+        would take its pointer as it is."""
         if not x.is_cuda or x.dtype not in (torch.bfloat16, torch.float16) or x.shape[0] == 0:
             return False
         if torch.is_grad_enabled() and (x.requires_grad or self.in_proj.requires_grad or self.out_proj.requires_grad):
@@ -191,7 +194,9 @@ class GatedDeltaNet(nn.Module):
             return False
         return (type(x) is torch.Tensor and type(self.in_proj) is nn.Parameter and type(self.out_proj) is nn.Parameter
                 and self.in_proj.dtype == x.dtype and self.out_proj.dtype == x.dtype
-                and self.norm_weight.dim() == 1)
+                and self.norm_weight.dim() == 1
+                and _lib.same_device(x, self.in_proj, self.conv1d_weight, self.A_log, self.dt_bias, self.norm_weight,
+                                     self.out_proj))
 
     def _forward_decode(self, x, conv_state_indices, recurrent_state_indices) -> torch.Tensor:
         """A decode step: in_proj, the fused step with the gated norm, out_proj."""
@@ -199,8 +204,6 @@ class GatedDeltaNet(nn.Module):
         proj = _linear(x, self.in_proj)
         cz = self.conv_dim + self.v_size
         o = torch.empty(T, Hv, V, dtype=x.dtype, device=x.device)
-        _lib.require_device(x, self.in_proj, self.conv1d_weight, self.A_log, self.dt_bias, self.norm_weight,
-                            self.out_proj)
         _lib.call("gdn_decode_step_fused_norm", proj[:, : self.conv_dim], self.conv1d_weight, self.conv_state,
                   conv_state_indices, proj[:, cz + Hv:], proj[:, cz: cz + Hv], self.A_log, self.dt_bias,
                   self.recurrent_state, recurrent_state_indices, proj[:, self.conv_dim: cz].view(T, Hv, V),
