@@ -128,6 +128,19 @@ struct AttnArgs {
 template <int D> constexpr int64_t prefill_part_wave() { return 32 * D + 128; }
 template <int D> constexpr int64_t prefill_part_floats() { return 4 * prefill_part_wave<D>(); }
 
+// Element offset in a query row of `dim` dims of the 8 that lane half hh reads
+// for k-step s; a piece past the row reads the row's first (its value is
+// dropped), so that no lane reads outside the row (dims of 8 have one piece).
+__host__ __device__ constexpr int q_piece(int s, int hh, int dim) {
+  return 16 * s + 8 * hh < dim ? 16 * s + 8 * hh : 0;
+}
+constexpr bool q_pieces_inside(int dq) {
+  for (int dim = 8; dim <= dq; dim += 8)
+    for (int p = 0; p < dq / 8; ++p)
+      if (q_piece(p / 2, p % 2, dim) + 8 > dim) return false;
+  return true;
+}
+
 template <bool PAGED>
 GDN_DEVICE const char* kv_row(const KvSource& s, const PagedTable& tb, int64_t n, int64_t s0, int64_t j, int kvh) {
   if (PAGED) {
@@ -337,9 +350,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   // where the fragments are staged, below)
   v8 qf[NKS];
   {
-    const T* qp = reinterpret_cast<const T*>(a.q) + (s0 + (qvalid ? qi : 0)) * a.q_st + (int64_t)head * a.q_sh + 8 * hh;
+    static_assert(!RAG || q_pieces_inside(DQ), "query pieces are read inside their row");
+    const T* qp = reinterpret_cast<const T*>(a.q) + (s0 + (qvalid ? qi : 0)) * a.q_st + (int64_t)head * a.q_sh;
 #pragma unroll
-    for (int s = 0; s < NKS; ++s) qf[s] = *reinterpret_cast<const v8*>(qp + (!RAG || 16 * s + 8 * hh < a.dim ? 16 * s : 0));
+    for (int s = 0; s < NKS; ++s) qf[s] = *reinterpret_cast<const v8*>(qp + (RAG ? q_piece(s, hh, a.dim) : 16 * s + 8 * hh));
   }
   // the softmax below assumes c > 0: a negative scale is folded into q (an
   // exact sign flip), a zero scale is q = 0 with c = 1 (equal weights)
