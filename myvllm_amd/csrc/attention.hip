@@ -300,6 +300,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   const uint32_t piece = SPLIT && !past ? blockIdx.x / srows : 0u;
   const uint32_t row_id = past ? srows + (blockIdx.x - srows * (uint32_t)a.splits) : blockIdx.x - piece * srows;
   const SeqTile st = attn_tile_lookup<D, PAGED>(a, 32 * qsubs, row_id / hg, lookup);
+  // (no tile is left past the grid's rows unless the offsets decrease: nothing
+  // is kept for it in the workspace)
+  if (past && st.seq >= 0) return;
   if (st.seq < 0) {
     if (piece > 0) return;
     const uint32_t tiles = (SPLIT ? srows : gridDim.x - hg) / hg + 1;

@@ -82,3 +82,24 @@ def test_split_paged_prefill_uncovered_rows(dev, tail):
     assert (out[45:] == 0).all()
     assert_out_close(out[:45], paged_attention_ref(case.q, case.k_cache, case.v_cache, case.block_tables,
                                                    case.context_lens, case.cu, case.scale))
+
+
+@pytest.mark.gpu
+def test_split_paged_prefill_decreasing_offsets(dev):
+    """Offsets that decrease give more query tiles than the grid has rows: those past it have no
+    place in the workspace, which ends where its size function says."""
+    T, N, cap = 256, 5, 4096
+    case = paged_case([cap] * N, [T] * N, page=16, seed=5, Hq=16, Hkv=2, D=256)
+    n = _lib.load().paged_attention_prefill_workspace_size(T, N, 16, 2, 256, case.block_tables.shape[1] * 16)
+    assert n > 0
+    guard = 1 << 20
+    buf = torch.full((n + guard,), 3.0, device=dev)
+    cu = torch.tensor([0, T, 0, T, 0, T], dtype=torch.int32, device=dev)
+    q = case.q[:T].to(dev)
+    out = torch.empty_like(q)
+    print("split paged prefill, decreasing offsets", flush=True)
+    _lib.call("paged_attention_prefill_split", q, *(t.to(dev) for t in (case.k_cache, case.v_cache, case.block_tables,
+                                                                        case.context_lens)), cu, out, buf[:n], T,
+              float(case.scale))
+    assert (buf[n:] == 3.0).all()
+    assert torch.isfinite(out).all()
