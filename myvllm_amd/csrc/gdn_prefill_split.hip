@@ -557,7 +557,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
       d.p[0] = frag(l16b, pr);
       d.p[1] = frag(l16b, pr + (w >= 2 ? kPieceBytes : 0));
     };
-    // output rows 16w + 4q + r of a chunk, through a descriptor that ends after its last row
+    // output rows 16w + 4q + r of a chunk, through a descriptor that ends with
+    // this workgroup's columns of its last row (64 whole rows of the largest
+    // token stride, 2^24, are 2^32 bytes of fp32)
     const uint32_t orow = (uint32_t)a.o_s0 * kOut;
     const uint32_t ooff = (uint32_t)(16 * w + 4 * q) * orow + kOut * c;
     // A touch reads one dword of each 128-byte line of a chunk's records into
@@ -601,7 +603,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
       lds_barrier();
       const int64_t t0 = s0 + (int64_t)C * ch;
       const uint32_t rows = (uint32_t)(s1 - t0 < C ? s1 - t0 : C);
-      const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(ob + t0 * (int64_t)orow, 0, rows * orow, 0x00020000);
+      const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
+          ob + t0 * (int64_t)orow, 0, (rows - 1) * orow + kOut * kCols * NT, 0x00020000);
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
         const ScanSmem& sm = smt[nt];

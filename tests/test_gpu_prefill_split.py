@@ -145,3 +145,20 @@ def test_split_prefill_fp32(dev, lengths, Hk, Hv):
     st_ref = c.state.clone()
     o_ref = chunk_gated_delta_rule_ref(c.q, c.k, c.v, c.g, c.beta, st_ref, idx, c.cu)
     assert_out_close(o[:T], o_ref, rtol=2e-3, atol=1e-3)
+
+
+@pytest.mark.gpu
+def test_split_prefill_fp32_largest_token_stride(dev):
+    """fp32 rows 2^24 elements apart, the largest stride the entry takes (13 GB of rows): 64 of
+    them are 2^32 bytes.  Bit for bit the result of contiguous rows."""
+    c = _case([200], Hk=1, Hv=2, dtype=torch.float32)
+    assert _floats(200, 1, 1, 2) > 0
+    d = [t.to(dev) for t in (c.q, c.k, c.v, c.g, c.beta)]
+    print("split prefill fp32, token stride 2^24", flush=True)
+    outs = []
+    for out in (None, torch.empty(199 * 2**24 + 256, device=dev).as_strided((200, 2, 128), (2**24, 128, 1))):
+        st = c.state.to(dev)
+        if out is not None:
+            out.fill_(7.0)
+        outs.append((chunk_gated_delta_rule(*d, st, c.idx.to(dev), c.cu.to(dev), out=out).clone(), st))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
