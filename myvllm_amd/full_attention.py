@@ -189,6 +189,19 @@ def paged_flash_attention_decode_noalloc(
     return out
 
 
+def _prefill_workspace(q, k_cache, block_tables, cu_seqlens, page):
+    """Workspace of the split paged prefill when these sizes run split, else
+    None: one workgroup per row, also where the memory is not to be had."""
+    n = _lib.workspace_size("paged_attention_prefill_workspace_size", q.shape[0], cu_seqlens.numel() - 1, q.shape[1],
+                            k_cache.shape[2], q.shape[2], block_tables.shape[1] * page)
+    if n <= 0:
+        return None
+    try:
+        return torch.empty(n, dtype=torch.float32, device=q.device)
+    except torch.OutOfMemoryError:
+        return None
+
+
 def paged_flash_attention_prefill(
     q: torch.Tensor,
     k_cache: torch.Tensor,
@@ -208,7 +221,7 @@ def paged_flash_attention_prefill(
     per-16-row work list) is accepted for interface parity and not needed:
     the kernel tiles the queries itself from ``cu_seqlens``.  Few new tokens
     over a long cache are split over the keys as well; the partials then take a
-    temporary workspace of up to 512 MiB."""
+    temporary workspace of up to 512 MiB, without which nothing is split."""
     if k_cache.shape[1] != page_block_size:
         raise ValueError(f"page_block_size {page_block_size} != k_cache.shape[1] {k_cache.shape[1]}")
     dev = _lib.require_device(q, k_cache, v_cache, page_block_tables, context_lens, cu_seqlens)
@@ -216,10 +229,8 @@ def paged_flash_attention_prefill(
         max_seqlen = _max_seqlen(cu_seqlens)
     q, k_cache, v_cache = _lib.vec16(q), _lib.vec16(k_cache), _lib.vec16(v_cache)
     o = _out_for(out, (q.shape[0], q.shape[1], v_cache.shape[-1]), q.dtype, dev)
-    n_ws = _lib.workspace_size("paged_attention_prefill_workspace_size", q.shape[0], cu_seqlens.numel() - 1, q.shape[1],
-                               k_cache.shape[2], q.shape[2], page_block_tables.shape[1] * page_block_size)
-    if n_ws > 0:
-        ws = torch.empty(n_ws, dtype=torch.float32, device=dev)
+    ws = _prefill_workspace(q, k_cache, page_block_tables, cu_seqlens, page_block_size)
+    if ws is not None:
         _lib.call("paged_attention_prefill_split", q, k_cache, v_cache, page_block_tables, context_lens, cu_seqlens, o,
                   ws, int(max_seqlen), float(scale))
     else:

@@ -103,3 +103,24 @@ def test_split_paged_prefill_decreasing_offsets(dev):
               float(case.scale))
     assert (buf[n:] == 3.0).all()
     assert torch.isfinite(out).all()
+
+
+@pytest.mark.gpu
+def test_paged_prefill_without_room_for_a_workspace(dev, monkeypatch):
+    """Where the workspace is not to be had the call runs unsplit, as it needs none."""
+    case = paged_case([3000, 40], [5, 40], page=16, seed=3, Hq=16, Hkv=2, D=256)
+    d = [t.to(dev) for t in (case.q, case.k_cache, case.v_cache, case.block_tables, case.context_lens, case.cu)]
+    plain = torch.empty_like(d[0])
+    _lib.call("paged_attention_prefill", *d, plain, 40, float(case.scale))
+    real, refused = torch.empty, []
+
+    def empty(*a, **kw):
+        if kw.get("dtype") is torch.float32:
+            refused.append(a)
+            raise torch.OutOfMemoryError("no room")
+        return real(*a, **kw)
+
+    monkeypatch.setattr(torch, "empty", empty)
+    print("paged prefill, no workspace", flush=True)
+    out = paged_flash_attention_prefill(*d, None, case.scale, 16, max_seqlen=40)
+    assert refused and torch.equal(out, plain)
