@@ -189,9 +189,14 @@ def paged_flash_attention_decode_noalloc(
     return out
 
 
-def _prefill_workspace(q, k_cache, block_tables, cu_seqlens, page):
+def _prefill_workspace(q, k_cache, v_cache, block_tables, cu_seqlens, page):
     """Workspace of the split paged prefill when these sizes run split, else
-    None: one workgroup per row, also where the memory is not to be had."""
+    None: one workgroup per row, also where the memory is not to be had.
+    Pages of a multiple of 16 keys only, with block strides below 4 GiB: the
+    launcher serves the others by a kernel that looks every row up and is not
+    split."""
+    if page % 16 or max(k_cache.stride(0), v_cache.stride(0)) * k_cache.element_size() >= 2**32:
+        return None
     n = _lib.workspace_size("paged_attention_prefill_workspace_size", q.shape[0], cu_seqlens.numel() - 1, q.shape[1],
                             k_cache.shape[2], q.shape[2], block_tables.shape[1] * page)
     if n <= 0:
@@ -229,7 +234,7 @@ def paged_flash_attention_prefill(
         max_seqlen = _max_seqlen(cu_seqlens)
     q, k_cache, v_cache = _lib.vec16(q), _lib.vec16(k_cache), _lib.vec16(v_cache)
     o = _out_for(out, (q.shape[0], q.shape[1], v_cache.shape[-1]), q.dtype, dev)
-    ws = _prefill_workspace(q, k_cache, page_block_tables, cu_seqlens, page_block_size)
+    ws = _prefill_workspace(q, k_cache, v_cache, page_block_tables, cu_seqlens, page_block_size)
     if ws is not None:
         _lib.call("paged_attention_prefill_split", q, k_cache, v_cache, page_block_tables, context_lens, cu_seqlens, o,
                   ws, int(max_seqlen), float(scale))

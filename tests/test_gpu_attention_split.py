@@ -8,6 +8,7 @@ import torch
 
 from conftest import assert_out_close
 from myvllm_amd import _lib, paged_flash_attention_prefill
+from myvllm_amd.full_attention import _prefill_workspace
 from myvllm_amd.workloads import paged_case
 from oracle.attention import paged_attention_ref
 
@@ -35,6 +36,23 @@ def test_split_rule():
     for T in (1, 100, 2000, 30000):
         for cap in (1 << 12, 1 << 20, 1 << 30):
             assert _lib.load().paged_attention_prefill_workspace_size(T, 3, 16, 2, 256, cap) * 4 <= 1 << 29
+
+
+def _on_host(page=16, block_stride=None):
+    """Tensors of a call that is split at pages of 16 (never read)."""
+    q = torch.empty(5, 4, 64, dtype=torch.bfloat16)
+    kc = torch.empty(1, page, 1, 64, dtype=torch.bfloat16)
+    if block_stride:
+        kc = kc.as_strided(kc.shape, (block_stride, *kc.stride()[1:]))
+    return q, kc, kc, torch.zeros(1, 4096 // page, dtype=torch.int32), torch.tensor([0, 5], dtype=torch.int32), page
+
+
+def test_workspace_only_where_the_kernel_splits():
+    """Pages that are no multiple of 16 and wide block strides take the per-row kernel: no workspace."""
+    assert _prefill_workspace(*_on_host()) is not None and _prefill_workspace(*_on_host(page=32)) is not None
+    assert _prefill_workspace(*_on_host(page=8)) is None and _prefill_workspace(*_on_host(page=24)) is None
+    assert _prefill_workspace(*_on_host(block_stride=2**31)) is None
+    assert _prefill_workspace(*_on_host(block_stride=2**31 - 8)) is not None
 
 
 @pytest.mark.gpu
