@@ -195,6 +195,8 @@ def _prefill_workspace(q, k_cache, v_cache, block_tables, cu_seqlens, page):
     Pages of a multiple of 16 keys only, with block strides below 4 GiB: the
     launcher serves the others by a kernel that looks every row up and is not
     split."""
+    if q.dim() != 3 or k_cache.dim() != 4 or v_cache.dim() != 4 or block_tables.dim() != 2 or cu_seqlens.dim() != 1:
+        return None  # (the entry refuses the call)
     if page % 16 or max(k_cache.stride(0), v_cache.stride(0)) * k_cache.element_size() >= 2**32:
         return None
     n = _lib.workspace_size("paged_attention_prefill_workspace_size", q.shape[0], cu_seqlens.numel() - 1, q.shape[1],

@@ -55,6 +55,25 @@ def test_workspace_only_where_the_kernel_splits():
     assert _prefill_workspace(*_on_host(block_stride=2**31 - 8)) is not None
 
 
+def test_wrong_ranks_are_left_to_the_entry():
+    q, kc, vc, tab, cu, page = _on_host()
+    for args in ((q[0], kc, vc, tab, cu), (q, kc[0], vc, tab, cu), (q, kc, vc[0], tab, cu), (q, kc, vc, tab[0], cu),
+                 (q, kc, vc, tab, cu[0])):
+        assert _prefill_workspace(*args, page) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bad", ["q", "tables", "cu"])
+def test_paged_prefill_wrong_rank(dev, bad):
+    """Refused by the entry's own error, as a wrong rank is everywhere else."""
+    case = paged_case([3000, 40], [5, 40], page=16, seed=3, Hq=16, Hkv=2, D=256)
+    d = dict(q=case.q, k=case.k_cache, v=case.v_cache, tables=case.block_tables, ctx=case.context_lens, cu=case.cu)
+    d[bad] = d[bad][0]
+    d = [t.to(dev) for t in d.values()]
+    with pytest.raises(_lib.GdnError, match="dimensions"):
+        paged_flash_attention_prefill(*d, None, case.scale, 16, max_seqlen=40)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize(
     "ctx, new, page, Hq, Hkv, Dh, dtype, tab64",
