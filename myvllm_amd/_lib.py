@@ -224,22 +224,21 @@ def check(fn: str, code: int) -> None:
         raise GdnError(fn, code, strerror(code))
 
 
-def vec16(t: torch.Tensor) -> torch.Tensor:
-    """t itself when the kernels can read it with 16-byte vector accesses (unit
-    inner stride, 16-byte aligned data and outer strides), else a contiguous
-    copy: the reference passes every stride to its kernels, so any strided
-    input is accepted, at the cost of a copy when it is misaligned."""
+def vec16_ok(t: torch.Tensor) -> bool:
+    """Whether the kernels can read t with 16-byte vector accesses: unit inner
+    stride, 16-byte aligned data and outer strides."""
     ok = (_fast or _load_fast()).vec16_ok(t)
     if ok is not None:
-        return t if ok else t.contiguous()
+        return ok
     es = t.element_size()
-    if t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all((t.stride(i) * es) % 16 == 0 for i in range(t.dim() - 1)):
-        return t
-    return t.contiguous()
+    return t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all((t.stride(i) * es) % 16 == 0 for i in range(t.dim() - 1))
 
 
-def vec16_ok(t: torch.Tensor) -> bool:
-    return vec16(t) is t
+def vec16(t: torch.Tensor) -> torch.Tensor:
+    """t itself when the kernels can read it with 16-byte vector accesses, else a
+    contiguous copy: the reference passes every stride to its kernels, so any
+    strided input is accepted, at the cost of a copy when it is misaligned."""
+    return t if vec16_ok(t) else t.contiguous()
 
 
 def same_device(*tensors: torch.Tensor) -> bool:

@@ -7,7 +7,7 @@ import torch
 
 from conftest import assert_out_close, assert_state_close
 from myvllm_amd import _lib, gated_delta_net_decode_step
-from myvllm_amd.layer import _own_linear
+from myvllm_amd.layer import _linear, _own_linear
 from myvllm_amd.norm import rms_norm_gated
 
 
@@ -15,6 +15,16 @@ def test_own_linear_rule():
     assert _own_linear(1, 12352, 2048) and _own_linear(7, 12352, 2048) and not _own_linear(8, 12352, 2048)
     assert _own_linear(16, 2048, 4096) and not _own_linear(17, 64, 256) and not _own_linear(0, 64, 256)
     assert not _own_linear(1, 64, 128) and not _own_linear(1, 62, 256) and not _own_linear(1, 64, 0)
+
+
+def test_misaligned_operands_are_not_copied(monkeypatch):
+    """A weight the kernel cannot read goes to torch's product as it lies: the test of its alignment copies nothing."""
+    x = torch.ones(1, 256, dtype=torch.bfloat16)
+    w = torch.ones(64 * 256 + 1, dtype=torch.bfloat16)[1:].view(64, 256)
+    assert w.data_ptr() % 16 and _own_linear(1, 64, 256)
+    monkeypatch.setattr(torch.Tensor, "contiguous", lambda *a, **kw: pytest.fail("copied"))
+    assert not _lib.vec16_ok(w) and not _lib.vec16_ok(x.t()) and _lib.vec16_ok(x)
+    assert (_linear(x, w) == 256).all()
 
 
 @pytest.mark.parametrize(
