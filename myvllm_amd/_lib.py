@@ -236,9 +236,10 @@ def vec16_ok(t: torch.Tensor) -> bool:
 
 def vec16(t: torch.Tensor) -> torch.Tensor:
     """t itself when the kernels can read it with 16-byte vector accesses, else a
-    contiguous copy: the reference passes every stride to its kernels, so any
-    strided input is accepted, at the cost of a copy when it is misaligned."""
-    return t if vec16_ok(t) else t.contiguous()
+    contiguous copy (also of a contiguous one at a misaligned address): the
+    reference passes every stride to its kernels, so any strided input is
+    accepted, at the cost of a copy when it is misaligned."""
+    return t if vec16_ok(t) else t.clone(memory_format=torch.contiguous_format)
 
 
 def same_device(*tensors: torch.Tensor) -> bool:

@@ -63,6 +63,27 @@ def test_any_head_dim(dev, Dh, Hq, Hkv, causal, dtype):
     assert err < 5e-3, f"relative error norm {err:.3e}"
 
 
+def test_misaligned_contiguous_input_is_copied():
+    t = torch.arange(2 * 3 * 8 + 1, dtype=torch.bfloat16)[1:].view(2, 3, 8)
+    assert t.is_contiguous() and t.data_ptr() % 16
+    c = _lib.vec16(t)
+    assert c.data_ptr() % 16 == 0 and torch.equal(c, t)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Dh", [72, 64])
+def test_misaligned_contiguous_rows(dev, Dh):
+    """q, k and v contiguous at odd addresses, as views of one flat buffer."""
+    case = attn_varlen_case([40, 33], seed=Dh, Hq=4, Hkv=4, D=Dh)
+    buf = torch.empty(3 * case.q.numel() + 1, dtype=case.q.dtype, device=dev)
+    q, k, v = (buf[1 + i * case.q.numel():][: case.q.numel()].view(case.q.shape).copy_(t)
+               for i, t in enumerate((case.q, case.k, case.v)))
+    assert q.is_contiguous() and q.data_ptr() % 16
+    print(f"misaligned contiguous rows D={Dh}", flush=True)
+    got = flash_attention_prefill(q, k, v, case.cu.to(dev), case.scale, 4, 4, Dh, Dh, True)
+    assert_out_close(got, flash_attention_prefill_ref(case.q, case.k, case.v, case.cu, case.scale))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("N", [1, 63, 64, 65])  # ranked by length up to 64 sequences, in index order past that
 @pytest.mark.parametrize("Dh", [64, 72, 128])
