@@ -75,7 +75,7 @@ def flash_attention_prefill(
     if not own and not _direct_head_dim(q, k, v, head_dim, head_v_dim, max_seqlen):
         return _padded_prefill(q, k, v, cu_seqlens, scale, head_dim, head_v_dim, is_causal, max_seqlen, out)
     q, k, v = _lib.vec16(q), _lib.vec16(k), _lib.vec16(v)
-    o = _out_for(out, (q.shape[0], q.shape[1], head_v_dim), q.dtype, dev)
+    o = _out_for(out if own or _apart(out, q, k, v) else None, (q.shape[0], q.shape[1], head_v_dim), q.dtype, dev)
     _lib.call("flash_attention_varlen" if own else "flash_attention_varlen_any_dim", q, k, v, cu_seqlens, o,
               int(max_seqlen), float(scale), int(bool(is_causal)))
     return _finish(out, o)
@@ -96,6 +96,14 @@ def _direct_head_dim(q, k, v, head_dim, head_v_dim, max_seqlen) -> bool:
         return False
     st = max(k.stride(0), v.stride(0), k.shape[1] * head_dim)
     return min(k.stride(0), v.stride(0)) >= head_dim and max(max_seqlen, 64) * st * q.element_size() < 2**31
+
+
+def _apart(out, q, k, v) -> bool:
+    """Whether a result of q's shape can go to `out` directly: of the same shape,
+    dtype and device and in memory of its own.  The padded path copies its result
+    into whatever `out` is, one of the inputs among them."""
+    return (out is not None and out.shape == q.shape and out.dtype == q.dtype and out.device == q.device
+            and out.untyped_storage().data_ptr() not in {t.untyped_storage().data_ptr() for t in (q, k, v)})
 
 
 def _padded_prefill(q, k, v, cu_seqlens, scale, head_dim, head_v_dim, is_causal, max_seqlen, out):

@@ -85,6 +85,24 @@ def test_misaligned_contiguous_rows(dev, Dh):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["fp32", "host", "q", "k", "v", "shifted"])
+def test_out_of_any_kind(dev, kind):
+    """An out of another dtype or device, or in an input's memory, takes a copy of the result, as it
+    does where the head dim is padded."""
+    case = attn_varlen_case([200, 65], seed=9, Hq=4, Hkv=4, D=72)
+    q, k, v = (t.to(dev) for t in (case.q, case.k, case.v))
+    want = flash_attention_prefill(q, k, v, case.cu.to(dev), case.scale, 4, 4, 72, 72, True)
+    buf = torch.empty(k.numel() + 8 * 72, dtype=k.dtype, device=dev)
+    if kind == "shifted":
+        k = buf[8 * 72:].view(k.shape).copy_(k)
+    out = {"fp32": torch.empty_like(q, dtype=torch.float32), "host": torch.empty_like(case.q), "q": q, "k": k, "v": v,
+           "shifted": buf[: k.numel()].view(k.shape)}[kind]
+    print(f"attention out {kind}", flush=True)
+    got = flash_attention_prefill(q, k, v, case.cu.to(dev), case.scale, 4, 4, 72, 72, True, out=out)
+    assert got is out and torch.equal(got.to(want.device, want.dtype), want)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("N", [1, 63, 64, 65])  # ranked by length up to 64 sequences, in index order past that
 @pytest.mark.parametrize("Dh", [64, 72, 128])
 def test_sequence_order(dev, N, Dh):
