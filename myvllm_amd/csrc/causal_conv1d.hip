@@ -186,15 +186,16 @@ GDN_DEVICE void conv_tile(const ConvArgs& a, int64_t seq, int64_t tile, int64_t 
   }
 }
 
-// One workgroup per (tile, channel block); blockIdx.x is the linear tile id.
+// One workgroup per (tile, channel block); blockIdx.z and .x are the linear tile id.
 template <typename TX, typename TW, typename TS, int W>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(W <= 4 && sizeof(TX) == 2 ? 4 : 1)))
 void causal_conv1d_varlen_kernel(ConvArgs a) {
   __shared__ int32_t lds[8];
   // output rows no sequence covers are zero, as the reference allocates y
   // zero-filled (ops/causal_conv1d.py:241)
+  const int64_t id = (int64_t)blockIdx.z * gridDim.x + blockIdx.x;
   zero_uncovered_rows<(int)sizeof(TX)>(a.out, a.o_s0, 0, 1, a.D, a.cu, a.cu64, a.nseq, a.T,
-                                       (int64_t)blockIdx.x * gridDim.y + blockIdx.y, (int64_t)gridDim.x * gridDim.y,
+                                       id * gridDim.y + blockIdx.y, (int64_t)gridDim.x * gridDim.y * gridDim.z,
                                        threadIdx.x, kThreads);
   const int64_t d0 = ((int64_t)blockIdx.y * kThreads + threadIdx.x) * kCh;
   const bool active = d0 < a.D;
@@ -205,7 +206,7 @@ void causal_conv1d_varlen_kernel(ConvArgs a) {
     scale_taps(wr, W);
   }
   int64_t seq, tile;
-  find_seq_tile<kThreads>(a.cu, a.cu64, a.nseq, a.T, kTile, blockIdx.x, seq, tile, lds);
+  find_seq_tile<kThreads>(a.cu, a.cu64, a.nseq, a.T, kTile, id, seq, tile, lds);
   if (seq < 0 || !active) return;
   conv_tile<TX, TS, W>(a, seq, tile, d0, wr);
 }
@@ -295,14 +296,20 @@ hipError_t launch_conv(bool varlen, const gdn_tensor* x, const gdn_tensor* w, gd
   a.cu64 = cu && cu->dtype == GDN_DTYPE_I64;
   const int W = (int)w->shape[1];
   const int64_t ch_blocks = (a.D / kCh + kThreads - 1) / kThreads;
-  int64_t gx;
+  int64_t gx, gz = 1;
   if (varlen) {
     gx = (a.T + kTile - 1) / kTile + a.nseq;  // upper bound on the number of tiles
+    // a grid's x has fewer than 2^32 threads: 2^24 workgroups, 400 million tokens
+    constexpr int64_t kMaxX = int64_t(1) << 23;
+    if (gx > kMaxX) {
+      gz = (gx + kMaxX - 1) / kMaxX;
+      gx = kMaxX;
+    }
   } else {
     gx = a.T;
   }
   if (gx == 0 || ch_blocks == 0) return hipSuccess;
-  dim3 grid((unsigned)gx, (unsigned)ch_blocks);
+  dim3 grid((unsigned)gx, (unsigned)ch_blocks, (unsigned)gz);
   switch (x->dtype) {
     case GDN_DTYPE_BF16: return launch_weight<bf16_t>(varlen, a, w->dtype, cs->dtype, W, grid, st);
     case GDN_DTYPE_F16: return launch_weight<f16_t>(varlen, a, w->dtype, cs->dtype, W, grid, st);

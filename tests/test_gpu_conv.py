@@ -106,3 +106,28 @@ def test_conv_tile_edges(dev, W):
     y, st, y_ref, st_ref = _prefill(case, dev)
     assert_out_close(y, y_ref)
     assert torch.equal(st, st_ref)
+
+
+def test_conv_more_tiles_than_a_grid_axis(dev):
+    """402.7 million tokens of 8 channels: more 24-token tiles than the 2^24 workgroups of one grid
+    axis.  Rows are zero but for 100 at both ends and where the tile ids pass to the grid's next layer."""
+    T = 24 * 2**24 + 40
+    print(f"conv of {T} tokens", flush=True)
+    case = conv_prefill_case([100], seed=4, D=8, num_slots=2)
+    case.x.mul_(50)
+    case.weight.mul_(50)
+    x = torch.zeros(T, 8, dtype=case.x.dtype, device=dev)
+    at = [0, 24 * 2**23 - 50, T - 100]
+    for a in at:
+        x[a: a + 100] = case.x.to(dev)
+    st = case.state.to(dev)
+    cu = torch.tensor([0, T], dtype=torch.int32, device=dev)
+    y = causal_conv1d_fn(x, case.weight.to(dev), st, case.idx.to(dev), cu)
+    torch.cuda.synchronize()
+    for a in at:
+        st_ref = case.state.clone() if a == 0 else torch.zeros_like(case.state)
+        ref = causal_conv1d_fn_ref(case.x, case.weight, st_ref, case.idx, case.cu)
+        assert ref.float().abs().max() > 1
+        assert_out_close(y[a: a + 100], ref)
+    assert torch.equal(st.cpu()[case.idx.long()], st_ref[case.idx.long()])
+    assert not y[200: at[1] - 10].any()
