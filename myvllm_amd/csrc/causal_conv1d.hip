@@ -205,8 +205,15 @@ void causal_conv1d_varlen_kernel(ConvArgs a) {
     load_weights<TW, W>(a, d0, wr);
     scale_taps(wr, W);
   }
+  // Workgroups are dealt to the eight XCDs in turn: of 64 ids in a row each XCD
+  // takes eight tiles in a row, so that the W - 1 rows a tile reads of the one
+  // before it are in that XCD's L2.  In id order every tile read them from
+  // memory again: 64 prompts of 128 tokens 54 -> 51 us (tiles of 64 tokens
+  // 51), 64 of 192 75 -> 71 (73), 256 of 128 222 -> 212 (217).
+  const int64_t all = (int64_t)gridDim.x * gridDim.z, group = id & ~int64_t(63);
+  const int64_t target = group + 64 <= all ? group | (id & 7) << 3 | (id >> 3 & 7) : id;
   int64_t seq, tile;
-  find_seq_tile<kThreads>(a.cu, a.cu64, a.nseq, a.T, kTile, id, seq, tile, lds);
+  find_seq_tile<kThreads>(a.cu, a.cu64, a.nseq, a.T, kTile, target, seq, tile, lds);
   if (seq < 0 || !active) return;
   conv_tile<TX, TS, W>(a, seq, tile, d0, wr);
 }

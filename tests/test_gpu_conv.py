@@ -108,6 +108,19 @@ def test_conv_tile_edges(dev, W):
     assert torch.equal(st, st_ref)
 
 
+@pytest.mark.parametrize("lengths", [[24 * 62 + 1], [24 * 63], [24 * 127 - 3, 24, 1], [700, 0, 333, 24 * 40]])
+def test_conv_tile_order(dev, lengths):
+    """Grids of 63 tiles and more, whole and broken groups of 64: every row once, against the oracle
+    at unit scale (one bf16 rounding of y)."""
+    case = conv_prefill_case(lengths, seed=len(lengths), D=16, num_slots=6)
+    case.x.mul_(50)
+    case.weight.mul_(25)
+    y, st, y_ref, st_ref = _prefill(case, dev)
+    err = (y.double() - y_ref.double()).norm() / y_ref.double().norm()
+    assert err < 2**-8, err
+    assert torch.equal(st, st_ref)
+
+
 def test_conv_more_tiles_than_a_grid_axis(dev):
     """402.7 million tokens of 8 channels: more 24-token tiles than the 2^24 workgroups of one grid
     axis.  Rows are zero but for 100 at both ends and where the tile ids pass to the grid's next layer."""
