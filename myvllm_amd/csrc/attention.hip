@@ -167,7 +167,9 @@ GDN_DEVICE const char* kv_row(const KvSource& s, const PagedTable& tb, int64_t n
 // workgroup of a padded grid exits idle).  Below D = 256 batches of up to 64
 // sequences go longest first (by keys, ties by index), so that what runs last
 // is short: every lane ranks one sequence against the others and sums the
-// tiles before it, with no barrier.  Six images of 450 to 2,900 patches 143 ->
+// tiles before it, past eight sequences a quarter of them per wave (a wave
+// against all 64 took 10 us of a call: 64 x 100 tokens at D = 64 28.8 us, 18.3
+// shared, in index order 17.1).  Six images of 450 to 2,900 patches 143 ->
 // 137 us, eight causal prompts of 512 to 4,096 tokens 171 -> 159 (D = 64) and
 // 259 -> 247 (128), eight chunks over up to 4,096 cached keys 340 -> 331 (128).
 // Past the last tile seq is -1 and tile counts from there.
@@ -180,24 +182,34 @@ template <int D, bool PAGED>
 GDN_DEVICE SeqTile attn_tile_lookup(const AttnArgs& a, int tile_len, int64_t target, int32_t* lds) {
   SeqTile r;
   if (D < 256 && a.nseq <= 64) {
-    const int lane = threadIdx.x & 63, sh = __builtin_ctz(tile_len);
-    int nt = 0, key = 0;
+    __shared__ int32_t before[4][64];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), sh = __builtin_ctz(tile_len);
+    int nt = 0;
+    uint32_t key = 0;
     if (lane < a.nseq) {
       int64_t s, e;
       seq_range(a.cu, a.cu64, lane, a.T, s, e);
       nt = (int)((e - s + tile_len - 1) >> sh);
-      key = PAGED ? (int)clamp64(load_index(a.ctx, lane, a.ctx64), 0, 0x7fffffff) : (int)(e - s);
+      key = (uint32_t)clamp64(PAGED ? load_index(a.ctx, lane, a.ctx64) : e - s, 0, (1 << 26) - 1);
     }
-    int base = 0, total = 0;
-    for (int j = 0; j < (int)a.nseq; ++j) {
-      const int kj = __builtin_amdgcn_readlane(key, j), tj = __builtin_amdgcn_readlane(nt, j);
-      base += kj > key || (kj == key && j < lane) ? tj : 0;
-      total += tj;
+    key = key << 6 | (63 - lane);  // (unique, so one comparison ranks)
+    const bool share = a.nseq > 8;  // each wave against a quarter of the sequences
+    int base = 0;
+    for (int j = share ? w : 0; j < (int)a.nseq; j += share ? 4 : 1) {
+      const uint32_t kj = (uint32_t)__builtin_amdgcn_readlane((int)key, j);
+      const int tj = __builtin_amdgcn_readlane(nt, j);
+      base += kj > key ? tj : 0;
+    }
+    if (share) {
+      before[w][lane] = base;
+      __syncthreads();
+      base = before[0][lane] + before[1][lane] + before[2][lane] + before[3][lane];
     }
     const int t = (int)target - base;
     const uint64_t own = __builtin_amdgcn_ballot_w64(t >= 0 && t < nt);
     r.seq = own ? __builtin_ctzll(own) : -1;
-    r.tile = own ? __builtin_amdgcn_readlane(t, (int)r.seq) : target - total;
+    r.tile = own ? __builtin_amdgcn_readlane(t, (int)r.seq)
+                 : target - __builtin_amdgcn_readlane(wave_inclusive_scan_i32(nt), 63);
     return r;
   }
   find_seq_tile<256>(a.cu, a.cu64, a.nseq, a.T, tile_len, target, r.seq, r.tile, lds);

@@ -103,7 +103,8 @@ def test_out_of_any_kind(dev, kind):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("N", [1, 63, 64, 65])  # ranked by length up to 64 sequences, in index order past that
+# (ranked by length up to 64 sequences, past eight of them a quarter per wave; in index order past 64)
+@pytest.mark.parametrize("N", [1, 7, 8, 9, 10, 63, 64, 65])
 @pytest.mark.parametrize("Dh", [64, 72, 128])
 def test_sequence_order(dev, N, Dh):
     """Ragged batches with empty and equal sequences on both sides of the ranking's limit."""
