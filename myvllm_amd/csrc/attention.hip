@@ -250,7 +250,8 @@ GDN_DEVICE void zero_rows_tail(const AttnArgs& a, uint32_t wg, uint32_t n) {
 // 47 us, five of 18 over 11,700 301 -> 64 us.
 //
 // Key tiles: 32 keys, which at D = 64 and 128 leave room for two waves per
-// SIMD (at least) whose softmax and MFMAs overlap; D = 96 fits two with 64.
+// SIMD (at least) whose softmax and MFMAs overlap; D = 96 fits two with 64, and
+// at D = 64 few workgroups take 64 (few_workgroups).
 // At D = 128 tiles of 64 keys took 259 to 280 registers, one wave per SIMD:
 // eight prompts of 512 to 4,096 tokens (16 / 4 heads) 363 -> 254 us, with 64
 // keys held to 256 registers 259; eight chunks over up to 4,096 cached keys
@@ -1356,11 +1357,29 @@ hipError_t launch_prefill_t(const AttnArgs& a, int64_t nseq, int64_t max_len, hi
   return hipGetLastError();
 }
 
+// Whether packed rows at D = 64 take key tiles of 64 keys rather than 32: 180
+// registers and two workgroups a CU against 128 and four, with half the
+// barriers per key.  They win while fewer than three workgroups a CU are there
+// to run (causal ones are uneven, so a few more), 32 keys with more, or where
+// no sequence is longer than a few tiles.  16 heads, us at 64 / 32 keys: causal
+// 1 x 1,024 17.6 / 20.8, 1 x 4,096 58 / 67, 3,000 and 2,500 50 / 56, 4 x 1,500
+// 45 / 39, 16 x 256 14.7 / 13.6, eight of 512 to 4,096 152 / 139;
+// bidirectional 3,000 and 12 x 50 60 / 66, 3,000 and 2,500 88 / 83, 16 x 200
+// 12.8 / 12.2.
+bool few_workgroups(const AttnArgs& a, int64_t nseq, int64_t max_len) {
+  return max_len > 256 && (a.T / (32 * (4 / a.gh)) + nseq) * (a.Hq / a.gh) <= (a.causal ? 736 : 672);
+}
+template <typename T, int DQ>
+hipError_t launch_prefill_64(const AttnArgs& a, int64_t nseq, int64_t max_len, hipStream_t st) {
+  return few_workgroups(a, nseq, max_len) ? launch_prefill_t<T, 64, 64, false, DQ>(a, nseq, max_len, st)
+                                          : launch_prefill_t<T, 64, 32, false, DQ>(a, nseq, max_len, st);
+}
+
 // Packed rows of any head dim that is a multiple of 8 up to 256: the next
 // larger tile (the score product in steps of 16 dims, P V in steps of 32).
 template <typename T>
 hipError_t launch_prefill_ragged(const AttnArgs& a, int64_t nseq, int64_t max_len, hipStream_t st) {
-  if (a.dim <= 64) return launch_prefill_t<T, 64, 32, false, 64>(a, nseq, max_len, st);
+  if (a.dim <= 64) return launch_prefill_64<T, 64>(a, nseq, max_len, st);
   if (a.dim <= 80) return launch_prefill_t<T, 96, 64, false, 80>(a, nseq, max_len, st);
   if (a.dim <= 96) return launch_prefill_t<T, 96, 64, false, 96>(a, nseq, max_len, st);
   if (a.dim <= 128) return launch_prefill_t<T, 128, 32, false, 128>(a, nseq, max_len, st);
@@ -1373,6 +1392,9 @@ hipError_t launch_prefill(const AttnArgs& a, int dtype, int D, int64_t nseq, int
     if (D != 64 && D != 128 && D != 256)
       return dtype == GDN_DTYPE_BF16 ? launch_prefill_ragged<bf16_t>(a, nseq, max_len, st)
                                      : launch_prefill_ragged<f16_t>(a, nseq, max_len, st);
+    if (D == 64)
+      return dtype == GDN_DTYPE_BF16 ? launch_prefill_64<bf16_t, 0>(a, nseq, max_len, st)
+                                     : launch_prefill_64<f16_t, 0>(a, nseq, max_len, st);
   }
   if (dtype == GDN_DTYPE_BF16) {
     if (D == 64) return launch_prefill_t<bf16_t, 64, 32, PAGED>(a, nseq, max_len, st);

@@ -118,6 +118,28 @@ def test_sequence_order(dev, N, Dh):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("Dh", [64, 40])
+@pytest.mark.parametrize(
+    "lengths, causal",
+    [
+        ([257], True), ([256], True),  # 64-key tiles from 257 tokens on
+        ([639], True), ([640], True),  # 640 and 768 workgroups: 64 and 32 keys
+        ([639], False), ([640], False),
+        ([300, 65, 1], True), ([300, 127, 0, 33], False),
+    ],
+)
+def test_key_tiles_of_few_workgroups(dev, Dh, lengths, causal):
+    case = attn_varlen_case(lengths, seed=Dh, Hq=128, Hkv=128, D=Dh)
+    print(f"few workgroups D={Dh} {lengths} causal={causal}", flush=True)
+    got = flash_attention_prefill(case.q.to(dev), case.k.to(dev), case.v.to(dev), case.cu.to(dev), case.scale, 128, 128,
+                                  Dh, Dh, causal)
+    ref = flash_attention_prefill_ref(case.q, case.k, case.v, case.cu, case.scale, is_causal=causal)
+    assert_out_close(got, ref)
+    err = (got.double().cpu() - ref.double()).norm() / ref.double().norm()
+    assert err < 5e-3, f"relative error norm {err:.3e}"
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("Dh, N", [(256, 3), (72, 3), (128, 70), (64, 1)])
 @pytest.mark.parametrize("first, tail", [(0, 1), (5, 0), (7, 900)])
 def test_uncovered_rows_are_zero(dev, Dh, N, first, tail):
