@@ -351,10 +351,11 @@ int paged_attention_prefill(const gdn_tensor* q, const gdn_tensor* k_cache, cons
 /*
  * paged_attention_prefill with a workspace, in which rows (32 queries of up
  * to four heads) over long contexts are cut into pieces of keys that run as
- * workgroups of their own and are merged by a second launch.  Whether and how
- * far follows from the sizes alone; paged_attention_prefill_workspace_size is
- * the fp32 elements that the choice needs, 0 when nothing is split (max_keys =
- * max_blocks * page).  workspace: 1-D fp32, 16-byte aligned, overwritten.
+ * workgroups of their own and are merged by a second launch.  Whether a batch
+ * may be cut follows from the sizes: paged_attention_prefill_workspace_size is
+ * the fp32 elements that takes, 0 when nothing is split (max_keys = max_blocks
+ * * page).  How far it is follows from the lengths, on the device.  workspace:
+ * 1-D fp32, 16-byte aligned, overwritten.
  */
 int64_t paged_attention_prefill_workspace_size(int64_t num_tokens, int64_t num_seqs, int64_t num_q_heads,
                                                int64_t num_kv_heads, int64_t head_dim, int64_t max_keys);

@@ -116,10 +116,10 @@ struct AttnArgs {
   int32_t dim;          // head dim (a multiple of 8, at most the kernel's D)
   float c;              // softmax scale * log2(e)
   bool cu64, ctx64, causal;
-  // split prefill: key tiles of a piece (even), (tile, head group) rows of the
-  // grid, and the pieces' partials (slot row * splits + piece)
-  int32_t piece_tiles, splits;
+  // split prefill: (tile, head group) rows of the grid, workgroups for the
+  // rows' further pieces, and the pieces' partials (rows + extra slots)
   int64_t rows;
+  int32_t extra;
   float* part;
 };
 
@@ -178,7 +178,7 @@ GDN_DEVICE const char* kv_row(const KvSource& s, const PagedTable& tb, int64_t n
 struct SeqTile {
   int64_t seq, tile;
 };
-template <int D, bool PAGED>
+template <int D, bool PAGED, bool SPLIT>
 GDN_DEVICE SeqTile attn_tile_lookup(const AttnArgs& a, int tile_len, int64_t target, int32_t* lds) {
   SeqTile r;
   if (D < 256 && a.nseq <= 64) {
@@ -212,8 +212,190 @@ GDN_DEVICE SeqTile attn_tile_lookup(const AttnArgs& a, int tile_len, int64_t tar
                  : target - __builtin_amdgcn_readlane(wave_inclusive_scan_i32(nt), 63);
     return r;
   }
+  if (SPLIT && a.nseq <= 64) {  // index order without a barrier: split_tiles has just read the same lengths
+    const int lane = threadIdx.x & 63;
+    int nt = 0;
+    if (lane < a.nseq) {
+      int64_t s, e;
+      seq_range(a.cu, a.cu64, lane, a.T, s, e);
+      nt = (int)((e - s + tile_len - 1) >> __builtin_ctz(tile_len));
+    }
+    const int incl = wave_inclusive_scan_i32(nt), t = (int)target - (incl - nt);
+    const uint64_t own = __builtin_amdgcn_ballot_w64(t >= 0 && t < nt);
+    r.seq = own ? __builtin_ctzll(own) : -1;
+    r.tile = own ? __builtin_amdgcn_readlane(t, (int)r.seq) : target - __builtin_amdgcn_readlane(incl, 63);
+    return r;
+  }
   find_seq_tile<256>(a.cu, a.cu64, a.nseq, a.T, tile_len, target, r.seq, r.tile, lds);
   return r;
+}
+
+// How a split prefill cuts its rows: into pieces of `tiles` key tiles, the same
+// for all rows.  A row's first piece has the row's own workgroup; the further
+// ones take floor((n - 1) / tiles) of the extra workgroups per query tile and
+// head group of a sequence, n the key tiles of its last query (its other rows
+// may need fewer: those left over return).  All second pieces come first, then
+// all third ones, so that what runs together reads the same stretch of K and V
+// and the rows' short ends run last.
+// The length follows from the batch's own lengths.  Lane i prices the longest
+// row in i + 1 pieces, in key-tile steps of one workgroup (1.18 us at D = 256,
+// 1.05 at 128): the batch's work over the workgroups that run at once, with
+// kFixed steps per row (lookup, queries, pipeline fill, output) and kPiece per
+// further piece (that, and its share of the merge), and part of the length of
+// those that start last; a batch that fits one round takes as long as its
+// longest workgroup.  Fitted to 29 batches forced into 1 to 16 pieces: what it
+// chooses is 1 % off the best on average, 8 % at most.  A split has to win a
+// sixteenth over one piece per row and to fit the extra workgroups.  The
+// prefill and the combine kernel both work it out, in whole numbers, so that
+// they agree.
+struct SplitSeq {
+  int32_t ntile, n;  // query tiles, key tiles of the last one
+};
+struct SplitPlan {
+  int32_t tiles;  // kWholeRows: not split
+  SplitSeq q;     // sequence `lane` of the first 64; the others are read again
+};
+constexpr int kWholeRows = 1 << 26;  // (32 keys times that: past any row)
+constexpr int kMaxPieces = 64;
+template <int BN>
+GDN_DEVICE SplitSeq split_seq(const AttnArgs& a, int64_t seq, int sh) {
+  SplitSeq q{0, 0};
+  if (seq < a.nseq) {
+    int64_t s, e;
+    seq_range(a.cu, a.cu64, seq, a.T, s, e);
+    const int64_t keys = clamp64(load_index(a.ctx, seq, a.ctx64), 0, a.tab.cols * a.tab.page);
+    q.ntile = (int)((e - s + (1 << sh) - 1) >> sh);
+    q.n = q.ntile > 0 ? (int)((keys + BN - 1) / BN) : 0;
+  }
+  return q;
+}
+template <int BN>
+GDN_DEVICE SplitSeq split_seq(const AttnArgs& a, const SplitPlan& sp, int c, int sh) {
+  return c == 0 ? sp.q : split_seq<BN>(a, c + (threadIdx.x & 63), sh);
+}
+// floor((n - 1) / tiles), at most some 64: the float quotient is within one of it
+GDN_DEVICE int split_further(int n, int tiles, float inv) {
+  const int last = n > 0 ? n - 1 : 0;
+  int u = (int)((float)last * inv);
+  u -= u * tiles > last;
+  return u + ((u + 1) * tiles <= last);
+}
+GDN_DEVICE int wave_top(int x) {  // maximum of non-negative numbers, in the steps of wave_inclusive_scan_i32
+  auto up = [&](int y) __attribute__((always_inline)) { x = y > x ? y : x; };
+  up(__builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false));
+  up(__builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false));
+  up(__builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false));
+  up(__builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false));
+  up(__builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false));
+  up(__builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false));
+  return __builtin_amdgcn_readlane(x, 63);
+}
+GDN_DEVICE int wave_sum(int x) { return __builtin_amdgcn_readlane(wave_inclusive_scan_i32(x), 63); }
+
+template <int D, int BN>
+GDN_DEVICE int split_tiles(const AttnArgs& a, const SplitPlan& sp, int sh) {
+  constexpr int kSlots = D == 256 ? 256 : D == 128 ? 512 : 768, kSlots16 = kSlots / 16;  // workgroups that run at once
+  constexpr int kFixed = 10, kPiece = D == 256 ? 18 : 16;
+  const int lane = threadIdx.x & 63, hg = a.Hq / a.gh, nseq = (int)a.nseq;
+  // per head group: query tiles R, work W in units of 16 steps, and what one
+  // piece per row takes: the longest (last, these run first) query tile of each
+  // sequence starts when the sequences before it have been handed out.  Below
+  // D = 256 they are ranked (attn_tile_lookup), so the longest starts first and
+  // the shortest last.
+  int W = 0, R = 0, top = 0, late = 0, low = kWholeRows;
+  for (int c = 0; c < nseq; c += 64) {
+    const SplitSeq q = split_seq<BN>(a, sp, c, sh);
+    // (the query tiles before the last see 2^sh keys less each)
+    const int less = ((q.ntile - 1) << (sh - 5)) / (2 * BN / 32), half = (q.n + 1) >> 1;
+    const float w16 = (float)q.ntile * (float)(kFixed + (q.n - less > half ? q.n - less : half)) * 0.0625f;
+    const int w = w16 < 0x1p22f ? (int)w16 : 1 << 22, incl = wave_inclusive_scan_i32(w);
+    const int end = ((W + incl - w) / kSlots16) * hg + q.n;
+    late = q.n > 0 && end > late ? end : late;
+    low = q.n > 0 && q.n < low ? q.n : low;
+    top = q.n > top ? q.n : top;
+    W += __builtin_amdgcn_readlane(incl, 63);
+    R += wave_sum(q.ntile);
+    if ((int64_t)W * hg > (1 << 28) || (int64_t)R * hg > (1 << 20)) return kWholeRows;  // (past the sums below)
+  }
+  const int nmax = wave_top(top);
+  if (nmax <= 16) return kWholeRows;
+  const int rows = hg * R, work = hg * W;
+  int whole = kFixed + nmax;
+  if (rows > kSlots) {
+    const int last = D == 256 ? kFixed + wave_top(late < 1 << 24 ? late : 1 << 24) : (work / kSlots16) + kWholeRows - wave_top(kWholeRows - low);
+    whole = last > whole ? last : whole;
+  }
+  int tiles = (int)((float)(nmax + lane) * __builtin_amdgcn_rcpf((float)(lane + 1)));
+  tiles += tiles * (lane + 1) < nmax;
+  tiles += tiles & 1;
+  const float inv = __builtin_amdgcn_rcpf((float)tiles);
+  int x = 0;
+  for (int c = 0; c < nseq; c += 64) {
+    const SplitSeq q = split_seq<BN>(a, sp, c, sh);
+    const int m = nseq - c < 64 ? nseq - c : 64;
+    for (int j = 0; j < m; ++j)
+      x += __mul24(__builtin_amdgcn_readlane(q.ntile, j), split_further(__builtin_amdgcn_readlane(q.n, j), tiles, inv));
+  }
+  x = x < 1 << 16 ? x * hg : 1 << 24;
+  const int split = rows + x <= kSlots
+                        ? kFixed + 4 + tiles + ((rows + x) / kSlots16)
+                        : ((work + kPiece * x / 16) / kSlots16) + (D == 256 ? tiles / 2 + tiles / 8 : tiles / 2) + kFixed;
+  int cost = lane == 0 ? whole - whole / 16 : x > 0 && x <= a.extra && tiles >= 8 ? split : 1 << 24;
+  cost = cost < 1 << 24 ? cost : 1 << 24;
+  // (the smallest, of equals the one with fewer pieces)
+  const int best = 63 - (wave_top(((1 << 24) - cost) << 6 | (63 - lane)) & 63);
+  return best > 0 ? __builtin_amdgcn_readlane(tiles, best) : kWholeRows;
+}
+
+// Further pieces of index p = lane (1, 2, ...; lane 0: 0) per head group, of
+// all sequences and of those before `seq`.
+struct SplitCount {
+  int32_t all, before;
+};
+template <int BN>
+GDN_DEVICE SplitCount split_count(const AttnArgs& a, const SplitPlan& sp, int sh, int seq) {
+  const int lane = threadIdx.x & 63, nseq = (int)a.nseq;
+  const float inv = __builtin_amdgcn_rcpf((float)sp.tiles);
+  SplitCount k{0, 0};
+  for (int c = 0; c < nseq; c += 64) {
+    const SplitSeq q = split_seq<BN>(a, sp, c, sh);
+    const int f = split_further(q.n, sp.tiles, inv), m = nseq - c < 64 ? nseq - c : 64;
+    for (int j = 0; j < m; ++j) {
+      const int fj = __builtin_amdgcn_readlane(f, j), nt = __builtin_amdgcn_readlane(q.ntile, j);
+      const int x = fj >= lane && lane > 0 ? nt : 0;
+      k.all += x;
+      k.before += c + j < seq ? x : 0;
+    }
+  }
+  return k;
+}
+
+// Of extra workgroup group `target` (per head group): its sequence, query tile
+// and piece; seq -1 if it is left over.
+struct SplitPiece {
+  int64_t seq, tile;
+  int piece;
+};
+template <int BN>
+GDN_DEVICE SplitPiece split_piece(const AttnArgs& a, const SplitPlan& sp, int sh, int target) {
+  const int nseq = (int)a.nseq;
+  const int all = split_count<BN>(a, sp, sh, 0).all, incl = wave_inclusive_scan_i32(all), t = target - (incl - all);
+  const uint64_t own = __builtin_amdgcn_ballot_w64(t >= 0 && t < all);
+  if (own == 0) return {-1, 0, 0};
+  const int p = __builtin_ctzll(own);
+  int left = __builtin_amdgcn_readlane(t, p);
+  const float inv = __builtin_amdgcn_rcpf((float)sp.tiles);
+  for (int c = 0; c < nseq; c += 64) {
+    const SplitSeq q = split_seq<BN>(a, sp, c, sh);
+    const int x = split_further(q.n, sp.tiles, inv) >= p ? q.ntile : 0, sum = wave_inclusive_scan_i32(x), u = left - (sum - x);
+    const uint64_t mine = __builtin_amdgcn_ballot_w64(u >= 0 && u < x);
+    if (mine) {
+      const int l = __builtin_ctzll(mine);
+      return {c + l, __builtin_amdgcn_readlane(u, l), p};
+    }
+    left -= __builtin_amdgcn_readlane(sum, 63);
+  }
+  return {-1, 0, 0};
 }
 
 // Output rows that no sequence covers -- [0, cu[0]) and [cu[N], T), clamped
@@ -237,17 +419,19 @@ GDN_DEVICE void zero_rows_tail(const AttnArgs& a, uint32_t wg, uint32_t n) {
 }
 
 // SPLIT: the key range of every (query tile, head group) row is cut into
-// pieces of a.piece_tiles key tiles, one workgroup each (piece index
-// outermost in the grid, so that the pieces that run together read the same
-// stretch of their sequence's K/V rows).  A row of one piece writes its output
-// rows; otherwise every piece writes m, l and the unnormalised O to the
+// pieces (split_tiles), one workgroup each.  A row of one piece writes its
+// output rows; otherwise every piece writes m, l and the unnormalised O to the
 // workspace and attn_prefill_combine_kernel merges them.  It serves batches
 // whose rows are few or uneven for 256 CUs (one workgroup per CU at D = 256):
 // a workgroup runs 1.2 us per key tile, so 1,000 new tokens over a 15,000-key
 // prefix are 128 rows of 550 us each.  Measured (16 / 2 heads, D = 256, one
-// piece -> split): four prompts of 800 to 1,500 tokens over prefixes of 500 to
-// 15,800 keys 1,192 -> 951 us (574 -> 720 TFLOP/s), one of 512 over 8,000 98 ->
-// 47 us, five of 18 over 11,700 301 -> 64 us.
+// piece -> split): four prompts of 260 to 1,900 tokens over prefixes of up to
+// 15,800 keys 1,188 -> 965 us, one of 512 over 8,000 keys 309 -> 104, over 2,000
+// 88 -> 53, five of 18 over 11,700 444 -> 75; the same with tables of 131,072
+// keys (pieces cut from the table's width: 187 us at 8,000 keys, and nothing
+// split at 2,000).  Where there is nothing to split, the extra workgroups and
+// the second launch cost 1 to 6 us: four prompts of 1,000 tokens without a
+// prefix 87 -> 93 us (98 with pieces from the width).
 //
 // Key tiles: 32 keys, which at D = 64 and 128 leave room for two waves per
 // SIMD (at least) whose softmax and MFMAs overlap; D = 96 fits two with 64, and
@@ -306,21 +490,40 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   // sequence's workgroups run together and share its K/V rows in L2.
   __shared__ int32_t lookup[8];
   const int hg = a.Hq / gh;  // head groups
-  // (the grid ends with one tile's head groups more than the sequences can
-  // have: a split grid's come after its pieces)
-  const uint32_t srows = SPLIT ? (uint32_t)a.rows : 0u;
-  const bool past = SPLIT && blockIdx.x >= srows * (uint32_t)a.splits;
-  const uint32_t piece = SPLIT && !past ? blockIdx.x / srows : 0u;
-  const uint32_t row_id = past ? srows + (blockIdx.x - srows * (uint32_t)a.splits) : blockIdx.x - piece * srows;
-  const SeqTile st = attn_tile_lookup<D, PAGED>(a, 32 * qsubs, row_id / hg, lookup);
-  // (no tile is left past the grid's rows unless the offsets decrease: nothing
-  // is kept for it in the workspace)
-  if (past && st.seq >= 0) return;
-  if (st.seq < 0) {
-    if (piece > 0) return;
-    const uint32_t tiles = (SPLIT ? srows : gridDim.x - hg) / hg + 1;
-    zero_rows_tail<T>(a, (uint32_t)st.tile * hg + row_id % hg, (tiles - (row_id / hg - (uint32_t)st.tile)) * hg);
-    return;
+  // (the grid's rows end with one tile's head groups more than the sequences
+  // can have; a split grid's extra workgroups come after them)
+  const uint32_t srows = SPLIT ? (uint32_t)a.rows : gridDim.x - hg;
+  uint32_t row_id = blockIdx.x, slot = blockIdx.x;  // slot: of the piece's partial
+  int ptiles = kWholeRows, piece = 0;
+  SeqTile st;
+  bool further = false;
+  const int sh = __builtin_ctz(32 * qsubs);
+  SplitPlan sp;
+  if constexpr (SPLIT) {
+    sp.q = split_seq<BN>(a, lane, sh);
+    further = blockIdx.x >= srows + hg;
+    if (further) {
+      ptiles = sp.tiles = split_tiles<D, BN>(a, sp, sh);
+      if (ptiles == kWholeRows) return;
+      row_id = blockIdx.x - (srows + hg);
+      slot = srows + row_id;
+      const SplitPiece p = split_piece<BN>(a, sp, sh, (int)(row_id / hg));
+      if (p.seq < 0) return;
+      st.seq = p.seq;
+      st.tile = p.tile;
+      piece = p.piece;
+    }
+  }
+  if (!further) {
+    st = attn_tile_lookup<D, PAGED, SPLIT>(a, 32 * qsubs, row_id / hg, lookup);
+    // (no tile is left past the grid's rows unless the offsets decrease: nothing
+    // is kept for it in the workspace)
+    if (SPLIT && row_id >= srows && st.seq >= 0) return;
+    if (st.seq < 0) {
+      const uint32_t tiles = srows / hg + 1;
+      zero_rows_tail<T>(a, (uint32_t)st.tile * hg + row_id % hg, (tiles - (row_id / hg - (uint32_t)st.tile)) * hg);
+      return;
+    }
   }
   const int64_t n = st.seq;
   const int y = (int)(row_id % hg);
@@ -348,13 +551,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   const int64_t kend_row = a.causal ? clamp64(off + wg_qend, 0, Lk) : Lk;
   const int64_t kend_roww = q0 >= len ? 0 : (a.causal ? clamp64(off + w_qend, 0, Lk) : Lk);
   // this piece's key tiles [tile0, ntiles); keys past its end are not loaded
-  const int tile0 = SPLIT ? (int)piece * a.piece_tiles : 0;
-  const bool whole = !SPLIT || kend_row <= (int64_t)a.piece_tiles * BN;  // the row is one piece
+  const int tile0 = SPLIT ? piece * ptiles : 0;
   if (SPLIT && piece > 0 && (int64_t)tile0 * BN >= kend_row) return;
-  const int64_t piece_end = SPLIT ? (int64_t)(tile0 + a.piece_tiles) * BN : 0;
-  const int64_t kend = SPLIT && kend_row > piece_end ? piece_end : kend_row;
-  const int64_t kend_w = SPLIT && kend_roww > piece_end ? piece_end : kend_roww;
-  const int ntiles = (int)((kend + BN - 1) / BN);
+  int64_t kend = kend_row, kend_w = kend_roww;
+  bool whole = true;  // the row is one piece
+  auto cut = [&](int tiles) __attribute__((always_inline)) {
+    const int64_t end = (int64_t)(tile0 + tiles) * BN;
+    whole = kend_row <= (int64_t)tiles * BN;
+    kend = kend_row > end ? end : kend_row;
+    kend_w = kend_roww > end ? end : kend_roww;
+  };
+  if (SPLIT && further) cut(ptiles);
 
   // query fragments (B operand of S^T = K Q^T): lane holds query q0 + lane % 32,
   // dims 16 ks + 8 (lane / 32) .. +7
@@ -423,7 +630,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   // strides fit 32 bits (the launcher takes the per-row path otherwise)
   const uint32_t* trow = G16 ? reinterpret_cast<const uint32_t*>(a.tab.table) + (T64 ? 2 : 1) * (n * a.tab.row_stride)
                              : nullptr;
-  const uint32_t kend32 = (uint32_t)kend;
+  uint32_t kend32 = (uint32_t)kend;
   auto load_ids = [&](int t, uint32_t* lo, uint32_t* hi, bool* in, uint32_t* sl) {
 #pragma unroll
     for (int g = 0; g < NG; ++g) {
@@ -665,6 +872,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   // and tile t + 2 is in flight: two register sets (A: even tiles, B: odd)
   uint4 kA[NLD], vA[NLD], kB[NLD], vB[NLD];
   load_tile(tile0, kA, vA);
+  // (a row's first piece works out where it ends only now, with the first tile's
+  // loads in flight: no piece is shorter than that)
+  if constexpr (SPLIT) {
+    if (!further) {
+      cut(split_tiles<D, BN>(a, sp, sh));
+      kend32 = (uint32_t)kend;
+    }
+  }
+  const int ntiles = (int)((kend + BN - 1) / BN);
   stage_q();  // (waits for the query loads with tile 0's loads in flight)
   store_tile(0, kA, vA);
   load_tile(tile0 + 1, kB, vB);
@@ -701,7 +917,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   const float lt = lsum + __shfl_xor(lsum, 32);
   if constexpr (SPLIT) {
     if (!whole) {
-      float* pw = a.part + ((int64_t)row_id * a.splits + piece) * prefill_part_floats<D>() + w * prefill_part_wave<D>();
+      float* pw = a.part + (int64_t)slot * prefill_part_floats<D>() + w * prefill_part_wave<D>();
 #pragma unroll
       for (int d = 0; d < NDT; ++d)
 #pragma unroll
@@ -766,7 +982,12 @@ __global__ __launch_bounds__(256) void attn_prefill_combine_kernel(const AttnArg
   __shared__ int32_t lookup[8];
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int R = a.Hq / a.Hkv, gh = a.gh, qsubs = 4 / gh, groups = R / gh, hg = a.Hq / gh;
-  const SeqTile st = attn_tile_lookup<D, true>(a, 32 * qsubs, blockIdx.x / hg, lookup);
+  const int sh = __builtin_ctz(32 * qsubs);
+  SplitPlan sp;
+  sp.q = split_seq<BN>(a, lane, sh);
+  sp.tiles = split_tiles<D, BN>(a, sp, sh);
+  if (sp.tiles == kWholeRows) return;
+  const SeqTile st = attn_tile_lookup<D, true, true>(a, 32 * qsubs, blockIdx.x / hg, lookup);
   if (st.seq < 0) return;
   const int y = (int)(blockIdx.x % hg);
   const int head = (y / groups) * R + (y % groups) * gh + (w % gh);
@@ -779,37 +1000,47 @@ __global__ __launch_bounds__(256) void attn_prefill_combine_kernel(const AttnArg
   const int64_t Lk = clamp64(ctx, 0, a.tab.cols * a.tab.page);
   const int64_t wg_qend = qb + 32 * qsubs < len ? qb + 32 * qsubs : len;
   const int64_t kend = clamp64(ctx - len + wg_qend, 0, Lk);
-  const int64_t pk = (int64_t)a.piece_tiles * BN;
-  const int np = (int)((kend + pk - 1) / pk);  // at most a.splits: kend <= columns x page
+  const int64_t pk = (int64_t)sp.tiles * BN;
+  const int np = (int)((kend + pk - 1) / pk);
   const int64_t qi = qb + (w / gh) * 32 + (lane & 31);
-  if (np <= 1 || qi >= len) return;
-  const float* base = a.part + (int64_t)blockIdx.x * a.splits * prefill_part_floats<D>() + w * prefill_part_wave<D>();
-  float mx = -INFINITY;
-  for (int p = 0; p < np; ++p) mx = fmaxf(mx, base[p * prefill_part_floats<D>() + 32 * D + lane]);
-  f32x4 acc[4 * DG];
+  if (np <= 1) return;
+  // slots of the row's further pieces, in lane order; the first has the row's own
+  const SplitCount k = split_count<BN>(a, sp, sh, (int)st.seq);
+  const int extra = wave_inclusive_scan_i32(k.all) - k.all + k.before + (int)st.tile;
+  const int slots = lane == 0 ? (int)blockIdx.x : (int)a.rows + extra * hg + y;
+  // (lanes past the sequence's end go along: their slots are read by the others)
+  const float* const mine = a.part + w * prefill_part_wave<D>();
+  for (int g = blockIdx.y; g < D / (32 * DG); g += gridDim.y) {
+    f32x4 acc[4 * DG];
 #pragma unroll
-  for (int i = 0; i < 4 * DG; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float l = 0.f;
-  for (int p = 0; p < np; ++p) {
-    const float* pp = base + p * prefill_part_floats<D>();
-    const float m = pp[32 * D + lane];
-    const float wt = m == -INFINITY ? 0.f : exp2_fast(m - mx);
-    l += wt * pp[32 * D + 64 + lane];
+    for (int i = 0; i < 4 * DG; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float mx = -INFINITY, l = 0.f;
+#pragma unroll 2
+    for (int p = 0; p < np; ++p) {
+      const float* pp = mine + (int64_t)__builtin_amdgcn_readlane(slots, p) * prefill_part_floats<D>();
+      const float m = pp[32 * D + lane], lp = pp[32 * D + 64 + lane];
+      f32x4 o[4 * DG];
+#pragma unroll
+      for (int i = 0; i < 4 * DG; ++i) o[i] = *reinterpret_cast<const f32x4*>(pp + ((4 * DG * g + i) * 64 + lane) * 4);
+      // (a piece, or all so far, without keys has weight 0)
+      const float top = fmaxf(mx, m);
+      const float was = mx == -INFINITY ? 0.f : exp2_fast(mx - top), now = m == -INFINITY ? 0.f : exp2_fast(m - top);
+      mx = top;
+      l = l * was + lp * now;
+#pragma unroll
+      for (int i = 0; i < 4 * DG; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][e] = acc[i][e] * was + o[i][e] * now;
+    }
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    T* op = reinterpret_cast<T*>(a.o) + (s0 + qi) * a.o_st + (int64_t)head * a.o_sh + 4 * (lane >> 5) + 32 * DG * g;
 #pragma unroll
     for (int i = 0; i < 4 * DG; ++i) {
-      const f32x4 o = *reinterpret_cast<const f32x4*>(pp + ((4 * DG * blockIdx.y + i) * 64 + lane) * 4);
+      v4 ov;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc[i][e] += wt * o[e];
+      for (int e = 0; e < 4; ++e) ov[e] = (T)(acc[i][e] * inv);
+      if (qi < len) *reinterpret_cast<v4*>(op + 8 * i) = ov;
     }
-  }
-  const float inv = l > 0.f ? 1.f / l : 0.f;
-  T* op = reinterpret_cast<T*>(a.o) + (s0 + qi) * a.o_st + (int64_t)head * a.o_sh + 4 * (lane >> 5) + 32 * DG * blockIdx.y;
-#pragma unroll
-  for (int i = 0; i < 4 * DG; ++i) {
-    v4 ov;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) ov[e] = (T)(acc[i][e] * inv);
-    *reinterpret_cast<v4*>(op + 8 * i) = ov;
   }
 }
 
@@ -1337,8 +1568,8 @@ hipError_t launch_prefill_t(const AttnArgs& a, int64_t nseq, int64_t max_len, hi
   } else if (a.tab.page % 16 == 0 && a.k.sb < (int64_t(1) << 32) && a.v.sb < (int64_t(1) << 32) && a.tab.cols > 0 &&
              a.tab.cols * a.tab.page < (int64_t(1) << 31) && a.tab.num_blocks < (int64_t(1) << 31)) {
     // whole 16-row groups per page, 32-bit table arithmetic
-    if (a.splits > 1) {
-      const dim3 sgrid((unsigned)(a.rows * a.splits + a.Hq / a.gh));
+    if (a.extra > 0) {
+      const dim3 sgrid((unsigned)(a.rows + a.Hq / a.gh + a.extra));
       constexpr int DG = D == 256 ? 2 : 1;  // 32-dim blocks per combine workgroup
       if (a.tab.is64)
         hipLaunchKernelGGL((attn_prefill_kernel<T, D, BN, 3, true>), sgrid, dim3(256), 0, st, a);
@@ -1346,8 +1577,9 @@ hipError_t launch_prefill_t(const AttnArgs& a, int64_t nseq, int64_t max_len, hi
         hipLaunchKernelGGL((attn_prefill_kernel<T, D, BN, 2, true>), sgrid, dim3(256), 0, st, a);
       const hipError_t e = hipGetLastError();
       if (e != hipSuccess) return e;
-      hipLaunchKernelGGL((attn_prefill_combine_kernel<T, D, BN, DG>), dim3((unsigned)a.rows, D / (32 * DG)), dim3(256),
-                         0, st, a);
+      // (many rows fill the chip by themselves)
+      hipLaunchKernelGGL((attn_prefill_combine_kernel<T, D, BN, DG>),
+                         dim3((unsigned)a.rows, a.rows >= 256 ? 1 : D / (32 * DG)), dim3(256), 0, st, a);
     } else if (a.tab.is64)
       hipLaunchKernelGGL((attn_prefill_kernel<T, D, BN, 3, false>), grid, dim3(256), 0, st, a);
     else
@@ -1408,33 +1640,35 @@ hipError_t launch_prefill(const AttnArgs& a, int dtype, int D, int64_t nseq, int
 
 int heads_per_group(int R) { return R % 4 == 0 ? 4 : (R % 2 == 0 ? 2 : 1); }
 
-// Pieces per row of a split paged prefill over at most `cap` keys (1: not
-// split) and the key tiles of a piece.  The host does not see the context
-// lengths, so the choice prices the batch in key-tile steps of one workgroup
-// (1.18 us at D = 256) as if its rows held half the table's capacity on
-// average and the last row to start all of it: per workgroup slot
-// rows n / slots pieces of kFixed + nt / 2n steps, the last piece's nt / n,
-// and for n > 1 the combine (its launch, and the partials' traffic).  The
-// fixed part of a workgroup (tile lookup, query staging, pipeline fill,
-// output) was measured at about 10 steps.  One split from about 2,000 rows on
-// (16 prompts of 1,200 tokens over 16 heads): there the rows themselves fill
-// the chip evenly.
+// Whether a paged prefill over at most `cap` keys per sequence runs split, and
+// with how many workgroups for the rows' further pieces (0: not split).  The
+// host does not see the context lengths, so it prices the batch as if its rows
+// held half the table's capacity on average and the last row to start all of
+// it: per workgroup slot rows n / slots pieces of kFixed + nt / 2n steps, the
+// last piece's nt / n, and for n > 1 the combine (its launch, and the partials'
+// traffic).  The pieces' length is the device's choice, from the lengths
+// themselves (split_tiles); what a table wider than its contexts costs is the
+// extra workgroups, which find nothing to do, and the combine's launch.  So there
+// are no more of them than kMaxExtra, or one per row.
+// Not split from about 2,000 rows on (16 prompts of 1,200 tokens over 16
+// heads): there the rows themselves fill the chip evenly.
 struct PrefillSplit {
-  int32_t splits, piece_tiles;
-  int64_t rows;
+  int64_t rows, extra;
 };
 PrefillSplit prefill_split(int64_t T, int64_t nseq, int64_t Hq, int64_t Hkv, int64_t D, int64_t cap) {
   constexpr double kSlots = 256, kFixed = 10, kCombine = 6, kPiece = 0.03;
   constexpr int64_t kMaxSplits = 64, kMaxFloats = int64_t(1) << 27;  // partials of at most 512 MiB
-  PrefillSplit r{1, 0, 0};
+  PrefillSplit r{0, 0};
   if (T <= 0 || nseq <= 0 || Hkv <= 0 || cap <= 0) return r;
   const int gh = heads_per_group((int)(Hq / Hkv));
   constexpr int BN = 32;
   r.rows = (T / (32 * (4 / gh)) + nseq) * (Hq / gh);
   const int64_t nt = (cap + BN - 1) / BN;
   const double slots = D == 256 ? kSlots : 2 * kSlots;  // D <= 128: two workgroups fit a CU
+  const int64_t kMaxExtra = D == 256 ? 1280 : 3584;
   const int64_t per_piece = 4 * (32 * D + 128);
   double best = 0;
+  int64_t splits = 1;
   for (int64_t n = 1; n <= kMaxSplits; ++n) {
     if (n > 1 && (nt / n < 8 || r.rows * n * per_piece > kMaxFloats)) break;
     const double step = (double)nt / n;
@@ -1444,14 +1678,10 @@ PrefillSplit prefill_split(int64_t T, int64_t nseq, int64_t Hq, int64_t Hkv, int
       best = 0.9 * t;  // (a split has to win clearly)
     } else if (t < best) {
       best = t;
-      r.splits = (int32_t)n;
+      splits = n;
     }
   }
-  if (r.splits > 1) {
-    r.piece_tiles = (int32_t)((nt + r.splits - 1) / r.splits);
-    r.piece_tiles += r.piece_tiles & 1;
-    r.splits = (int32_t)((nt + r.piece_tiles - 1) / r.piece_tiles);
-  }
+  r.extra = r.rows * std::min(splits - 1, std::max<int64_t>(kMaxExtra / r.rows, 1));
   return r;
 }
 
@@ -1512,13 +1742,11 @@ hipError_t attn_paged_prefill_launch(const gdn_tensor* q, const gdn_tensor* kc, 
   const int64_t nseq = cu->shape[0] - 1;
   if (q->shape[0] == 0) return hipSuccess;
   AttnArgs a{};
-  a.splits = 1;
   if (workspace) {
     const PrefillSplit sp = prefill_split(q->shape[0], nseq, q->shape[1], kc->shape[2], q->shape[2],
                                           tab->shape[1] * kc->shape[1]);
-    a.splits = sp.splits;
-    a.piece_tiles = sp.piece_tiles;
     a.rows = sp.rows;
+    a.extra = (int32_t)sp.extra;
     a.part = workspace;
   }
   a.q = q->data;
@@ -1547,7 +1775,7 @@ hipError_t attn_paged_prefill_launch(const gdn_tensor* q, const gdn_tensor* kc, 
 
 int64_t attn_paged_prefill_workspace(int64_t T, int64_t nseq, int64_t Hq, int64_t Hkv, int64_t D, int64_t cap) {
   const PrefillSplit sp = prefill_split(T, nseq, Hq, Hkv, D, cap);
-  return sp.splits > 1 ? sp.rows * sp.splits * 4 * (32 * D + 128) : 0;
+  return sp.extra > 0 ? (sp.rows + sp.extra) * 4 * (32 * D + 128) : 0;
 }
 
 namespace {

@@ -3,6 +3,8 @@ range of a row runs as several workgroups) vs the fp64 oracle and vs the
 unsplit entry.  Same bars as the attention tests; between the two entries the
 outputs differ by the order of fp32 sums and by P rounded against another
 base, so they also share the 5e-3 relative norm."""
+import random
+
 import pytest
 import torch
 
@@ -161,3 +163,73 @@ def test_paged_prefill_without_room_for_a_workspace(dev, monkeypatch):
     print("paged prefill, no workspace", flush=True)
     out = paged_flash_attention_prefill(*d, None, case.scale, 16, max_seqlen=40)
     assert refused and torch.equal(out, plain)
+
+
+def _against_unsplit(d, max_len, scale):
+    """The split entry over a marked workspace, and whether it wrote partials; the unsplit one."""
+    q, kc, tab = d[0], d[1], d[3]
+    n = _lib.load().paged_attention_prefill_workspace_size(q.shape[0], tab.shape[0], q.shape[1], kc.shape[2], q.shape[2],
+                                                           tab.shape[1] * kc.shape[1])
+    assert n > 0
+    ws = torch.full((n + 4096,), 3.0, device=q.device)
+    out, plain = torch.full_like(q, 9.0), torch.full_like(q, 9.0)
+    _lib.call("paged_attention_prefill_split", *d, out, ws[:n], max_len, scale)
+    _lib.call("paged_attention_prefill", *d, plain, max_len, scale)
+    assert (ws[n:] == 3.0).all()
+    return out, bool((ws[:n] != 3.0).any()), plain
+
+
+def _close(out, plain):
+    assert torch.isfinite(out).all()
+    assert_out_close(out, plain)
+    err = (out.double() - plain.double()).norm() / plain.double().norm().clamp_min(1e-12)
+    assert err < 5e-3, f"relative error norm {err:.3e}"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Hkv, Dh", [(2, 256), (4, 128), (4, 64)])
+@pytest.mark.parametrize(
+    "ctx, new, split",
+    [
+        ([4000, 130, 1500], [3, 40, 40], True),  # pieces of the contexts' lengths, not of the table's
+        ([300, 90, 512], [30, 90, 64], False),  # nothing long enough: no partial is written
+        ([0, 0, 6000], [0, 5, 1], True),
+    ],
+)
+def test_split_paged_prefill_wide_table(dev, Hkv, Dh, ctx, new, split):
+    """Tables 64 times as wide as the longest context (a server's, of its largest length)."""
+    case = paged_case(ctx, new, page=16, seed=len(new), Hq=16, Hkv=Hkv, D=Dh)
+    tab = torch.full((3, 64 * case.block_tables.shape[1]), -1, dtype=torch.int32)
+    tab[:, : case.block_tables.shape[1]] = case.block_tables
+    d = [t.to(dev) for t in (case.q, case.k_cache, case.v_cache, tab, case.context_lens, case.cu)]
+    print(f"wide table D={Dh} ctx={ctx}", flush=True)
+    out, wrote, plain = _against_unsplit(d, max(new), float(case.scale))
+    assert wrote == split
+    _close(out, plain)
+    _close(out.cpu(), paged_attention_ref(case.q, case.k_cache, case.v_cache, case.block_tables, case.context_lens,
+                                          case.cu, case.scale).nan_to_num(0.0))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("seed", range(16))
+def test_split_paged_prefill_batches(dev, seed):
+    """Batches of every kind against the unsplit entry: 1 to 150 sequences (more than a wave's lanes),
+    empty ones, contexts shorter than their new tokens, tables tight and wide, either index type."""
+    r = random.Random(seed)
+    N = r.choice([1, 2, 5, 63, 64, 65, 150])
+    Hq, Hkv, Dh = r.choice([(4, 1, 256), (4, 1, 128), (4, 1, 64)] if N > 5 else
+                           [(16, 2, 256), (4, 1, 256), (16, 4, 128), (4, 4, 128), (8, 2, 64)])
+    new = [r.choice([0, 1, 33, r.randint(1, 100)]) if N > 5 else r.randint(1, 300) for _ in range(N)]
+    new[0] = max(new[0], 1)
+    ctx = [max(0, n + r.choice([0, -5, r.randint(0, 300), r.randint(1500, 5000) if r.random() < 0.4 else 16]))
+           for n in new]
+    ctx[r.randrange(N)] = 6000
+    case = paged_case([max(c, n) for c, n in zip(ctx, new)], new, page=r.choice([16, 48]), seed=seed, Hq=Hq, Hkv=Hkv,
+                      D=Dh, dtype=r.choice([torch.bfloat16, torch.float16]))
+    tab = torch.nn.functional.pad(case.block_tables, (0, r.choice([0, 200, 3000])), value=-1)
+    wide = r.choice([torch.int32, torch.int64])
+    d = [t.to(dev) for t in (case.q, case.k_cache, case.v_cache, tab.to(wide), torch.tensor(ctx, dtype=wide),
+                             case.cu.to(r.choice([torch.int32, torch.int64])))]
+    print(f"split batch {seed}: N={N} Hq={Hq} Hkv={Hkv} D={Dh} {int(case.cu[-1])} tokens", flush=True)
+    out, _, plain = _against_unsplit(d, max(new), float(case.scale))
+    _close(out, plain)
