@@ -179,7 +179,9 @@ class GatedDeltaNet(nn.Module):
         """Whether a decode step runs as three launches (:meth:`_forward_decode`):
         plain 16-bit tensors in one dtype and on one device, with nothing
         recording the torch products that the general path makes (autograd,
-        autocast, a dispatch or function mode, a compiler).  The caches and
+        autocast, a compiler, any dispatch or function mode: the one of
+        ``torch.set_default_device`` is such a mode, so a program that sets it
+        decodes by the general path).  The caches and
         indices are on x's device already (:meth:`_check_inputs`); a parameter
         that is not goes to the general path, whose ops refuse it: the kernels
         would take its pointer as it is."""
