@@ -41,9 +41,19 @@ def test_both_paths_agree(dev):
     assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
     with pytest.raises(_lib.GdnError, match="shape"):
         recurrent_gated_delta_rule(d[0][:3], *d[1:], c.state.to(dev), c.idx.to(dev))
+    # on the current stream, in order: the inputs are written there behind some milliseconds of work
+    late = [torch.zeros_like(t) for t in d]
+    st = torch.zeros_like(c.state.to(dev))
+    state, idx = c.state.to(dev), c.idx.to(dev)
+    big = torch.randn(8192, 8192, device=dev)
     s = torch.cuda.Stream()
-    with torch.cuda.stream(s):  # the current stream of the tensors' device
-        st = c.state.to(dev)
-        o = recurrent_gated_delta_rule(*d, st, c.idx.to(dev))
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        for _ in range(4):
+            big = torch.tanh(big @ big)
+        for t, src in zip(late, d):
+            t.copy_(src)
+        st.copy_(state)
+        o = recurrent_gated_delta_rule(*late, st, idx)
     s.synchronize()
     assert torch.equal(o, outs[0][0]) and torch.equal(st, outs[0][1])

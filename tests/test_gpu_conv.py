@@ -103,8 +103,11 @@ def test_conv_strided_weight(dev):
 def test_conv_tile_edges(dev, W):
     """Lengths around the kernel's 24-token tiles and 4-row batches; the states are exact copies."""
     case = conv_prefill_case([23, 24, 25, 4, 47, 48, 49, 5, 73, 96], seed=10 + W, D=136, W=W, num_slots=12)
+    case.x.mul_(50)  # (unit scale: at the workload's own, y is below the bar's absolute floor)
+    case.weight.mul_(25)
     y, st, y_ref, st_ref = _prefill(case, dev)
-    assert_out_close(y, y_ref)
+    err = (y.double() - y_ref.double()).norm() / y_ref.double().norm()
+    assert err < 2**-8, err  # one bf16 rounding
     assert torch.equal(st, st_ref)
 
 
