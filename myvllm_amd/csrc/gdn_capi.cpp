@@ -214,7 +214,7 @@ int check_conv(const gdn_tensor* x, const gdn_tensor* w, const gdn_tensor* cs, c
     if (!vec_ok(cs, 16)) return GDN_ERR_ALIGN;
   }
   if (T > kMaxGrid || D / 8 > kMaxGrid) return GDN_ERR_RANGE;
-  // the varlen kernel addresses the rows of a 64-token tile with 32-bit byte offsets
+  // the varlen kernel addresses the rows of a tile (24 tokens) with 32-bit byte offsets
   if (x->stride[0] > (int64_t(1) << 23) || out->stride[0] > (int64_t(1) << 23)) return GDN_ERR_RANGE;
   return GDN_OK;
 }
@@ -360,16 +360,11 @@ GDN_EXPORT int64_t gdn_chunk_prefill_workspace_size(int64_t T, int64_t num_seqs,
   return gdn_chunk_prefill_split_floats(T, num_seqs, num_k_heads, num_v_heads, k_head_dim, v_head_dim);
 }
 
-GDN_EXPORT int gdn_chunk_prefill_split_ex(const gdn_tensor* q, const gdn_tensor* k, const gdn_tensor* v,
-                                          const gdn_tensor* g, const gdn_tensor* beta, gdn_tensor* state,
-                                          const gdn_tensor* state_indices, const gdn_tensor* cu_seqlens,
-                                          gdn_tensor* out, const gdn_tensor* workspace, float scale,
-                                          int32_t chunk_size, int32_t flags, void* stream) {
-  if (chunk_size != 64) return GDN_ERR_CHUNK;
-  constexpr int32_t kKnown = GDN_PREFILL_ZERO_INIT | GDN_PREFILL_ACCUM_STATE | GDN_PREFILL_ACCUM_OUT;
-  if ((flags & ~kKnown) != 0) return GDN_ERR_ARG;
-  const bool f32_out = out && out->dtype == GDN_DTYPE_F32;
-  if ((flags & GDN_PREFILL_ACCUM_OUT) && !f32_out) return GDN_ERR_DTYPE;
+namespace {
+int chunk_prefill_split(const gdn_tensor* q, const gdn_tensor* k, const gdn_tensor* v, const gdn_tensor* g,
+                        const gdn_tensor* beta, gdn_tensor* state, const gdn_tensor* state_indices,
+                        const gdn_tensor* cu_seqlens, gdn_tensor* out, const gdn_tensor* workspace, float scale,
+                        int32_t flags, bool f32_out, void* stream) {
   GDN_TRY(check_recurrent(q, k, v, g, beta, state, state_indices, out, cu_seqlens, true, f32_out));
   const int64_t need = gdn_chunk_prefill_workspace_size(q->shape[0], cu_seqlens->shape[0] - 1, q->shape[1], v->shape[1],
                                                         q->shape[2], v->shape[2]);
@@ -385,15 +380,29 @@ GDN_EXPORT int gdn_chunk_prefill_split_ex(const gdn_tensor* q, const gdn_tensor*
                                                   reinterpret_cast<float*>(workspace->data), scale, flags,
                                                   reinterpret_cast<hipStream_t>(stream)));
 }
+}  // namespace
+
+GDN_EXPORT int gdn_chunk_prefill_split_ex(const gdn_tensor* q, const gdn_tensor* k, const gdn_tensor* v,
+                                          const gdn_tensor* g, const gdn_tensor* beta, gdn_tensor* state,
+                                          const gdn_tensor* state_indices, const gdn_tensor* cu_seqlens,
+                                          gdn_tensor* out, const gdn_tensor* workspace, float scale,
+                                          int32_t chunk_size, int32_t flags, void* stream) {
+  if (chunk_size != 64) return GDN_ERR_CHUNK;
+  constexpr int32_t kKnown = GDN_PREFILL_ZERO_INIT | GDN_PREFILL_ACCUM_STATE | GDN_PREFILL_ACCUM_OUT;
+  if ((flags & ~kKnown) != 0) return GDN_ERR_ARG;
+  const bool f32_out = out && out->dtype == GDN_DTYPE_F32;
+  if ((flags & GDN_PREFILL_ACCUM_OUT) && !f32_out) return GDN_ERR_DTYPE;
+  return chunk_prefill_split(q, k, v, g, beta, state, state_indices, cu_seqlens, out, workspace, scale, flags, f32_out,
+                             stream);
+}
 
 GDN_EXPORT int gdn_chunk_prefill_split(const gdn_tensor* q, const gdn_tensor* k, const gdn_tensor* v,
                                        const gdn_tensor* g, const gdn_tensor* beta, gdn_tensor* state,
                                        const gdn_tensor* state_indices, const gdn_tensor* cu_seqlens,
                                        gdn_tensor* out, const gdn_tensor* workspace, float scale, int32_t chunk_size,
                                        void* stream) {
-  GDN_TRY(check_recurrent(q, k, v, g, beta, state, state_indices, out, cu_seqlens, true));
-  return gdn_chunk_prefill_split_ex(q, k, v, g, beta, state, state_indices, cu_seqlens, out, workspace, scale,
-                                    chunk_size, 0, stream);
+  if (chunk_size != 64) return GDN_ERR_CHUNK;
+  return chunk_prefill_split(q, k, v, g, beta, state, state_indices, cu_seqlens, out, workspace, scale, 0, false, stream);
 }
 
 GDN_EXPORT int gdn_chunk_prefill_ex(const gdn_tensor* q, const gdn_tensor* k, const gdn_tensor* v,
