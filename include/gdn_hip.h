@@ -143,8 +143,8 @@ int gdn_chunk_prefill(const gdn_tensor* q, const gdn_tensor* k, const gdn_tensor
  * gdn_chunk_prefill in two launches over a workspace, for batches of few
  * sequences (no counterpart in the reference): what does not depend on the
  * state is computed for all chunks at once, then each sequence and head is
- * walked by eight workgroups.  The result is gdn_chunk_prefill's to the
- * rounding of its operands' splits.
+ * walked by eight workgroups (four past 32 of them).  The result is
+ * gdn_chunk_prefill's to the rounding of its operands' splits.
  *   gdn_chunk_prefill_workspace_size: floats of workspace with which a batch
  *     of T tokens in num_seqs sequences runs so; 0 where gdn_chunk_prefill is
  *     the faster one (no workspace is read then, and the call is the same).

@@ -613,8 +613,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
   // also drains every LDS access in flight).  The rows then load through a
   // buffer descriptor of the kv head's rows of the page: 32-bit offsets, rows
   // past the range or of an invalid block read zero.
-  // The 16-row groups are enumerated in order (load_ids runs for tiles 0, 1,
-  // 2, ...), so a group's table column and first page slot are counted up,
+  // The 16-row groups are enumerated in order (load_ids runs for tiles tile0,
+  // tile0 + 1, ...), so a group's table column and first page slot are counted up,
   // not divided out.
   // An id is kept as the two raw 32-bit words it was loaded as (an int32
   // table: the entry twice) and decoded only where it is used: converting it

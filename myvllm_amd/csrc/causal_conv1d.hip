@@ -6,13 +6,13 @@
 // yuyifanbupt/myvllm).  Both are HBM-streaming kernels: each thread owns 8
 // consecutive channels (one 16-byte bf16 vector) and walks tokens, keeping
 // the W-1 previous inputs in registers, so x is read once (plus a W-1 row
-// halo per 64-token tile) and y written once, fully coalesced.
+// halo per tile of kTile tokens) and y written once, fully coalesced.
 //
-// Prefill tiling: each sequence is cut into 64-token tiles; blockIdx.x is a
-// linear tile id resolved to (sequence, tile) on the device, so no host sync
+// Prefill tiling: each sequence is cut into tiles of kTile tokens; a workgroup's
+// linear tile id is resolved to (sequence, tile) on the device, so no host sync
 // is needed (the reference calls .tolist() on cu_seqlens, ops/causal_conv1d.py:230).
 // Only a sequence's first tile reads its old conv state (a later tile's
-// window starts >= 64 > W-1 tokens into the sequence), and that same tile
+// window starts kTile - (W-1) >= 0 tokens into the sequence), and that same tile
 // writes the new state, so the read-before-write order on a slot is the
 // program order of one thread.
 #include "gdn_common.h"
@@ -95,6 +95,7 @@ GDN_DEVICE void conv_tile(const ConvArgs& a, int64_t seq, int64_t tile, int64_t 
     return;
   }
 
+  static_assert(kTile >= W - 1, "only a sequence's first tile reads its old state");
   // window[m] = input at position t - (W-1) + m for the next token t
   float win[W - 1][kCh];
   TS* st = reinterpret_cast<TS*>(a.state) + slot * a.st_s0 + d0;

@@ -4,8 +4,8 @@
 // torch linears).
 //
 // Bound by the read of w, so a workgroup takes 16 rows of w and its eight
-// waves an eighth of K each: every CU has some 64 KB of w in flight at once,
-// and the tile count fills the chip for any N of the layer.  The rows of w are
+// waves an eighth of K each: 64 KB of w in flight per workgroup.  The layer's
+// in_proj is 772 workgroups, its out_proj only 128, on half the CUs.  The rows of w are
 // the A operand (16x16x32 MFMA, fragments straight from memory, nothing
 // staged), the tokens the B operand; the waves' partial tiles meet in LDS.
 // Measured against the library's product with other weights in turn (us):
