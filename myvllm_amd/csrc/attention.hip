@@ -243,11 +243,10 @@ GDN_DEVICE SeqTile attn_tile_lookup(const AttnArgs& a, int tile_len, int64_t tar
 // kFixed steps per row (lookup, queries, pipeline fill, output) and kPiece per
 // further piece (that, and its share of the merge), and part of the length of
 // those that start last; a batch that fits one round takes as long as its
-// longest workgroup.  Fitted to 29 batches forced into 1 to 16 pieces: what it
-// chooses is 1 % off the best on average, 8 % at most.  A split has to win a
-// sixteenth over one piece per row and to fit the extra workgroups.  The
-// prefill and the combine kernel both work it out, in whole numbers, so that
-// they agree.
+// longest workgroup.  Fitted to 30 batches forced into 1 to 16 pieces: what it
+// chooses is 1 % off the best on average, 8 % at most.  A split has to win 3 %
+// over one piece per row and to fit the extra workgroups.  The prefill and the
+// combine kernel both work it out, in whole numbers, so that they agree.
 struct SplitSeq {
   int32_t ntile, n;  // query tiles, key tiles of the last one
 };
@@ -295,7 +294,7 @@ GDN_DEVICE int wave_sum(int x) { return __builtin_amdgcn_readlane(wave_inclusive
 template <int D, int BN>
 GDN_DEVICE int split_tiles(const AttnArgs& a, const SplitPlan& sp, int sh) {
   constexpr int kSlots = D == 256 ? 256 : D == 128 ? 512 : 768, kSlots16 = kSlots / 16;  // workgroups that run at once
-  constexpr int kFixed = 10, kPiece = D == 256 ? 18 : 16;
+  constexpr int kFixed = 10, kPiece = D == 256 ? 24 : 16;
   const int lane = threadIdx.x & 63, hg = a.Hq / a.gh, nseq = (int)a.nseq;
   // per head group: query tiles R, work W in units of 16 steps, and what one
   // piece per row takes: the longest (last, these run first) query tile of each
@@ -340,7 +339,7 @@ GDN_DEVICE int split_tiles(const AttnArgs& a, const SplitPlan& sp, int sh) {
   const int split = rows + x <= kSlots
                         ? kFixed + 4 + tiles + ((rows + x) / kSlots16)
                         : ((work + kPiece * x / 16) / kSlots16) + (D == 256 ? tiles / 2 + tiles / 8 : tiles / 2) + kFixed;
-  int cost = lane == 0 ? whole - whole / 16 : x > 0 && x <= a.extra && tiles >= 8 ? split : 1 << 24;
+  int cost = lane == 0 ? whole - whole / 32 : x > 0 && x <= a.extra && tiles >= 8 ? split : 1 << 24;
   cost = cost < 1 << 24 ? cost : 1 << 24;
   // (the smallest, of equals the one with fewer pieces)
   const int best = 63 - (wave_top(((1 << 24) - cost) << 6 | (63 - lane)) & 63);
@@ -426,7 +425,7 @@ GDN_DEVICE void zero_rows_tail(const AttnArgs& a, uint32_t wg, uint32_t n) {
 // a workgroup runs 1.2 us per key tile, so 1,000 new tokens over a 15,000-key
 // prefix are 128 rows of 550 us each.  Measured (16 / 2 heads, D = 256, one
 // piece -> split): four prompts of 260 to 1,900 tokens over prefixes of up to
-// 15,800 keys 1,188 -> 965 us, one of 512 over 8,000 keys 309 -> 104, over 2,000
+// 15,800 keys 1,188 -> 957 us, one of 512 over 8,000 keys 309 -> 104, over 2,000
 // 88 -> 53, five of 18 over 11,700 444 -> 75; the same with tables of 131,072
 // keys (pieces cut from the table's width: 187 us at 8,000 keys, and nothing
 // split at 2,000).  Where there is nothing to split, the extra workgroups and
