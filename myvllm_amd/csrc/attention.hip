@@ -183,7 +183,8 @@ GDN_DEVICE SeqTile attn_tile_lookup(const AttnArgs& a, int tile_len, int64_t tar
   SeqTile r;
   if (D < 256 && a.nseq <= 64) {
     __shared__ int32_t before[4][64];
-    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), sh = __builtin_ctz(tile_len);
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int sh = __builtin_ctz(tile_len);
     int nt = 0;
     uint32_t key = 0;
     if (lane < a.nseq) {
@@ -321,7 +322,8 @@ GDN_DEVICE int split_tiles(const AttnArgs& a, const SplitPlan& sp, int sh) {
   const int rows = hg * R, work = hg * W;
   int whole = kFixed + nmax;
   if (rows > kSlots) {
-    const int last = D == 256 ? kFixed + wave_top(late < 1 << 24 ? late : 1 << 24) : (work / kSlots16) + kWholeRows - wave_top(kWholeRows - low);
+    const int last = D == 256 ? kFixed + wave_top(late < 1 << 24 ? late : 1 << 24)
+                              : work / kSlots16 + kWholeRows - wave_top(kWholeRows - low);
     whole = last > whole ? last : whole;
   }
   int tiles = (int)((float)(nmax + lane) * __builtin_amdgcn_rcpf((float)(lane + 1)));
@@ -336,9 +338,9 @@ GDN_DEVICE int split_tiles(const AttnArgs& a, const SplitPlan& sp, int sh) {
       x += __mul24(__builtin_amdgcn_readlane(q.ntile, j), split_further(__builtin_amdgcn_readlane(q.n, j), tiles, inv));
   }
   x = x < 1 << 16 ? x * hg : 1 << 24;
-  const int split = rows + x <= kSlots
-                        ? kFixed + 4 + tiles + ((rows + x) / kSlots16)
-                        : ((work + kPiece * x / 16) / kSlots16) + (D == 256 ? tiles / 2 + tiles / 8 : tiles / 2) + kFixed;
+  const int tail = D == 256 ? tiles / 2 + tiles / 8 : tiles / 2;
+  const int split = rows + x <= kSlots ? kFixed + 4 + tiles + (rows + x) / kSlots16
+                                       : (work + kPiece * x / 16) / kSlots16 + tail + kFixed;
   int cost = lane == 0 ? whole - whole / 32 : x > 0 && x <= a.extra && tiles >= 8 ? split : 1 << 24;
   cost = cost < 1 << 24 ? cost : 1 << 24;
   // (the smallest, of equals the one with fewer pieces)
@@ -386,7 +388,8 @@ GDN_DEVICE SplitPiece split_piece(const AttnArgs& a, const SplitPlan& sp, int sh
   const float inv = __builtin_amdgcn_rcpf((float)sp.tiles);
   for (int c = 0; c < nseq; c += 64) {
     const SplitSeq q = split_seq<BN>(a, sp, c, sh);
-    const int x = split_further(q.n, sp.tiles, inv) >= p ? q.ntile : 0, sum = wave_inclusive_scan_i32(x), u = left - (sum - x);
+    const int x = split_further(q.n, sp.tiles, inv) >= p ? q.ntile : 0;
+    const int sum = wave_inclusive_scan_i32(x), u = left - (sum - x);
     const uint64_t mine = __builtin_amdgcn_ballot_w64(u >= 0 && u < x);
     if (mine) {
       const int l = __builtin_ctzll(mine);
@@ -575,7 +578,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 256 ? 
     static_assert(!RAG || q_pieces_inside(DQ), "query pieces are read inside their row");
     const T* qp = reinterpret_cast<const T*>(a.q) + (s0 + (qvalid ? qi : 0)) * a.q_st + (int64_t)head * a.q_sh;
 #pragma unroll
-    for (int s = 0; s < NKS; ++s) qf[s] = *reinterpret_cast<const v8*>(qp + (RAG ? q_piece(s, hh, a.dim) : 16 * s + 8 * hh));
+    for (int s = 0; s < NKS; ++s)
+      qf[s] = *reinterpret_cast<const v8*>(qp + (RAG ? q_piece(s, hh, a.dim) : 16 * s + 8 * hh));
   }
   // the softmax below assumes c > 0: a negative scale is folded into q (an
   // exact sign flip), a zero scale is q = 0 with c = 1 (equal weights)

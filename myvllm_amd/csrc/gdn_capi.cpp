@@ -402,7 +402,8 @@ GDN_EXPORT int gdn_chunk_prefill_split(const gdn_tensor* q, const gdn_tensor* k,
                                        gdn_tensor* out, const gdn_tensor* workspace, float scale, int32_t chunk_size,
                                        void* stream) {
   if (chunk_size != 64) return GDN_ERR_CHUNK;
-  return chunk_prefill_split(q, k, v, g, beta, state, state_indices, cu_seqlens, out, workspace, scale, 0, false, stream);
+  return chunk_prefill_split(q, k, v, g, beta, state, state_indices, cu_seqlens, out, workspace, scale, 0, false,
+                             stream);
 }
 
 GDN_EXPORT int gdn_chunk_prefill_ex(const gdn_tensor* q, const gdn_tensor* k, const gdn_tensor* v,

@@ -44,7 +44,8 @@ def test_fused_prefill_zero_decay_beta_one(dev):
     _check(case, *_fused(case, dev))
 
 
-@pytest.mark.parametrize("rho, spiky", [(1.0, False), (8.0, False), (64.0, False), (128.0, False), (8.0, True), (128.0, True)])
+@pytest.mark.parametrize("rho, spiky", [(1.0, False), (8.0, False), (64.0, False), (128.0, False), (8.0, True),
+                                        (128.0, True)])
 def test_fused_prefill_key_magnitudes(dev, rho, spiky):
     """Keys of norm rho, in random directions or with their mass in one coordinate, over many chunks;
     beta divided by |k|^2, outputs and states in units of 1 / |k| (as test_prefill_key_magnitudes)."""
